@@ -454,7 +454,7 @@ int gfr_ratio(gfr_ctx* ctx, const gfr_geometry* g, const float* d_proj, const fl
   GFR_NONNULL(ctx, d_y, "d_y");
   GFR_NONNULL(ctx, d_corr, "d_corr");
   if (bad_subset(ctx, gd, subset, nsub)) return GFR_EINVAL;
-  GFR_HIP(ctx, launch_ratio(gd->dev, d_proj, d_y, d_bg, GFR_STORE_F32, 1.f, d_corr, nullptr, nullptr, subset, nsub,
+  GFR_HIP(ctx, launch_ratio(gd->dev, d_proj, d_y, d_bg, GFR_STORE_F32, 1.f, d_corr, PackedRows{}, nullptr, subset, nsub,
                             stream_of(ctx, stream)));
   return GFR_OK;
 }
@@ -492,11 +492,13 @@ int gfr_back_project(gfr_ctx* ctx, const gfr_geometry* g, const float* d_corr,
   hipError_t e = hipSuccess;
   {
     std::lock_guard<std::mutex> lk(ctx->mu);
-    float2* c2 = (float2*)scratch_acquire(ctx, ctx->pack, bytes, st, &e);
-    if (c2) e = launch_pack(gd->dev, d_corr, d_mask, c2, subset, nsub, st);
-    if (c2 && e == hipSuccess)
-      e = launch_back_packed(gd->dev, c2, d_numer, d_denom, subset, nsub, nullptr, gd->tune[nsub], st);
-    if (c2) scratch_release(ctx->pack, st);
+    void* buf = scratch_acquire(ctx, ctx->pack, bytes, st, &e);
+    const PackedRows P =
+        packed_rows(gd->dev, buf, subset, nsub, ctx->d_scratch_u32 + 128, ++ctx->pack_epoch);
+    if (buf) e = launch_pack(gd->dev, d_corr, d_mask, P, subset, nsub, st);
+    if (buf && e == hipSuccess)
+      e = launch_back_packed(gd->dev, P, d_numer, d_denom, subset, nsub, nullptr, gd->tune[nsub], st);
+    if (buf) scratch_release(ctx->pack, st);
   }
   if (e != hipSuccess) return hip_err(ctx, e, "back projection");
   return GFR_OK;
@@ -515,8 +517,7 @@ int gfr_sensitivity(gfr_ctx* ctx, const gfr_geometry* g, const uint8_t* d_mask, 
   {
     std::lock_guard<std::mutex> lk(ctx->mu);
     float2* c2 = (float2*)scratch_acquire(ctx, ctx->pack, bytes, st, &e);
-    if (c2) e = launch_pack(gd->dev, nullptr, d_mask, c2, subset, nsub, st);
-    if (c2 && e == hipSuccess) e = launch_sensitivity(gd->dev, c2, d_sens, subset, nsub, st);
+    if (c2) e = launch_sensitivity(gd->dev, d_mask, c2, d_sens, subset, nsub, st);
     if (c2) scratch_release(ctx->pack, st);
   }
   if (e != hipSuccess) return hip_err(ctx, e, "sensitivity");

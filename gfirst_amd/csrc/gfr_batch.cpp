@@ -36,7 +36,8 @@ struct Lane {
   hipStream_t st = nullptr;
   hipEvent_t join = nullptr;
   float *xb = nullptr, *num = nullptr, *den = nullptr, *work = nullptr, *R = nullptr;
-  float2* corr2 = nullptr;
+  float* rows = nullptr;                 // packed rows of a lone frame
+  unsigned* bad = nullptr;               // PackedRows::bad
   float* corr4 = nullptr;                // interleaved rows of a frame group
   float* num_g[kMaxGroup] = {};          // numerators / denominators of a group
   float* den_g[kMaxGroup] = {};          // ([0] = num / den)
@@ -62,17 +63,17 @@ size_t store_bytes(int storage) { return storage == GFR_STORE_F32 ? 4 : 2; }
 int group_of(const gfr_batch_params* p) { return p->group == 0 ? kMaxGroup : p->group; }
 
 struct Sizes {
-  size_t img, corr2, corr4, rot, llh, frame_nobg, frame_bg, shared;
+  size_t img, rows, corr4, rot, llh, frame_nobg, frame_bg, shared;
 };
 
 Sizes sizes_of(const GeomHost& h, const gfr_batch_params* p) {
   Sizes z{};
   const size_t nav = (size_t)(h.g.nang + p->min_nsub - 1) / p->min_nsub;
   z.img = sizeof(float) * (size_t)h.info.nvox;
-  z.corr2 = sizeof(float2) * nav * ((size_t)h.info.nsinogs + 2 * (size_t)h.g.nseg) *
+  z.rows = 2 * sizeof(float) * nav * ((size_t)h.info.nsinogs + 2 * (size_t)h.g.nseg) *
             ((size_t)h.g.nrad + 2);  // packed rows: NRAD + 2 entries
   const int grp = group_of(p);
-  z.corr4 = grp > 1 ? 2 * z.corr2 : 0;
+  z.corr4 = grp > 1 ? 2 * z.rows : 0;
   z.rot = sizeof(float) * (size_t)(h.info.lambda1 - h.info.lambda0 + 1) * h.g.nzs * h.g.nrad *
           std::min(nav, (size_t)kRotChunk);
   z.llh = sizeof(double) * (size_t)llh_capacity(h, p->min_nsub) + 64;
@@ -80,7 +81,7 @@ Sizes sizes_of(const GeomHost& h, const gfr_batch_params* p) {
   z.frame_nobg = z.img + sino;
   z.frame_bg = z.img + 2 * sino;
   const size_t per_lane =
-      (4 + 2 * (size_t)(grp - 1)) * z.img + z.corr2 + z.corr4 + z.rot + z.llh;
+      (4 + 2 * (size_t)(grp - 1)) * z.img + z.rows + z.corr4 + z.rot + z.llh;
   const size_t slots = (size_t)p->max_frames * (3 * sizeof(int) + sizeof(double)) + 256;
   z.shared = (size_t)p->lanes * per_lane + (size_t)h.info.ndata /* mask */ + slots;
   return z;
@@ -101,6 +102,7 @@ struct gfr_batch {
   int* d_sub = nullptr;     // [max_frames] subset index per slot
   int* d_nsub = nullptr;    // [max_frames]
   int* d_slots = nullptr;   // [max_frames] active slots of the current graph
+  unsigned* d_bad = nullptr;  // [lanes] PackedRows::bad
   double* d_llh = nullptr;  // [max_frames] FP64 log-likelihood of the last pass
   std::vector<void*> owned;
   size_t bytes = 0;
@@ -138,7 +140,7 @@ hipError_t enqueue_forward(gfr_batch* b, int f, const Lane& L, int chan) {
   hipError_t e = launch_blur_xy(G, tf, fr.x, L.xb, L.st);
   FwdOut fo;
   if (chan < 0) {
-    fo.corr2 = L.corr2;
+    fo.rows = packed_rows(G, L.rows, 0, fr.nsub, L.bad, 1);
   } else {
     fo.corr4 = L.corr4;
     fo.chan = chan;
@@ -174,7 +176,7 @@ hipError_t enqueue_group(gfr_batch* b, const std::vector<int>& grp, const Lane& 
   if (grp.size() == 1) {
     e = enqueue_forward(b, grp[0], L, -1);
     if (e == hipSuccess)
-      e = launch_back_packed(G, L.corr2, L.num, L.den, 0, f0.nsub, b->d_sub + grp[0], f0.tune,
+      e = launch_back_packed(G, packed_rows(G, L.rows, 0, f0.nsub, L.bad, 1), L.num, L.den, 0, f0.nsub, b->d_sub + grp[0], f0.tune,
                              L.st);
     if (e == hipSuccess) e = enqueue_update(b, grp[0], L.num, L.den, L);
     return e;
@@ -370,14 +372,16 @@ int gfr_batch_create(gfr_ctx* ctx, const gfr_geometry* g, const gfr_batch_params
             A((void**)&b->d_sub, sizeof(int) * p->max_frames) &&
             A((void**)&b->d_nsub, sizeof(int) * p->max_frames) &&
             A((void**)&b->d_slots, sizeof(int) * p->max_frames) &&
-            A((void**)&b->d_llh, sizeof(double) * p->max_frames);
+            A((void**)&b->d_llh, sizeof(double) * p->max_frames) && A((void**)&b->d_bad, 64) &&
+            launch_zero(b->d_bad, 64, b->st) == hipSuccess;
   b->lanes.resize(p->lanes);
   for (Lane& L : b->lanes) {
     if (!ok) break;
+    L.bad = b->d_bad + (&L - b->lanes.data());  // at most 16 lanes
     ok = hipStreamCreateWithFlags(&L.st, hipStreamNonBlocking) == hipSuccess &&
          hipEventCreateWithFlags(&L.join, hipEventDisableTiming) == hipSuccess &&
          A((void**)&L.xb, z.img) && A((void**)&L.num, z.img) && A((void**)&L.den, z.img) &&
-         A((void**)&L.work, z.img) && A((void**)&L.corr2, z.corr2) && A((void**)&L.R, z.rot) &&
+         A((void**)&L.work, z.img) && A((void**)&L.rows, z.rows) && A((void**)&L.R, z.rot) &&
          A((void**)&L.llh_part, z.llh);
     L.num_g[0] = L.num;
     L.den_g[0] = L.den;
@@ -504,14 +508,14 @@ int gfr_batch_add(gfr_batch* b, int niter, int nsub, const float* prompts, const
   if (!t.tuned && !(env && env[0] == '0')) {
     Lane& L = b->lanes[0];
     FwdOut fo;
-    fo.corr2 = L.corr2;
+    fo.rows = packed_rows(G, L.rows, 0, nsub, L.bad, 1);
     fo.mask = b->mask;
     fo.y = fr.y;
     fo.bg = fr.bg;
     fo.storage = b->p.storage;
     fo.yscale = (float)b->g.res;
     fo.llh_part = L.llh_part;
-    e = tune_shapes(G, nsub, fo, fr.x, L.R, L.r_floats, L.corr2, L.num, L.den, st, &t);
+    e = tune_shapes(G, nsub, fo, fr.x, L.R, L.r_floats, L.num, L.den, st, &t);
     if (e != hipSuccess) return undo(hip_err(ctx, e, "gfr_batch_add tuning"));
     std::lock_guard<std::mutex> lk(ctx->mu);
     b->gd->tune[nsub] = t;

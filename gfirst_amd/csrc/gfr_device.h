@@ -86,10 +86,19 @@ __device__ __forceinline__ void xcd_region(int& bx, int& by, int& bz) {
   }
 }
 
-// Packed {ratio, calib} rows of a subset for the backprojector. Per angle of
-// the subset and per segment, the segment's planes zmin..NZS-zmin-1 are
-// preceded and followed by one extra row, so that every plane a voxel can
-// blend (zmin-1 .. NZS-zmin) is addressable without a test:
+// Lanes of one wave exchange values through LDS: orders what the wave wrote
+// before what it reads, without a barrier (DS operations of a wave are in
+// order).
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Packed rows of a subset for the backprojector (PackedRows): one ratio per
+// bin. Per angle of the subset and per segment, the segment's planes
+// zmin..NZS-zmin-1 are preceded and followed by one extra row, so that every
+// plane a voxel can blend (zmin-1 .. NZS-zmin) is addressable without a test:
 //  - segments with zmin > 0: the extra rows hold -1000, the value the
 //    reference stores outside the segment's planes (GFIRST.cu:447);
 //  - the direct segment (zmin = 0): the extra rows repeat planes 0 and NZS-1,
@@ -97,13 +106,86 @@ __device__ __forceinline__ void xcd_region(int& bx, int& by, int& bz) {
 // Each row holds NRAD + 2 entries: bin r at r + 1, and copies of bins 0 and
 // NRAD-1 at both ends, so the pair of bins a radial position blends under
 // clamp-to-edge, (clamp(i), clamp(i + 1)), is the two adjacent entries at
-// clamp(i, -1, NRAD-1) + 1: one 16-byte load.
+// clamp(i, -1, NRAD-1) + 1.
+// The calibration (1, or -1000 in gaps and in the extra rows of oblique
+// segments) has no storage of its own: a bin with calibration -1000 reads
+// kInvalid in `v` and its ratio is in `side`, which holds nothing else. A
+// ratio whose bits are kInvalid's (far below zero: it drops every sample that
+// weighs it) is in `side` as well.
+// *bad == epoch says that some ratio of the pass lies outside the range for
+// which the fast summation is exact (regular_ratio).
+constexpr float kInvalid = -0x1.5a5a5ap126f;
 __host__ __device__ __forceinline__ size_t packed_row_len(int nrad) { return (size_t)nrad + 2; }
 __device__ __forceinline__ size_t packed_rows_per_angle(const DevGeom& G) {
   return (size_t)G.nsinogs + 2 * (size_t)G.nseg;
 }
-__device__ __forceinline__ void store_packed(const DevGeom& G, float2* c2, int ag, int s, int r,
-                                             float2 v) {
+// 0 <= c <= 2^60 or -2^60 <= c <= -2^-32 (gaps are -1000): interpolated
+// values stay below 2^61 in magnitude, and negative ones above 2^-127 (every
+// weight is a multiple of 2^-24).
+__device__ __forceinline__ bool regular_ratio(float c) {
+  return (c >= 0.f && c <= 0x1p60f) || (c <= -0x1p-32f && c >= -0x1p60f);
+}
+// Writes the N <= 4 consecutive bins r .. r + N - 1 (N wave-uniform or not) of
+// one sinogram and angle.
+struct __align__(4) Float4u { float x, y, z, w; };
+__device__ __forceinline__ void store_packed(const DevGeom& G, const PackedRows& P, int ag, int s,
+                                             int r, int N, const float (&c)[4],
+                                             const bool (&valid)[4]) {
+  const int2 sp = G.sino[s];
+  const SegEntry se = G.seg[sp.x];
+  const size_t row0 = (size_t)ag * packed_rows_per_angle(G) + se.nza + 2 * (size_t)sp.x;
+  const int k = sp.y - se.zmin;
+  const int nz = G.nzs - 2 * se.zmin;
+  const size_t L = packed_row_len(G.nrad);
+  bool out = false, inv = false;
+  float f[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    f[i] = valid[i] ? c[i] : kInvalid;
+    if (i < N) {
+      out |= !regular_ratio(c[i]);
+      inv |= f[i] == kInvalid;
+    }
+  }
+  if (out) *P.bad = P.epoch;
+  auto put = [&](size_t row, const float (&val)[4], const float (&sd)[4], bool side) {
+    const size_t o = row * L + r + 1;
+    if (N == 4) {
+      *(Float4u*)(P.v + o) = Float4u{val[0], val[1], val[2], val[3]};
+    } else {
+#pragma unroll
+      for (int i = 0; i < 3; i++)
+        if (i < N) P.v[o + i] = val[i];
+    }
+    if (r == 0) P.v[o - 1] = val[0];
+    if (r + N == G.nrad) P.v[o + N] = val[N - 1 > 2 ? 3 : N - 1 > 1 ? 2 : N - 1 > 0 ? 1 : 0];
+    if (side) {
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        if (i < N && val[i] == kInvalid) {
+          P.side[o + i] = sd[i];
+          if (r + i == 0) P.side[o - 1] = sd[i];
+          if (r + i == G.nrad - 1) P.side[o + i + 1] = sd[i];
+        }
+    }
+  };
+  put(row0 + 1 + k, f, c, inv);
+  if (k == 0 || k == nz - 1) {
+    const float gap[4] = {kInvalid, kInvalid, kInvalid, kInvalid};
+    const float out4[4] = {-1000.f, -1000.f, -1000.f, -1000.f};
+    if (se.zmin == 0) {
+      if (k == 0) put(row0, f, c, inv);
+      if (k == nz - 1) put(row0 + nz + 1, f, c, inv);
+    } else {
+      if (k == 0) put(row0, gap, out4, true);
+      if (k == nz - 1) put(row0 + nz + 1, gap, out4, true);
+    }
+  }
+}
+
+// The same rows as {ratio 1, calib} pairs, for the FP64 sensitivity.
+__device__ __forceinline__ void store_calib(const DevGeom& G, float2* c2, int ag, int s, int r,
+                                            float2 v) {
   const int2 sp = G.sino[s];
   const SegEntry se = G.seg[sp.x];
   const size_t row0 = (size_t)ag * packed_rows_per_angle(G) + se.nza + 2 * (size_t)sp.x;

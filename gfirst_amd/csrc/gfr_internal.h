@@ -43,6 +43,17 @@ struct DevGeom {
 
 struct Taps9 { float g[9]; };
 
+// The backprojector's rows of a subset (layout: gfr_device.h): one float per
+// entry in v, ratios of the invalid bins in side, each `bytes` long. *bad is
+// set to epoch when some ratio is out of the fast summation's range.
+struct PackedRows {
+  float* v;
+  float* side;
+  unsigned bytes;
+  unsigned epoch;
+  unsigned* bad;
+};
+
 // Tile shapes of the projectors (chosen per geometry and subset count by the
 // autotuner; none of them changes any summation order).
 struct Tune {
@@ -118,7 +129,8 @@ struct gfr_ctx {
   size_t kept_bytes = 0;
   size_t kept_max = 0;  // GFR_KEPT_MAX_MB (MiB), default kKeptMax
   std::vector<hipStream_t> kept_streams;  // idle non-blocking streams
-  unsigned int* d_scratch_u32 = nullptr;  // 256 words for small reductions
+  unsigned int* d_scratch_u32 = nullptr;  // 256 words: [0] small reductions, [128] PackedRows::bad
+  unsigned pack_epoch = 0;                // of the last per-operation pack (ctx->mu)
   gfr::Scratch rot;                       // rotation stage of per-operation forward calls
   gfr::Scratch pack;                      // packed ratio of per-operation backprojections
   std::mutex mu;
@@ -187,10 +199,10 @@ hipError_t launch_blur_xy(const DevGeom& G, const Taps9& t, const float* in, flo
 struct FwdOut {
   float* proj = nullptr;          // projection, full sinogram layout
   float* corr = nullptr;          // ratio, full layout
-  float2* corr2 = nullptr;        // {ratio, calib} packed [angle of subset][s][r]
+  PackedRows rows{};              // packed rows of the subset (v NULL: not written)
   float* corr4 = nullptr;         // or: channel `chan` of interleaved 3-frame rows
   int chan = 0;
-  const uint8_t* mask = nullptr;  // calibration mask (needed with corr2)
+  const uint8_t* mask = nullptr;  // calibration mask (needed with rows)
   const void* y = nullptr;        // measured prompts (storage format, unscaled)
   const void* bg = nullptr;       // background or NULL
   int storage = GFR_STORE_F32;
@@ -207,9 +219,11 @@ int forward_llh_blocks(const DevGeom& G, int subset, int nsub, int sg);
 hipError_t launch_forward(const DevGeom& G, const float* img, float* R, size_t r_cap_floats,
                           const FwdOut& out, int subset, int nsub, const int* dsub,
                           const Tune& tune, hipStream_t st);
-hipError_t launch_back_packed(const DevGeom& G, const float2* corr2, float* numer, float* denom,
+hipError_t launch_back_packed(const DevGeom& G, const PackedRows& P, float* numer, float* denom,
                               int subset, int nsub, const int* dsub, const Tune& tune,
                               hipStream_t st);
+// Whether a wave's window of zb slices holds every read of a tile.
+bool back_window_fits(const DevGeom& G, int zb);
 // Multi-frame backprojection: nf (2 or 3) frames' interleaved rows
 // (packed4_bytes) -> numer[f], denom[f]; the sums of launch_back_packed on
 // each frame's own rows, bit for bit. zb: 4 or 6 slices per thread.
@@ -219,21 +233,24 @@ hipError_t launch_back_multi(const DevGeom& G, const float* corr4, float* const*
                              float* const* denom, int nf, int subset, int nsub, const int* dsub,
                              int zb, hipStream_t st);
 // Sensitivity of a subset: the backprojector's denominator half in FP64
-// (packed rows carry ratio 1, so only calibration gaps apply).
-hipError_t launch_sensitivity(const DevGeom& G, const float2* corr2, double* sens, int subset,
-                              int nsub, hipStream_t st);
+// ({1, calib} pairs, packed_bytes of scratch, so only calibration gaps apply).
+hipError_t launch_sensitivity(const DevGeom& G, const uint8_t* mask, float2* c2, double* sens,
+                              int subset, int nsub, hipStream_t st);
 // FP64 log-likelihood of the last forward pass (sum of its block partials).
 hipError_t launch_llh_sum(const DevGeom& G, const double* part, int subset, int nsub,
                           const int* dsub, int sg, double* out, hipStream_t st);
 hipError_t launch_ratio(const DevGeom& G, const float* proj, const float* y, const void* bg,
-                        int storage, float yscale, float* corr, float2* corr2,
+                        int storage, float yscale, float* corr, const PackedRows& P,
                         const uint8_t* mask, int subset, int nsub, hipStream_t st);
 hipError_t launch_calib_mask(const DevGeom& G, const float* pb, const float* norm,
                              uint8_t* mask, hipStream_t st);
-// Full-layout ratio + mask -> packed {ratio, calib} of the subset (packed_bytes).
+// Full-layout ratio + mask -> packed rows of the subset in a buffer of
+// packed_bytes (with a device-side subset index: of subset 0, the largest).
 size_t packed_bytes(const DevGeom& G, int subset, int nsub);
-hipError_t launch_pack(const DevGeom& G, const float* corr, const uint8_t* mask, float2* c2,
-                       int subset, int nsub, hipStream_t st);
+PackedRows packed_rows(const DevGeom& G, void* buf, int subset, int nsub, unsigned* bad,
+                       unsigned epoch);
+hipError_t launch_pack(const DevGeom& G, const float* corr, const uint8_t* mask,
+                       const PackedRows& P, int subset, int nsub, hipStream_t st);
 hipError_t launch_update(const DevGeom& G, const Taps9& t9, const Taps5& t5, const float* numer,
                          const float* denom, float* x, float* work, hipStream_t st);
 hipError_t launch_jbf(const DevGeom& G, const float* in, const float* guide,
@@ -263,8 +280,7 @@ int llh_capacity(const GeomHost& h, int nsub);
 // Times each tile shape of the two projectors on the given buffers (subset 0)
 // and returns the fastest; any shape gives identical results.
 hipError_t tune_shapes(const DevGeom& G, int nsub, const FwdOut& fo, const float* img, float* R,
-                       size_t r_floats, const float2* corr2, float* num, float* den,
-                       hipStream_t st, Tune* out);
+                       size_t r_floats, float* num, float* den, hipStream_t st, Tune* out);
 
 // VLOR.
 hipError_t launch_vlor_count(const int* i1, const int* i2, long long nev, float* v0,

@@ -17,8 +17,7 @@ namespace {
 template <int S>
 __global__ void k_ratio(DevGeom G, const float* __restrict__ proj, const float* __restrict__ y,
                         const void* __restrict__ bg, float yscale, float* __restrict__ corr,
-                        float2* __restrict__ corr2, const uint8_t* __restrict__ mask, int subset,
-                        int nsub) {
+                        PackedRows P, const uint8_t* __restrict__ mask, int subset, int nsub) {
   const int r = blockIdx.x * kWave + threadIdx.x;
   const int s = blockIdx.y * 4 + threadIdx.y;
   const int it = subset + (int)blockIdx.z * nsub;
@@ -31,7 +30,11 @@ __global__ void k_ratio(DevGeom G, const float* __restrict__ proj, const float* 
   const float den = p + bv;
   const float c = (den >= 0.01f) ? yv / den : -1000.f;
   if (corr) corr[bin] = c;
-  if (corr2) store_packed(G, corr2, blockIdx.z, s, r, make_float2(c, mask[bin] ? 1.f : -1000.f));
+  if (P.v) {
+    const float c4[4] = {c, 0.f, 0.f, 0.f};
+    const bool valid[4] = {mask[bin] != 0, true, true, true};
+    store_packed(G, P, blockIdx.z, s, r, 1, c4, valid);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -568,19 +571,19 @@ hipError_t launch_blur_xy(const DevGeom& G, const Taps9& t, const float* in, flo
 }
 
 hipError_t launch_ratio(const DevGeom& G, const float* proj, const float* y, const void* bg,
-                        int storage, float yscale, float* corr, float2* corr2,
+                        int storage, float yscale, float* corr, const PackedRows& P,
                         const uint8_t* mask, int subset, int nsub, hipStream_t st) {
   const int nav = nav_of(G, subset, nsub);
   dim3 grid((G.nrad + kWave - 1) / kWave, (G.nsinogs + 3) / 4, nav);
   if (storage == GFR_STORE_F16)
     hipLaunchKernelGGL(k_ratio<GFR_STORE_F16>, grid, dim3(kWave, 4), 0, st, G, proj, y, bg,
-                       yscale, corr, corr2, mask, subset, nsub);
+                       yscale, corr, P, mask, subset, nsub);
   else if (storage == GFR_STORE_BF16)
     hipLaunchKernelGGL(k_ratio<GFR_STORE_BF16>, grid, dim3(kWave, 4), 0, st, G, proj, y, bg,
-                       yscale, corr, corr2, mask, subset, nsub);
+                       yscale, corr, P, mask, subset, nsub);
   else
     hipLaunchKernelGGL(k_ratio<GFR_STORE_F32>, grid, dim3(kWave, 4), 0, st, G, proj, y, bg,
-                       yscale, corr, corr2, mask, subset, nsub);
+                       yscale, corr, P, mask, subset, nsub);
   return hipGetLastError();
 }
 

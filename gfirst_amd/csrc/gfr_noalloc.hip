@@ -12,6 +12,7 @@
 // Calls share the device's array: two calls in flight at once on one device
 // (different streams) race. Every entry the backprojector reads is rewritten
 // by the pack of the same call, so nothing needs clearing between calls.
+#include <atomic>
 #include <mutex>
 
 #include "gfr_device.h"
@@ -21,7 +22,8 @@ namespace gfr {
 namespace {
 
 constexpr size_t kScratchBytes = size_t(64) << 20;  // 64 MiB
-static __device__ __align__(256) float2 scratch[kScratchBytes / sizeof(float2)];
+// the packed rows, then the word PackedRows::bad
+static __device__ __align__(256) float2 scratch[kScratchBytes / sizeof(float2) + 32];
 
 constexpr int kMaxDevices = 64;
 std::mutex g_mu;
@@ -75,10 +77,14 @@ extern "C" int gfr_back_project_noalloc(gfr_ctx* ctx, const gfr_geometry* g, con
                        "(use more subsets, or gfr_back_project)");
   const hipStream_t st = stream_of(ctx, stream);
   const Tune t = tune_lookup(ctx, gd, nsub);
-  hipError_t e = launch_pack(gd->dev, d_corr, d_mask, (float2*)p, subset, nsub, st);
+  // A captured call keeps its epoch: a replay after one with ratios out of
+  // range then takes the slower, equally exact summation.
+  static std::atomic<unsigned> epoch{0};
+  const PackedRows P = packed_rows(gd->dev, p, subset, nsub, (unsigned*)((char*)p + kScratchBytes),
+                                   ++epoch);
+  hipError_t e = launch_pack(gd->dev, d_corr, d_mask, P, subset, nsub, st);
   if (e == hipSuccess)
-    e = launch_back_packed(gd->dev, (const float2*)p, d_numer, d_denom, subset, nsub, nullptr, t,
-                           st);
+    e = launch_back_packed(gd->dev, P, d_numer, d_denom, subset, nsub, nullptr, t, st);
   if (e != hipSuccess) return hip_err(ctx, e, "gfr_back_project_noalloc");
   return GFR_OK;
 }

@@ -167,10 +167,10 @@ __global__ __launch_bounds__(256) void k_rotate_tile(DevGeom G, const float* __r
 struct FwdArgs {
   float* proj;           // full sinogram layout, or NULL
   float* corr;           // full layout ratio, or NULL
-  float2* corr2;         // packed [angle of subset][s][r] {ratio, calib}, or NULL
+  PackedRows rows;       // packed rows of the subset (v NULL: not written)
   float* corr4;          // interleaved rows of a frame group (channel chan), or NULL
   int chan;
-  const uint8_t* mask;   // calibration mask (full layout) for corr2 / corr4
+  const uint8_t* mask;   // calibration mask (full layout) for rows / corr4
   const void* y;         // measured prompts (storage format), unscaled
   const void* bg;        // background or NULL
   float yscale;          // RES (GFIRST.cu:224-260)
@@ -274,34 +274,41 @@ __global__ __launch_bounds__(256) void k_zsum(DevGeom G, const float* __restrict
         if (i >= ns) break;
         const int s = s0 + i;
         const float av[4] = {acc[i].x, acc[i].y, acc[i].z, acc[i].w};
+        const int N = min(4, G.nrad - r);
+        const size_t bin0 = ((size_t)s * G.nang + it) * G.nrad + r;
+        float c[4];
+        bool valid[4];
 #pragma unroll
         for (int h = 0; h < 4; h++) {
-          const int rr2 = r + h;
-          if (rr2 >= G.nrad) break;
+          c[h] = 0.f;
+          valid[h] = true;
+          if (h >= N) continue;
+          const size_t bin = bin0 + h;
           const float accv = av[h];
-          const size_t bin = ((size_t)s * G.nang + it) * G.nrad + rr2;
           if (o.proj) o.proj[bin] = accv;
           if constexpr (RATIO) {
             const float yv = o.yscale * load_store<S>(o.y, bin);
             float bv = o.bg ? o.yscale * load_store<S>(o.bg, bin) : 0.f;
             if (bv < 0.f) bv = 0.f;
             const float den = accv + bv;
-            const float c = (den >= 0.01f) ? yv / den : -1000.f;
-            if (o.corr) o.corr[bin] = c;
-            if (o.corr2)
-              store_packed(G, o.corr2, ag, s, rr2, make_float2(c, o.mask[bin] ? 1.f : -1000.f));
+            c[h] = (den >= 0.01f) ? yv / den : -1000.f;
+            if (o.mask) valid[h] = o.mask[bin] != 0;
+            if (o.corr) o.corr[bin] = c[h];
             if (o.corr4)
-              store_packed4(G, o.corr4, ag, s, rr2, o.chan, c, o.mask[bin] ? 1.f : -1000.f);
+              store_packed4(G, o.corr4, ag, s, r + h, o.chan, c[h], valid[h] ? 1.f : -1000.f);
             if constexpr (LLH) {
               // Poisson log-likelihood in count units over the bins whose
               // ratio enters the backprojection: model mean den/RES, counts
               // yv/RES (yv and den as the ratio sees them).
-              if (den >= 0.01f && (!o.mask || o.mask[bin])) {
+              if (den >= 0.01f && valid[h]) {
                 const double m = (double)den / (double)o.yscale;
                 ll += ((double)yv / (double)o.yscale) * log(m) - m;
               }
             }
           }
+        }
+        if constexpr (RATIO) {
+          if (o.rows.v && N > 0) store_packed(G, o.rows, ag, s, r, N, c, valid);
         }
       }
     }
@@ -319,43 +326,40 @@ __global__ __launch_bounds__(256) void k_zsum(DevGeom G, const float* __restrict
   }
 }
 
-// Full-layout ratio (NULL: 1 everywhere) + byte mask -> packed {ratio,
-// calib} rows of a subset.
+// Full-layout ratio + byte mask -> packed rows of a subset.
 __global__ void k_pack(DevGeom G, const float* __restrict__ corr, const uint8_t* __restrict__ mask,
-                       float2* __restrict__ c2, int subset, int nsub) {
+                       PackedRows P, int subset, int nsub) {
   const int r = blockIdx.x * kWave + threadIdx.x;
   const int s = blockIdx.y * 4 + threadIdx.y;
   const int a = blockIdx.z;
   if (r >= G.nrad || s >= G.nsinogs) return;
   const size_t bin = ((size_t)s * G.nang + subset + a * nsub) * G.nrad + r;
-  store_packed(G, c2, a, s, r, make_float2(corr ? corr[bin] : 1.f, mask[bin] ? 1.f : -1000.f));
+  const float c[4] = {corr[bin], 0.f, 0.f, 0.f};
+  const bool valid[4] = {mask[bin] != 0, true, true, true};
+  store_packed(G, P, a, s, r, 1, c, valid);
 }
 
+// Byte mask -> {1, calib} pairs of a subset.
+__global__ void k_pack_calib(DevGeom G, const uint8_t* __restrict__ mask, float2* __restrict__ c2,
+                             int subset, int nsub) {
+  const int r = blockIdx.x * kWave + threadIdx.x;
+  const int s = blockIdx.y * 4 + threadIdx.y;
+  const int a = blockIdx.z;
+  if (r >= G.nrad || s >= G.nsinogs) return;
+  const size_t bin = ((size_t)s * G.nang + subset + a * nsub) * G.nrad + r;
+  store_calib(G, c2, a, s, r, make_float2(1.f, mask[bin] ? 1.f : -1000.f));
+}
 
 // ---------------------------------------------------------------------------
-// Backprojector (BACKWPROJ_K, GFIRST_GPU_Kernels.cu:112-160): per voxel and
-// view, bilinear (radial bin, plane) interpolation of the packed {ratio,
-// calib} rows, the -1000 gap rule, sums over views in the reference's order
-// (segments outer, angles inner, GFIRST.cu:439-467).
-//
-// Block: 4 waves, each an 8x8 tile of voxel columns (16x16 per block) times
-// ZB slices. Per view the block needs a small window of the view's rows: the
-// bins its 16x16 columns project to (<= 16*sqrt2*fxb + 2) times the planes
-// its slices tilt to (<= ZB + 16*sqrt2*|fzb| + 2). The window is copied into
-// LDS with coalesced loads, double-buffered so that the next view's window is
-// in flight while the current one is used; the per-voxel reads then come from
-// LDS. Window bounds are exact: every per-lane coordinate is a monotone
-// function (correctly rounded fma/add, floor) of the column position and the
-// slice, so its extremes over the block are at the corner columns and the
-// first/last slice.
+// FP64 sensitivity: the denominator half of the backprojector (BACKWPROJ_K,
+// GFIRST_GPU_Kernels.cu:112-160; gfr_back_window.hip has the pair of sums): per
+// voxel and view, bilinear (radial bin, plane) interpolation of {1, calib}
+// pairs, the -1000 gap rule, sums over views in the reference's order (segments
+// outer, angles inner, GFIRST.cu:439-467).
 // ---------------------------------------------------------------------------
-constexpr int kBW = 33;  // LDS row stride in float2 (odd: rows fall on different banks)
-constexpr int kBinsMax = 32;
-
 // Per-lane state of one view.
 struct LaneView {
   float yr, w0, wl, s0, au;
-  int r0, r1;  // clamped bins (GFIRST_GPU_Kernels.cu texture clamp)
   int iq;      // clamp(floor(u - 0.5), -1, NRAD-1): packed entry pair at iq + 1
   bool any;
 };
@@ -376,8 +380,6 @@ __device__ __forceinline__ LaneView lane_view(const DevGeom& G, float xv, float 
   const float f = floorf(t);
   const int i = (int)f;
   v.au = t - f;
-  v.r0 = min(max(i, 0), G.nrad - 1);
-  v.r1 = min(max(i + 1, 0), G.nrad - 1);
   v.iq = min(max(i, -1), G.nrad - 1);
   return v;
 }
@@ -483,9 +485,9 @@ __device__ __forceinline__ void accumulate_view(const LaneView& v, float fzb, fl
   }
 }
 
-// Rows straight from the packed array: one 16-byte buffer load per plane
-// gives both bins (32-bit offsets).
-struct FetchGlobal {
+// {ratio, calib} pairs: one 16-byte buffer load per plane gives both bins
+// (32-bit offsets).
+struct FetchPairs {
   __amdgpu_buffer_rsrc_t rc;
   unsigned vrow, rowb, oq, rb0 = 0;
   __device__ __forceinline__ void rows(int i0) { rb0 = (vrow + (unsigned)i0) * rowb; }
@@ -501,238 +503,28 @@ struct FetchGlobal {
   }
 };
 
-// Rows from the block's LDS window (row stride kBW, entries of bins
-// rlo - 1 ...); every index is clamped into the window, which only changes
-// lanes outside the view.
 template <int ZB>
-struct FetchLds {
-  const float2* t;
-  int lo, hr, c0, c1;
-  const float2 *p0 = nullptr, *p1 = nullptr;
-  __device__ __forceinline__ void rows(int i0) {
-    const int r = min(max(i0 - lo, 0), hr - ZB);
-    p0 = t + r * kBW + c0;
-    p1 = t + r * kBW + c1;
-  }
-  __device__ __forceinline__ void pair(int k, float2& a0, float2& a1) const {
-    a0 = p0[k * kBW];
-    a1 = p1[k * kBW];
-  }
-  __device__ __forceinline__ void get2(int ii, float2& a0, float2& a1) const {
-    const int r = min(max(ii - lo, 0), hr);
-    a0 = t[r * kBW + c0];
-    a1 = t[r * kBW + c1];
-  }
-};
-
-// Block-uniform window of one view: planes [lo, lo + nr) and bins
-// [rlo, rlo + nb) cover every access of the block's lanes.
-struct Window {
-  int lo, nr, rlo, nb;
-  bool used;  // some column and slice of the block can fall in the segment's planes
-};
-
-__device__ __forceinline__ Window view_window(const DevGeom& G, float x0, float x1, float y0,
-                                              float y1, float st, float ct, float fzb, float fz0,
-                                              float fzl, float fzm, float fzhi) {
-  // yr = fma(yv, ct, -(xv*st)) and xr = fma(yv, st, xv*ct) are monotone in
-  // xv and yv: extremes at the corners.
-  const float ya = fmaf(y0, ct, -(x0 * st)), yb = fmaf(y0, ct, -(x1 * st));
-  const float yc = fmaf(y1, ct, -(x0 * st)), yd = fmaf(y1, ct, -(x1 * st));
-  const float ymn = fminf(fminf(ya, yb), fminf(yc, yd));
-  const float ymx = fmaxf(fmaxf(ya, yb), fmaxf(yc, yd));
-  const float pa = fmaf(ymn, fzb, fz0), pb = fmaf(ymx, fzb, fz0);
-  const float qa = fmaf(ymn, fzb, fzl), qb = fmaf(ymx, fzb, fzl);
-  const float smn = fminf(pa, pb), smx = fmaxf(qa, qb);
-  const float wmn = smn + 0.5f, wmx = smx + 0.5f;
-  Window wd;
-  wd.used = wmx >= fzm && wmn < fzhi;
-  const int lo = (int)floorf(wmn - 0.5f);
-  const int hi = (int)floorf(wmx - 0.5f) + 1;
-  wd.lo = lo;
-  wd.nr = hi - lo + 1;
-  const float xa = fmaf(y0, st, x0 * ct), xb = fmaf(y0, st, x1 * ct);
-  const float xc = fmaf(y1, st, x0 * ct), xd = fmaf(y1, st, x1 * ct);
-  const float umn = fmaf(fminf(fminf(xa, xb), fminf(xc, xd)), G.fxb, G.RADM) + 0.5f;
-  const float umx = fmaf(fmaxf(fmaxf(xa, xb), fmaxf(xc, xd)), G.fxb, G.RADM) + 0.5f;
-  int ra, rb, rc, rd;
-  float dummy;
-  axis(umn, G.nrad, ra, rb, dummy);
-  axis(umx, G.nrad, rc, rd, dummy);
-  wd.rlo = ra;
-  wd.nb = rd - ra + 1;
-  return wd;
-}
-
-template <int ZB>
-__global__ __launch_bounds__(256) void k_back(DevGeom G, const float2* __restrict__ c2,
-                                              unsigned c2_bytes, float* __restrict__ numer,
-                                              float* __restrict__ denom, int subset, int nsub,
-                                              const int* __restrict__ dsub, int rmax) {
-  extern __shared__ float2 tile[];  // [2][rmax][kBW]
-  __shared__ int4 wtab[256];        // windows of a chunk of 256 views
-  __shared__ short wlist[256];      // chunk entries the block touches, in view order
-  __shared__ int wcnt[4];
-  if (dsub) subset = *dsub;
-  const int nav = (G.nang - subset + nsub - 1) / nsub;
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wv = tid >> 6;
-  // blocks of one z-slab are consecutive logical ids, and each XCD walks a
-  // contiguous range of logical ids
-  const unsigned nbx = (G.res + 15) / 16, nxy = nbx * nbx;
-  const unsigned b = xcd_remap(blockIdx.x, gridDim.x);
-  const int bz = (int)(b / nxy), byx = (int)(b - (unsigned)bz * nxy);
-  const int bx = byx % (int)nbx, by = byx / (int)nbx;
-  const int ix = bx * 16 + (wv & 1) * 8 + (lane & 7);
-  const int iy = by * 16 + (wv >> 1) * 8 + (lane >> 3);
-  const int zb = bz * ZB;
-  const bool act = ix < G.res && iy < G.res;
-  const __amdgpu_buffer_rsrc_t rc2 = rsrc(c2, c2_bytes);
-  const float xv = (float)ix - G.RESM, yv = (float)iy - G.RESM;
-  // active corner columns of the block
-  const float cx0 = (float)(bx * 16) - G.RESM, cx1 = (float)min(bx * 16 + 15, G.res - 1) - G.RESM;
-  const float cy0 = (float)(by * 16) - G.RESM, cy1 = (float)min(by * 16 + 15, G.res - 1) - G.RESM;
-  const unsigned rowb = (unsigned)packed_row_len(G.nrad) * 8u;
-  const unsigned nrows = (unsigned)(G.nsinogs + 2 * G.nseg);
-  const float fz0 = (float)zb, fzl = (float)(zb + ZB - 1);
-  float n[ZB], d[ZB];
-#pragma unroll
-  for (int j = 0; j < ZB; j++) n[j] = d[j] = 0.f;
-  // window loader: thread t copies column t % 32 of rows t / 32 + 8 k
-  const int lc = tid & 31, lr = tid >> 5;
-  constexpr int kPre = 6;  // rows per thread: rmax <= 48
-  float2 pre[kPre];
-  // The host launches this kernel only when its row bound fits rmax and the
-  // bin bound fits kBinsMax; the clamps keep every LDS access inside its
-  // buffer regardless.
-  auto issue = [&](const int4 w) {
-    const int lo = w.x, nrr = min(w.y & 0xffff, rmax), nbb = min(w.y >> 16, kBinsMax);
-    const int si = w.w & 0xffff, a = w.w >> 16;
-    const SegEntry se = G.seg[si];
-    const unsigned vrow = (unsigned)a * nrows + (unsigned)(se.nza + 2 * si + 1 - se.zmin);
-#pragma unroll
-    for (int k = 0; k < kPre; k++) {
-      const int r = lr + 8 * k;
-      pre[k] = make_float2(0.f, 0.f);
-      if (r < nrr && lc < nbb)
-        pre[k] = ld_f2(rc2, (vrow + (unsigned)(lo + r)) * rowb + (unsigned)(w.z + 1 + lc) * 8u, 0);
-    }
-  };
-  auto commit = [&](const int4 w, int buf) {
-    const int nrr = min(w.y & 0xffff, rmax), nbb = min(w.y >> 16, kBinsMax);
-    float2* t = tile + buf * rmax * kBW;
-#pragma unroll
-    for (int k = 0; k < kPre; k++) {
-      const int r = lr + 8 * k;
-      if (r < nrr && lc < nbb) t[r * kBW + lc] = pre[k];
-    }
-  };
-  const int nviews = G.nseg * nav;  // view v: segment v / nav, angle v % nav
-  for (int c0 = 0; c0 < nviews; c0 += 256) {
-    __syncthreads();  // the previous chunk's tables and tiles are no longer read
-    // windows of this chunk's views, one per thread, and the list of the
-    // ones the block touches (ballot compaction keeps view order)
-    bool used = false;
-    {
-      const int vi = c0 + tid;
-      if (vi < nviews) {
-        const int si = vi / nav, a = vi - si * nav;
-        const SegEntry se = G.seg[si];
-        const int it = subset + a * nsub;
-        const Window w = view_window(G, cx0, cx1, cy0, cy1, G.sin_t[it], G.cos_t[it], se.fzb,
-                                     fz0, fzl, (float)se.zmin, (float)(G.nzs - se.zmin));
-        used = w.used;
-        wtab[tid] = make_int4(w.lo, (w.nr & 0xffff) | (w.nb << 16), w.rlo, si | (a << 16));
-      }
-    }
-    const unsigned long long m = __builtin_amdgcn_ballot_w64(used);
-    if (lane == 0) wcnt[wv] = __popcll(m);
-    __syncthreads();
-    int off = 0;
-    for (int k = 0; k < wv; k++) off += wcnt[k];
-    const int total = wcnt[0] + wcnt[1] + wcnt[2] + wcnt[3];
-    if (used) {
-      const unsigned lo32 = (unsigned)m, hi32 = (unsigned)(m >> 32);
-      const int below = __builtin_amdgcn_mbcnt_hi(hi32, __builtin_amdgcn_mbcnt_lo(lo32, 0u));
-      wlist[off + below] = (short)tid;
-    }
-    __syncthreads();
-    if (total == 0) continue;
-    int4 cw = wtab[wlist[0]];
-    issue(cw);
-    commit(cw, 0);
-    __syncthreads();
-    int buf = 0;
-    for (int e = 0; e < total; e++) {
-      const bool more = e + 1 < total;
-      int4 nw = make_int4(0, 0, 0, 0);
-      if (more) {
-        nw = wtab[wlist[e + 1]];
-        issue(nw);
-      }
-      const int si = cw.w & 0xffff, a = cw.w >> 16;
-      const SegEntry se = G.seg[si];
-      const int it = subset + a * nsub;
-      const float fzm = (float)se.zmin, fzhi = (float)(G.nzs - se.zmin);
-      const LaneView v = lane_view(G, xv, yv, G.sin_t[it], G.cos_t[it], se.fzb, fz0, fzl, fzm,
-                                   fzhi, act);
-      if (__builtin_amdgcn_ballot_w64(v.any) != 0) {
-        const int hc = min(cw.y >> 16, kBinsMax) - 1;
-        FetchLds<ZB> f;
-        f.t = tile + buf * rmax * kBW;
-        f.lo = cw.x;
-        f.hr = min(cw.y & 0xffff, rmax) - 1;
-        f.c0 = min(max(v.r0 - cw.z, 0), hc);
-        f.c1 = min(max(v.r1 - cw.z, 0), hc);
-        accumulate_view<ZB>(v, se.fzb, v.yr, zb, G.nzs, fzm, fzhi, f, n, d);
-      }
-      if (more) commit(nw, buf ^ 1);
-      __syncthreads();
-      buf ^= 1;
-      cw = nw;
-    }
-  }
-  if (!act) return;
-#pragma unroll
-  for (int j = 0; j < ZB; j++) {
-    const int iz = zb + j;
-    if (iz < G.nzs) {
-      const size_t iV = ((size_t)iz * G.res + iy) * G.res + ix;
-      numer[iV] = n[j];
-      denom[iV] = d[j];
-    }
-  }
-}
-
-// Same sums with every read from global memory: geometries whose window does
-// not fit the LDS bounds.
-// MINW > 0 asks the compiler for a register budget that keeps MINW waves per
-// SIMD resident (an autotuner candidate; more resident waves can also thrash
-// the L1). A block is BW waves of 8x8 columns: 4 (a 16x16 tile) or 1 (8x8,
-// four times the blocks for small images); each voxel's sum is the same.
-template <int ZB, int MINW, class T = float, int BW = 4>
-__global__ __launch_bounds__(64 * BW, MINW > 0 ? MINW : 1) void k_back_direct(
-    DevGeom G, const float2* __restrict__ c2, unsigned c2_bytes, T* __restrict__ numer,
-    T* __restrict__ denom, int subset, int nsub, const int* __restrict__ dsub) {
-  static_assert(BW == 1 || BW == 4, "blocks of 1 or 4 waves");
-  constexpr int kTile = BW == 4 ? 16 : 8;
-  if (dsub) subset = *dsub;
+__global__ __launch_bounds__(256) void k_sensitivity(DevGeom G, const float2* __restrict__ c2,
+                                                     unsigned c2_bytes,
+                                                     double* __restrict__ sens, int subset,
+                                                     int nsub) {
   const int nav = (G.nang - subset + nsub - 1) / nsub;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   int bx, by, bz;
   xcd_region(bx, by, bz);
-  const int ix = bx * kTile + (wv & 1) * 8 + (lane & 7);
-  const int iy = by * kTile + (wv >> 1) * 8 + (lane >> 3);
+  const int ix = bx * 16 + (wv & 1) * 8 + (lane & 7);
+  const int iy = by * 16 + (wv >> 1) * 8 + (lane >> 3);
   const int zb = bz * ZB;
   const bool act = ix < G.res && iy < G.res;
-  const __amdgpu_buffer_rsrc_t rc2 = rsrc(c2, c2_bytes);
+  FetchPairs f;
+  f.rc = rsrc(c2, c2_bytes);
+  f.rowb = (unsigned)packed_row_len(G.nrad) * 8u;
   const float xv = (float)ix - G.RESM, yv = (float)iy - G.RESM;
-  const unsigned rowb = (unsigned)packed_row_len(G.nrad) * 8u;
   const unsigned nr = (unsigned)(G.nsinogs + 2 * G.nseg);
   const float fz0 = (float)zb, fzl = (float)(zb + ZB - 1);
-  T n[ZB], d[ZB];
+  double n[ZB], d[ZB];
 #pragma unroll
-  for (int j = 0; j < ZB; j++) n[j] = d[j] = (T)0;
+  for (int j = 0; j < ZB; j++) n[j] = d[j] = 0.0;
   for (int si = 0; si < G.nseg; si++) {
     const SegEntry se = G.seg[si];
     const float fzm = (float)se.zmin, fzhi = (float)(G.nzs - se.zmin);
@@ -742,10 +534,7 @@ __global__ __launch_bounds__(64 * BW, MINW > 0 ? MINW : 1) void k_back_direct(
       const LaneView v = lane_view(G, xv, yv, G.sin_t[it], G.cos_t[it], se.fzb, fz0, fzl, fzm,
                                    fzhi, act);
       if (__builtin_amdgcn_ballot_w64(v.any) == 0) continue;
-      FetchGlobal f;
-      f.rc = rc2;
       f.vrow = (unsigned)a * nr + segrow;
-      f.rowb = rowb;
       f.oq = (unsigned)(v.iq + 1) * 8u;
       accumulate_view<ZB>(v, se.fzb, v.yr, zb, G.nzs, fzm, fzhi, f, n, d);
     }
@@ -754,11 +543,7 @@ __global__ __launch_bounds__(64 * BW, MINW > 0 ? MINW : 1) void k_back_direct(
 #pragma unroll
   for (int j = 0; j < ZB; j++) {
     const int iz = zb + j;
-    if (iz < G.nzs) {
-      const size_t iV = ((size_t)iz * G.res + iy) * G.res + ix;
-      if (numer) numer[iV] = n[j];
-      denom[iV] = d[j];
-    }
+    if (iz < G.nzs) sens[((size_t)iz * G.res + iy) * G.res + ix] = d[j];
   }
 }
 
@@ -952,88 +737,6 @@ __global__ __launch_bounds__(256) void k_back_multi(DevGeom G, const float* __re
   }
 }
 
-// One slice per thread for small images, where the grid is a few hundred
-// waves and each wave's walk over the views is a chain of memory round trips:
-// the rows of NA consecutive views are all requested before the first of them
-// is summed, so the chain waits once per NA views. With one slice the
-// per-slice formula of accumulate_view (plane position w0, its floor and
-// fraction, rows ii and ii + 1) is the whole computation, and the views are
-// summed in the same order, so the sums are those of k_back_direct<1>.
-template <int NA, int BW>
-__global__ __launch_bounds__(64 * BW) void k_back_ahead(DevGeom G, const float2* __restrict__ c2,
-                                                        unsigned c2_bytes, float* __restrict__ numer,
-                                                        float* __restrict__ denom, int subset,
-                                                        int nsub, const int* __restrict__ dsub) {
-  static_assert(BW == 1 || BW == 4, "blocks of 1 or 4 waves");
-  constexpr int kTile = BW == 4 ? 16 : 8;
-  if (dsub) subset = *dsub;
-  const int nav = (G.nang - subset + nsub - 1) / nsub;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int ix = blockIdx.x * kTile + (wv & 1) * 8 + (lane & 7);
-  const int iy = blockIdx.y * kTile + (wv >> 1) * 8 + (lane >> 3);
-  const int zb = blockIdx.z;
-  const bool act = ix < G.res && iy < G.res;
-  const __amdgpu_buffer_rsrc_t rc2 = rsrc(c2, c2_bytes);
-  const float xv = (float)ix - G.RESM, yv = (float)iy - G.RESM;
-  const unsigned rowb = (unsigned)packed_row_len(G.nrad) * 8u;
-  const unsigned nr = (unsigned)(G.nsinogs + 2 * G.nseg);
-  const float fz0 = (float)zb;
-  float n = 0.f, d = 0.f;
-  for (int si = 0; si < G.nseg; si++) {
-    const SegEntry se = G.seg[si];
-    const float fzm = (float)se.zmin, fzhi = (float)(G.nzs - se.zmin);
-    const unsigned segrow = (unsigned)(se.nza + 2 * si + 1 - se.zmin);
-    for (int a0 = 0; a0 < nav; a0 += NA) {
-      float4 p0[NA], p1[NA];
-      float au[NA], al[NA];
-      bool inr[NA], used[NA];
-#pragma unroll
-      for (int u = 0; u < NA; u++) {
-        const int a = a0 + u;
-        used[u] = false;
-        inr[u] = false;
-        au[u] = al[u] = 0.f;
-        if (a < nav) {
-          const int it = subset + a * nsub;
-          const LaneView v = lane_view(G, xv, yv, G.sin_t[it], G.cos_t[it], se.fzb, fz0, fz0,
-                                       fzm, fzhi, act);
-          used[u] = __builtin_amdgcn_ballot_w64(v.any) != 0;
-          if (used[u]) {
-            const float w = v.w0;
-            inr[u] = v.any && (zb < G.nzs) && w >= fzm && w < fzhi;
-            const float t = w - 0.5f;
-            const float f = floorf(t);
-            al[u] = t - f;
-            au[u] = v.au;
-            const unsigned rb = ((unsigned)a * nr + segrow + (unsigned)(int)f) * rowb +
-                                (unsigned)(v.iq + 1) * 8u;
-            p0[u] = ld_f4(rc2, rb, 0);
-            p1[u] = ld_f4(rc2, rb, rowb);
-          }
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < NA; u++) {
-        if (!used[u]) continue;  // wave-uniform: the view misses the wave
-        const float c0 = lerp1(p0[u].x, p0[u].z, au[u]), c1 = lerp1(p1[u].x, p1[u].z, au[u]);
-        const float q0 = lerp1(p0[u].y, p0[u].w, au[u]), q1 = lerp1(p1[u].y, p1[u].w, au[u]);
-        float A = inr[u] ? lerp1(c0, c1, al[u]) : 0.f;
-        float B = inr[u] ? lerp1(q0, q1, al[u]) : 0.f;
-        if (B < 0.f || A < 0.f) {  // gaps (GFIRST_GPU_Kernels.cu:157)
-          A = 0.f;
-          B = 0.f;
-        }
-        n += A;
-        d += B;
-      }
-    }
-  }
-  if (!act || zb >= G.nzs) return;
-  const size_t iV = ((size_t)zb * G.res + iy) * G.res + ix;
-  numer[iV] = n;
-  denom[iV] = d;
-}
-
 inline int nav_of(const DevGeom& G, int subset, int nsub) {
   return (G.nang - subset + nsub - 1) / nsub;
 }
@@ -1122,9 +825,9 @@ hipError_t launch_forward(const DevGeom& G, const float* img, float* R, size_t r
   // log-likelihood partials are indexed by pair: chunks must hold whole pairs
   if (out.llh_part && chunk < nav && (chunk & 1)) return hipErrorInvalidValue;
   if (out.corr4 && (out.chan < 0 || out.chan >= kMaxGroup)) return hipErrorInvalidValue;
-  FwdArgs o{out.proj, out.corr,  out.corr2,  out.corr4,   out.chan,
+  FwdArgs o{out.proj, out.corr,  out.rows,   out.corr4,   out.chan,
             out.mask, out.y,     out.bg,     out.yscale,  out.llh_part};
-  const bool ratio = out.corr || out.corr2 || out.corr4;
+  const bool ratio = out.corr || out.rows.v || out.corr4;
   for (int a0 = 0; a0 < nav; a0 += chunk) {
     const int na = min(chunk, nav - a0);
     const unsigned rbytes = (unsigned)((size_t)na * per * sizeof(float));
@@ -1160,18 +863,15 @@ hipError_t launch_llh_sum(const DevGeom& G, const double* part, int subset, int 
   return hipGetLastError();
 }
 
-// Rows of the backprojector's LDS window: ZB slices + 1 for the second
-// interpolation plane, the tilt of a 16x16 column tile (15*sqrt2 columns
-// times the largest |fzb|) and 2 for rounding; at most 48 (six rows per
-// loading thread), else 0 and the direct kernel reads global memory.
-int back_window_rows(const DevGeom& G, int zb) {
-  const int r = zb + 3 + (int)ceilf(21.3f * G.fzb_absmax);
-  return r <= 48 ? r : 0;  // 0: does not fit, read global memory directly
-}
-
 size_t packed_bytes(const DevGeom& G, int subset, int nsub) {
   return sizeof(float2) * (size_t)nav_of(G, subset, nsub) * (G.nsinogs + 2 * (size_t)G.nseg) *
          packed_row_len(G.nrad);
+}
+
+PackedRows packed_rows(const DevGeom& G, void* buf, int subset, int nsub, unsigned* bad,
+                       unsigned epoch) {
+  const size_t entries = packed_bytes(G, subset, nsub) / 8;
+  return PackedRows{(float*)buf, (float*)buf + entries, (unsigned)(entries * 4), epoch, bad};
 }
 
 size_t packed4_bytes(const DevGeom& G, int subset, int nsub) {
@@ -1202,78 +902,24 @@ hipError_t launch_back_multi(const DevGeom& G, const float* corr4, float* const*
   return hipGetLastError();
 }
 
-hipError_t launch_pack(const DevGeom& G, const float* corr, const uint8_t* mask, float2* c2,
-                       int subset, int nsub, hipStream_t st) {
+hipError_t launch_pack(const DevGeom& G, const float* corr, const uint8_t* mask,
+                       const PackedRows& P, int subset, int nsub, hipStream_t st) {
   dim3 grid((G.nrad + kWave - 1) / kWave, (G.nsinogs + 3) / 4, nav_of(G, subset, nsub));
-  hipLaunchKernelGGL(k_pack, grid, dim3(kWave, 4), 0, st, G, corr, mask, c2, subset, nsub);
+  hipLaunchKernelGGL(k_pack, grid, dim3(kWave, 4), 0, st, G, corr, mask, P, subset, nsub);
   return hipGetLastError();
 }
 
-hipError_t launch_sensitivity(const DevGeom& G, const float2* corr2, double* sens, int subset,
-                              int nsub, hipStream_t st) {
+hipError_t launch_sensitivity(const DevGeom& G, const uint8_t* mask, float2* c2, double* sens,
+                              int subset, int nsub, hipStream_t st) {
   const size_t bytes = packed_bytes(G, subset, nsub);
+  dim3 grid((G.nrad + kWave - 1) / kWave, (G.nsinogs + 3) / 4, nav_of(G, subset, nsub));
+  hipLaunchKernelGGL(k_pack_calib, grid, dim3(kWave, 4), 0, st, G, mask, c2, subset, nsub);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
   if (bytes >= 0xFFFFFFF0u) return hipErrorInvalidValue;
   const unsigned nbx = (G.res + 15) / 16;
-  hipLaunchKernelGGL((k_back_direct<4, 0, double>), dim3(nbx, nbx, (G.nzs + 3) / 4), dim3(256), 0,
-                     st, G, corr2, (unsigned)bytes, (double*)nullptr, sens, subset, nsub,
-                     (const int*)nullptr);
-  return hipGetLastError();
-}
-
-hipError_t launch_back_packed(const DevGeom& G, const float2* corr2, float* numer, float* denom,
-                              int subset, int nsub, const int* dsub, const Tune& tune,
-                              hipStream_t st) {
-  const size_t bytes = packed_bytes(G, dsub ? 0 : subset, nsub);
-  if (bytes >= 0xFFFFFFF0u) return hipErrorInvalidValue;
-  const unsigned nbx = (G.res + 15) / 16;
-  const bool bins_fit = 21.3f * G.fxb + 3.f <= (float)kBinsMax;
-#define GFR_BK(ZB, W)                                                                           \
-  {                                                                                             \
-    const int rmax = back_window_rows(G, ZB);                                                   \
-    if (tune.back_lds && bins_fit && rmax > 0) {                                                \
-      const unsigned nb = nbx * nbx * (unsigned)((G.nzs + ZB - 1) / ZB);                        \
-      hipLaunchKernelGGL(k_back<ZB>, dim3(nb), dim3(256), sizeof(float2) * 2 * rmax * kBW, st,  \
-                         G, corr2, (unsigned)bytes, numer, denom, subset, nsub, dsub, rmax);    \
-    } else if (tune.back_bw == 1) {                                                             \
-      const unsigned n8 = (G.res + 7) / 8;                                                      \
-      hipLaunchKernelGGL((k_back_direct<ZB, W, float, 1>), dim3(n8, n8, (G.nzs + ZB - 1) / ZB), \
-                         dim3(64), 0, st, G, corr2, (unsigned)bytes, numer, denom, subset,      \
-                         nsub, dsub);                                                           \
-    } else {                                                                                    \
-      hipLaunchKernelGGL((k_back_direct<ZB, W>), dim3(nbx, nbx, (G.nzs + ZB - 1) / ZB),         \
-                         dim3(256), 0, st, G, corr2, (unsigned)bytes, numer, denom, subset,     \
-                         nsub, dsub);                                                           \
-    }                                                                                           \
-  }
-  if (tune.back_ahead > 1 && tune.back_zb == 1 && !tune.back_lds && tune.back_waves == 0) {
-    const unsigned n8 = (G.res + 7) / 8;
-#define GFR_BA(NA, BW)                                                                            \
-  hipLaunchKernelGGL((k_back_ahead<NA, BW>), BW == 4 ? dim3(nbx, nbx, G.nzs) : dim3(n8, n8, G.nzs), \
-                     dim3(64 * BW), 0, st, G, corr2, (unsigned)bytes, numer, denom, subset, nsub, dsub)
-    if (tune.back_ahead == 4) {
-      if (tune.back_bw == 1) GFR_BA(4, 1); else GFR_BA(4, 4);
-    } else {
-      if (tune.back_bw == 1) GFR_BA(2, 1); else GFR_BA(2, 4);
-    }
-#undef GFR_BA
-    return hipGetLastError();
-  }
-  switch (tune.back_zb) {
-    case 1: GFR_BK(1, 0); break;
-    case 2: GFR_BK(2, 0); break;
-    case 4: GFR_BK(4, 0); break;
-    case 5: GFR_BK(5, 0); break;
-    case 6: GFR_BK(6, 0); break;
-    case 16: GFR_BK(16, 0); break;
-    default:
-      if (tune.back_waves == 6) {
-        GFR_BK(8, 6);
-      } else {
-        GFR_BK(8, 0);
-      }
-      break;
-  }
-#undef GFR_BK
+  hipLaunchKernelGGL(k_sensitivity<4>, dim3(nbx, nbx, (G.nzs + 3) / 4), dim3(256), 0, st, G, c2,
+                     (unsigned)bytes, sens, subset, nsub);
   return hipGetLastError();
 }
 
@@ -1283,8 +929,7 @@ int llh_capacity(const GeomHost& h, int nsub) {
 }
 
 hipError_t tune_shapes(const DevGeom& G, int nsub, const FwdOut& fo, const float* img, float* R,
-                       size_t r_floats, const float2* corr2, float* num, float* den,
-                       hipStream_t st, Tune* out) {
+                       size_t r_floats, float* num, float* den, hipStream_t st, Tune* out) {
   hipEvent_t e0, e1;
   if (hipEventCreate(&e0) != hipSuccess) return hipErrorUnknown;
   if (hipEventCreate(&e1) != hipSuccess) {
@@ -1332,31 +977,26 @@ hipError_t tune_shapes(const DevGeom& G, int nsub, const FwdOut& fo, const float
       t.rot_z = c;
     }
   }
-  // backprojector: (kind, slices, register budget, waves per block)
-  // (1 and 2 slices: small images, where each wave's sequential walk over
-  // the views, not the device's throughput, sets the time)
-  // (views whose rows are loaded ahead: 1-slice shapes only)
-  const int bcand[18][5] = {{0, 4, 0, 4, 1}, {0, 5, 0, 4, 1}, {0, 6, 0, 4, 1}, {0, 8, 0, 4, 1},
-                            {0, 8, 6, 4, 1}, {0, 16, 0, 4, 1}, {0, 4, 0, 1, 1}, {0, 6, 0, 1, 1},
-                            {0, 8, 0, 1, 1}, {1, 4, 0, 4, 1},  {1, 8, 0, 4, 1}, {1, 16, 0, 4, 1},
-                            {0, 1, 0, 1, 1}, {0, 2, 0, 1, 1},  {0, 2, 0, 4, 1}, {0, 1, 0, 1, 2},
-                            {0, 1, 0, 1, 4}, {0, 1, 0, 4, 4}};
+  // backprojector: (LDS window, slices, views loaded ahead). One slice and
+  // several views ahead: small images, where each wave's walk over the views,
+  // not the device's throughput, sets the time.
+  const int bcand[9][3] = {{1, 8, 1}, {1, 4, 1}, {1, 5, 1}, {1, 6, 1}, {1, 16, 1},
+                           {0, 1, 4}, {0, 2, 1}, {0, 4, 1}, {0, 6, 1}};
   for (const auto& c : bcand) {
     Tune tt = t;
+    // the gathering shapes serve what the windows cannot hold
+    if (c[2] == 1 && c[0] != (int)back_window_fits(G, c[1])) continue;
     tt.back_lds = c[0];
     tt.back_zb = c[1];
-    tt.back_waves = c[2];
-    tt.back_bw = c[3];
-    tt.back_ahead = c[4];
+    tt.back_ahead = c[2];
+    tt.tuned = true;
     const float ms = time_it([&] {
-      return launch_back_packed(G, corr2, num, den, 0, nsub, nullptr, tt, st);
+      return launch_back_packed(G, fo.rows, num, den, 0, nsub, nullptr, tt, st);
     });
     if (ms < bb) {
       bb = ms;
       t.back_lds = tt.back_lds;
       t.back_zb = tt.back_zb;
-      t.back_waves = tt.back_waves;
-      t.back_bw = tt.back_bw;
       t.back_ahead = tt.back_ahead;
     }
   }

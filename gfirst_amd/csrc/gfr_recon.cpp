@@ -38,7 +38,7 @@ struct gfr_recon {
         *work = nullptr, *jo = nullptr;
   // sinogram-sized
   float *pb = nullptr, *ptc = nullptr, *dv = nullptr;
-  float2* corr2 = nullptr;  // {ratio, calib} of the current subset, [angle][s][r]
+  float* rows = nullptr;    // packed rows of the current subset
   float* R = nullptr;       // rotation stage of the forward projector
   size_t r_floats = 0;
   void *yD = nullptr, *bD = nullptr, *yT = nullptr, *bT = nullptr;
@@ -46,12 +46,12 @@ struct gfr_recon {
   gfr_vlor* vl = nullptr;
   double* llh_part = nullptr;
   double* d_llh = nullptr;
-  unsigned int* d_maxbits = nullptr;
+  unsigned int* d_maxbits = nullptr;  // 16 words: [0] image maximum, [8 + chain] PackedRows::bad
   int llh_valid = 0;
   // triples chain (modes 2-3): stream, scratch, the doubles snapshot
   hipStream_t stT = nullptr;
   float *xbT = nullptr, *numT = nullptr, *denT = nullptr, *workT = nullptr, *xDs = nullptr;
-  float2* corr2T = nullptr;
+  float* rowsT = nullptr;
   float* RT = nullptr;
   double *llh_partT = nullptr, *d_llhT = nullptr;
   hipEvent_t ev_snap = nullptr;   // snapshot of the doubles image taken
@@ -78,7 +78,7 @@ namespace {
 size_t store_bytes(int storage) { return storage == GFR_STORE_F32 ? 4 : 2; }
 
 struct Plan {
-  size_t img, sino_f32, sino_store, mask, llh, corr2, rot;
+  size_t img, sino_f32, sino_store, mask, llh, rows, rot;
   int nimg, nsino_f32, nsino_store;
   bool two;  // second (triples) chain
 };
@@ -97,7 +97,7 @@ Plan plan_of(const GeomHost& h, const gfr_recon_params* p, bool bgD, bool bgT) {
   pl.mask = (size_t)h.info.ndata;
   pl.llh = sizeof(double) * (size_t)llh_capacity(h, p->nsub) + 64;
   const size_t nav = (size_t)(h.g.nang + p->nsub - 1) / p->nsub;
-  pl.corr2 = sizeof(float2) * nav * ((size_t)h.info.nsinogs + 2 * (size_t)h.g.nseg) *
+  pl.rows = 2 * sizeof(float) * nav * ((size_t)h.info.nsinogs + 2 * (size_t)h.g.nseg) *
              ((size_t)h.g.nrad + 2);  // packed rows: NRAD + 2 entries
   pl.rot = sizeof(float) * (size_t)(h.info.lambda1 - h.info.lambda0 + 1) * h.g.nzs * h.g.nrad *
            std::min(nav, (size_t)kRotChunk);
@@ -113,7 +113,7 @@ Plan plan_of(const GeomHost& h, const gfr_recon_params* p, bool bgD, bool bgT) {
 
 size_t plan_bytes(const Plan& pl) {
   return pl.nimg * pl.img + pl.nsino_f32 * pl.sino_f32 + pl.nsino_store * pl.sino_store +
-         pl.mask + (pl.two ? 2 : 1) * (pl.llh + pl.corr2 + pl.rot);
+         pl.mask + (pl.two ? 2 : 1) * (pl.llh + pl.rows + pl.rot);
 }
 
 hipEvent_t take_event(gfr_recon* r) {
@@ -174,7 +174,7 @@ hipError_t autotune(gfr_recon* r) {
     return hipSuccess;
   }
   FwdOut fo;
-  fo.corr2 = r->corr2;
+  fo.rows = packed_rows(gd->dev, r->rows, 0, S, r->d_maxbits + 8, 1);
   fo.mask = r->mask;
   fo.y = r->yD;
   fo.bg = r->bD;
@@ -182,8 +182,7 @@ hipError_t autotune(gfr_recon* r) {
   fo.yscale = (float)r->g.res;
   fo.llh_part = r->llh_part;
   Tune t;
-  hipError_t e = tune_shapes(gd->dev, S, fo, r->xb, r->R, r->r_floats, r->corr2, r->num, r->den,
-                             r->st, &t);
+  hipError_t e = tune_shapes(gd->dev, S, fo, r->xb, r->R, r->r_floats, r->num, r->den, r->st, &t);
   if (e != hipSuccess) return e;
   r->tune = t;
   std::lock_guard<std::mutex> lk(r->ctx->mu);
@@ -324,7 +323,7 @@ int gfr_recon_create(gfr_ctx* ctx, const gfr_geometry* g, const gfr_recon_params
   };
   bool ok = A((void**)&r->xD, pl.img) && A((void**)&r->num, pl.img) && A((void**)&r->den, pl.img) &&
             A((void**)&r->work, pl.img) && A((void**)&r->xb, pl.img) &&
-            A((void**)&r->corr2, pl.corr2) && A((void**)&r->R, pl.rot) &&
+            A((void**)&r->rows, pl.rows) && A((void**)&r->R, pl.rot) &&
             A((void**)&r->mask, pl.mask) && A((void**)&r->yD, pl.sino_store) &&
             A((void**)&r->llh_part, pl.llh) && A((void**)&r->d_maxbits, 64) &&
             A((void**)&r->d_llh, 64);
@@ -334,7 +333,7 @@ int gfr_recon_create(gfr_ctx* ctx, const gfr_geometry* g, const gfr_recon_params
          (!hasBgT || A(&r->bT, pl.sino_store)) && A((void**)&r->xbT, pl.img) &&
          A((void**)&r->numT, pl.img) && A((void**)&r->denT, pl.img) &&
          A((void**)&r->workT, pl.img) && A((void**)&r->xDs, pl.img) &&
-         A((void**)&r->corr2T, pl.corr2) && A((void**)&r->RT, pl.rot) && A((void**)&r->llh_partT, pl.llh) &&
+         A((void**)&r->rowsT, pl.rows) && A((void**)&r->RT, pl.rot) && A((void**)&r->llh_partT, pl.llh) &&
          A((void**)&r->d_llhT, 64);
   if (ok && r->ntypes == 2)
     ok = stream_take(ctx, &r->stT) == hipSuccess &&
@@ -376,7 +375,7 @@ int gfr_recon_create(gfr_ctx* ctx, const gfr_geometry* g, const gfr_recon_params
   if (e == hipSuccess) e = launch_calib_mask(G, r->pb, stage, r->mask, st);
   if (e == hipSuccess) e = hipStreamSynchronize(st);
   // Measured data, stored unscaled; kernels scale by RES on load (GFIRST.cu:224-260).
-  if (e == hipSuccess) e = launch_zero(bad, sizeof(unsigned int), st);
+  if (e == hipSuccess) e = launch_zero(bad, 64, st);
   if (e == hipSuccess) e = upload(d2, r->yD);
   if (e == hipSuccess && hasBgD) e = upload(d2 + nd, r->bD);
   if (e == hipSuccess && r->ntypes == 2) e = upload(t2, r->yT);
@@ -434,7 +433,7 @@ int gfr_recon_step(gfr_recon* r) {
   float* x = tc ? r->xT : r->xD;
   float* xb = tc ? r->xbT : r->xb;
   float* R = tc ? r->RT : r->R;
-  float2* corr2 = tc ? r->corr2T : r->corr2;
+  const PackedRows rows = packed_rows(G, tc ? r->rowsT : r->rows, s, S, r->d_maxbits + 8 + (tc ? 1 : 0), 1);
   float* num = tc ? r->numT : r->num;
   float* den = tc ? r->denT : r->den;
   float* work = tc ? r->workT : r->work;
@@ -473,7 +472,7 @@ int gfr_recon_step(gfr_recon* r) {
     int rc = gfr_vlor_assign(ctx, r->vl, r->ptc, r->dv, s, S, st);
     if (rc != GFR_OK) return rc;
     GFR_HIP(ctx, launch_ratio(G, r->ptc, r->dv, r->bT, p.storage, (float)r->g.res, nullptr,
-                              corr2, r->mask, s, S, st));
+                              rows, r->mask, s, S, st));
     r->llh_valid = 0;
   } else {
     const void* y = tc ? r->yT : r->yD;
@@ -481,7 +480,7 @@ int gfr_recon_step(gfr_recon* r) {
     {
       PhaseMark pm(r, GFR_PHASE_FORWARD, st);
       FwdOut fo;
-      fo.corr2 = corr2;
+      fo.rows = rows;
       fo.mask = r->mask;
       fo.y = y;
       fo.bg = bg;
@@ -497,7 +496,7 @@ int gfr_recon_step(gfr_recon* r) {
   // Backprojection of the subset (GFIRST.cu:436-469) and update (:482-502).
   {
     PhaseMark pm(r, GFR_PHASE_BACK, st);
-    GFR_HIP(ctx, launch_back_packed(G, corr2, num, den, s, S, nullptr, r->tune, st));
+    GFR_HIP(ctx, launch_back_packed(G, rows, num, den, s, S, nullptr, r->tune, st));
   }
   {
     PhaseMark pm(r, GFR_PHASE_UPDATE, st);
