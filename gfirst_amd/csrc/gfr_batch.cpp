@@ -255,6 +255,8 @@ hipError_t enqueue_step(gfr_batch* b) {
 // and, in graph mode, records and instantiates the step program.
 int rebuild(gfr_batch* b) {
   gfr_ctx* ctx = b->ctx;
+  // the last step's launch must be done before its program is destroyed
+  GFR_HIP(ctx, hipStreamSynchronize(b->st));
   drop_graph(b);
   b->active.clear();
   for (int f = 0; f < (int)b->frames.size(); f++)
