@@ -120,13 +120,29 @@ GeomDev* geom_for(gfr_ctx* ctx, const gfr_geometry* g) {
   const size_t off_seg = ((2 * n_ang * sizeof(float)) + 15) & ~size_t(15);
   const size_t off_sino = (off_seg + n_seg * sizeof(SegEntry) + 15) & ~size_t(15);
   const size_t off_zt = (off_sino + n_sino * sizeof(int2) + 15) & ~size_t(15);
-  const size_t total = off_zt + h.ztab.size() * sizeof(uint2);
+  size_t total = (off_zt + h.ztab.size() * sizeof(uint2) + 15) & ~size_t(15);
+  auto place = [&](size_t bytes) {
+    const size_t at = total;
+    total = (total + bytes + 15) & ~size_t(15);
+    return at;
+  };
+  const size_t off_za = place(h.za.size() * sizeof(float));
+  size_t off_zg[3], off_zr[3];
+  for (int k = 0; k < 3; k++) {
+    off_zg[k] = place(h.zgrp[k].size() * sizeof(int2));
+    off_zr[k] = place(h.zrow[k].size() * sizeof(uint32_t));
+  }
   std::vector<char> blob(total, 0);
   memcpy(blob.data(), h.sin_t.data(), n_ang * sizeof(float));
   memcpy(blob.data() + off_cos, h.cos_t.data(), n_ang * sizeof(float));
   memcpy(blob.data() + off_seg, h.seg.data(), n_seg * sizeof(SegEntry));
   memcpy(blob.data() + off_sino, h.sino.data(), n_sino * sizeof(int2));
   memcpy(blob.data() + off_zt, h.ztab.data(), h.ztab.size() * sizeof(uint2));
+  memcpy(blob.data() + off_za, h.za.data(), h.za.size() * sizeof(float));
+  for (int k = 0; k < 3; k++) {
+    memcpy(blob.data() + off_zg[k], h.zgrp[k].data(), h.zgrp[k].size() * sizeof(int2));
+    memcpy(blob.data() + off_zr[k], h.zrow[k].data(), h.zrow[k].size() * sizeof(uint32_t));
+  }
   hipError_t e = hipMalloc(&gd->block, total);
   if (e == hipSuccess) e = hipMemcpy(gd->block, blob.data(), total, hipMemcpyHostToDevice);
   if (e != hipSuccess) {
@@ -158,6 +174,12 @@ GeomDev* geom_for(gfr_ctx* ctx, const gfr_geometry* g) {
   d.seg = (const SegEntry*)(base + off_seg);
   d.sino = (const int2*)(base + off_sino);
   d.ztab = (const uint2*)(base + off_zt);
+  d.za = (const float*)(base + off_za);
+  for (int k = 0; k < 3; k++) {
+    d.zg[k].s = (const int2*)(base + off_zg[k]);
+    d.zg[k].row = (const uint32_t*)(base + off_zr[k]);
+    d.zg[k].n = (int)h.zgrp[k].size();
+  }
   ctx->geoms[key] = gd;
   return gd;
 }
@@ -248,7 +270,10 @@ int run_forward(gfr_ctx* ctx, GeomDev* gd, const float* d_img, const FwdOut& o, 
                 int nsub, hipStream_t st) {
   const int nav = (gd->dev.nang - subset + nsub - 1) / nsub;
   const size_t per = rotate_floats_per_angle(gd->dev);
-  const size_t floats = per * (size_t)std::min(nav, kRotChunk);
+  // Chunks of kRotChunk angles, more while the rotation stays small: every angle
+  // of a small study in one pair of launches instead of four.
+  const size_t more = ((size_t)64 << 20) / (per * sizeof(float));
+  const size_t floats = per * std::min((size_t)nav, std::max((size_t)kRotChunk, more));
   hipError_t e = hipSuccess;
   float* R;
   {
@@ -674,6 +699,7 @@ int gfr_tuning_set(gfr_ctx* ctx, const gfr_geometry* g, int nsub, const gfr_tuni
   t.back_lds = in->back_lds;
   t.back_waves = in->back_waves;
   t.zsum_sg = in->zsum_sg;
+  t.zsum_narrow = -1;
   t.rot_z = in->rot_z;
   t.back_bw = in->back_bw;
   t.back_ahead = ahead;

@@ -154,7 +154,8 @@ hipError_t enqueue_forward(gfr_batch* b, int f, const Lane& L, int chan) {
   if (e == hipSuccess)
     e = launch_forward(G, L.xb, L.R, L.r_floats, fo, 0, fr.nsub, dsub, fr.tune, L.st);
   if (e == hipSuccess)
-    e = launch_llh_sum(G, L.llh_part, 0, fr.nsub, dsub, fr.tune.zsum_sg, b->d_llh + f, L.st);
+    e = launch_llh_sum(G, L.llh_part, 0, fr.nsub, dsub, L.r_floats, fr.tune, b->d_llh + f,
+                       L.st);
   return e;
 }
 

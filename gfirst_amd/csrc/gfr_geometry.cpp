@@ -89,6 +89,25 @@ int derive_geometry(const gfr_geometry* g, GeomHost* out, std::string* err, bool
   // (GFIRST_GPU_Kernels.cu:88, 96), through the clamp-to-edge linear filter.
   // Same float operations as the device code (fmaf is exactly rounded on both).
   if (g->nzs > 0xFFFF) return fail("geometry: nzs too large");
+  for (int j = 0; j < 3; j++) {
+    const int sg = 4 + 2 * j;
+    h.zgrp[j].clear();
+    // four neighbouring segments of one sign (the direct one with the positive)
+    for (int first : {0, 1}) {
+      for (int k0 = first; k0 < g->nseg; k0 += 8) {
+        for (int p0 = h.zmin[k0]; p0 < g->nzs - h.zmin[k0]; p0 += sg) {
+          for (int k = k0; k < k0 + 8; k += 2) {
+            int2 e = make_int2(0, 0);
+            if (k < g->nseg) {
+              const int a = std::max(p0, h.zmin[k]), b = std::min(p0 + sg, g->nzs - h.zmin[k]);
+              if (b > a) e = make_int2(h.nza[k] + a - h.zmin[k], b - a);
+            }
+            h.zgrp[j].push_back(e);
+          }
+        }
+      }
+    }
+  }
   if (!with_ztab) return GFR_OK;
   const int nl = h.info.lambda1 - h.info.lambda0 + 1;
   h.ztab.resize((size_t)acc * nl);
@@ -106,6 +125,23 @@ int derive_geometry(const gfr_geometry* g, GeomHost* out, std::string* err, bool
       uint32_t ab;
       memcpy(&ab, &a, 4);
       h.ztab[(size_t)li * acc + s] = make_uint2((uint32_t)z0 | ((uint32_t)z1 << 16), ab);
+    }
+  }
+  h.za.assign((size_t)acc * nl + kZPad, 0.f);
+  for (size_t i = 0; i < h.ztab.size(); i++) memcpy(&h.za[i], &h.ztab[i].y, 4);
+  for (int j = 0; j < 3; j++) {
+    const size_t n = h.zgrp[j].size();
+    h.zrow[j].resize(n * nl);
+    for (int li = 0; li < nl; li++) {
+      const uint2* t = &h.ztab[(size_t)li * acc];
+      for (size_t q = 0; q < n; q++) {
+        int2& e = h.zgrp[j][q];
+        const uint32_t z = t[e.x].x & 0xffffu;
+        bool reg = true;
+        for (int i = 0; i < abs(e.y); i++) reg = reg && t[e.x + i].x == (z + i) + ((z + i + 1) << 16);
+        h.zrow[j][(size_t)li * n + q] = z | (reg ? kZReg : 0u);
+        if (!reg) e.y = -abs(e.y);
+      }
     }
   }
   return GFR_OK;

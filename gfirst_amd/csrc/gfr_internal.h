@@ -22,6 +22,19 @@ struct SegEntry {
   float fzb;  // backprojector z tilt (GFIRST_GPU_Kernels.cu:134, via double)
 };
 
+// Groups of the wide z-sum: up to SG (4, 6 or 8) consecutive planes of one
+// segment. s: first sinogram and number of sinograms of a group, negative when
+// some sample of the group lacks kZReg; row: per
+// sample [l1-l0+1][n] the row (image plane) of the group's first LOR, with
+// kZReg set where LOR i blends rows row + i and row + i + 1.
+struct ZGroups {
+  const int2* s;
+  const uint32_t* row;
+  int n;
+};
+constexpr uint32_t kZReg = 1u << 31;
+inline __host__ __device__ int zg_index(int sg) { return sg == 4 ? 0 : sg == 6 ? 1 : 2; }
+
 // Geometry as the kernels see it (by value). Pointers are device tables owned
 // by the context, built once per distinct geometry.
 struct DevGeom {
@@ -39,6 +52,8 @@ struct DevGeom {
   // [l1-l0+1][nsinogs]: z interpolation of each LOR sample, x = z0 | z1 << 16,
   // y = bits of alpha_z (GFIRST_GPU_Kernels.cu:88, 96 through the clamp filter)
   const uint2* ztab;
+  const float* za;          // [l1-l0+1][nsinogs]: alpha_z alone
+  ZGroups zg[3];            // groups of 4, 6 and 8 planes
 };
 
 struct Taps9 { float g[9]; };
@@ -59,6 +74,7 @@ struct PackedRows {
 struct Tune {
   int back_zb = 8;   // slices per backprojector thread: 4, 5, 6, 8 or 16
   int zsum_sg = 8;   // consecutive sinograms per z-sum wave: 4, 6 or 8
+  int zsum_narrow = -1;  // narrow z-sum waves: 1, 0, or by size (-1)
   int back_lds = 0;  // 1: backprojector reads its rows through an LDS window
   int back_waves = 0;     // register budget for this many waves per SIMD (0: compiler's)
   int rot_z = 16;         // planes per rotation block: 4, 16 or 32
@@ -79,9 +95,13 @@ struct GeomHost {
   std::vector<SegEntry> seg;
   std::vector<int2> sino;
   std::vector<uint2> ztab;
+  std::vector<float> za;  // kZPad zeros after (groups read whole)
+  std::vector<int2> zgrp[3];
+  std::vector<uint32_t> zrow[3];
   float RADM, RESM, fxf, fxb;
 };
 
+constexpr int kZPad = 16;
 // with_ztab: also build the per-sample z table (device tables only need it).
 int derive_geometry(const gfr_geometry* g, GeomHost* out, std::string* err, bool with_ztab = false);
 void psf_taps(float psf, float* g9);
@@ -207,12 +227,11 @@ struct FwdOut {
   const void* bg = nullptr;       // background or NULL
   int storage = GFR_STORE_F32;
   float yscale = 1.f;             // RES
-  double* llh_part = nullptr;     // forward_llh_blocks() doubles, or NULL
+  double* llh_part = nullptr;     // llh_capacity() doubles, or NULL
 };
 // Scratch of the rotation stage: floats per angle; the launcher processes the
 // subset's angles in chunks of r_cap_floats / rotate_floats_per_angle().
 size_t rotate_floats_per_angle(const DevGeom& G);
-int forward_llh_blocks(const DevGeom& G, int subset, int nsub, int sg);
 // dsub: optional device pointer to the subset index (read by the kernels, so
 // a captured graph stays valid while the index changes); grids then cover
 // the largest subset.
@@ -237,8 +256,10 @@ hipError_t launch_back_multi(const DevGeom& G, const float* corr4, float* const*
 hipError_t launch_sensitivity(const DevGeom& G, const uint8_t* mask, float2* c2, double* sens,
                               int subset, int nsub, hipStream_t st);
 // FP64 log-likelihood of the last forward pass (sum of its block partials).
+// (r_cap_floats and tune: those of the forward pass)
 hipError_t launch_llh_sum(const DevGeom& G, const double* part, int subset, int nsub,
-                          const int* dsub, int sg, double* out, hipStream_t st);
+                          const int* dsub, size_t r_cap_floats, const Tune& tune, double* out,
+                          hipStream_t st);
 hipError_t launch_ratio(const DevGeom& G, const float* proj, const float* y, const void* bg,
                         int storage, float yscale, float* corr, const PackedRows& P,
                         const uint8_t* mask, int subset, int nsub, hipStream_t st);

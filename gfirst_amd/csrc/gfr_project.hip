@@ -178,141 +178,55 @@ struct FwdArgs {
 };
 
 // ---------------------------------------------------------------------------
-// k_zsum: one wave per (pair of angles, SG consecutive sinograms, 128 radial
-// bins). Half-wave h takes angle 2p + h of the chunk and lane l of the half
-// owns bins 4l .. 4l+3, so a row load is one 16-byte access per lane and one
-// instruction fetches a row of both angles (the z interpolation depends on
-// the sinogram and the sample, not on the angle). The z interpolation of a
-// sample is wave-uniform (scalar loads of the transposed z table). When the
-// group's samples at l blend planes z0, z0+1, ..., z0+SG (consecutive planes:
-// the usual case inside a segment), the SG+1 rows are loaded once for the
-// group; otherwise each LOR loads its own two rows. Every LOR still sums its
-// samples in l order with its own weights. Epilogue: ratio
-// (GFIRST.cu:415-430) and the FP64 Poisson log-likelihood partial of the
-// block (bins with valid calibration and den >= 0.01: sum of (y/RES)
-// ln(den/RES) - den/RES; the reference computes no likelihood).
+// z-sums: every LOR of sinogram s, angle a, bin r sums its samples in l order,
+// each the lerp of two rows of R with the sample's weight.
+// Epilogue per LOR: projection, ratio (GFIRST.cu:415-430), packed row, and the
+// FP64 Poisson log-likelihood partial of the block (bins with valid calibration
+// and den >= 0.01: sum of (y/RES) ln(den/RES) - den/RES; the reference computes
+// no likelihood).
 // ---------------------------------------------------------------------------
-template <int S, bool RATIO, bool LLH, int SG>
-__global__ __launch_bounds__(256) void k_zsum(DevGeom G, const float* __restrict__ R,
-                                              unsigned r_bytes, FwdArgs o, int subset, int nsub,
-                                              const int* __restrict__ dsub, int a0, int na,
-                                              int nl, unsigned llh_off) {
-  if (dsub) subset = *dsub;
-  const unsigned b = xcd_remap(blockIdx.x, gridDim.x);
-  const unsigned nrb = (G.nrad + 127) / 128, ngb = (G.nsinogs + 4 * SG - 1) / (4 * SG);
-  const unsigned rb = b % nrb;
-  const unsigned q = b / nrb;
-  const unsigned gb = q % ngb;
-  const int ap = (int)(q / ngb);
-  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int s0 = __builtin_amdgcn_readfirstlane((int)((gb * 4 + wv) * SG));
-  const int a = 2 * ap + (lane >> 5);  // angle of the chunk
-  const int r = (int)rb * 128 + 4 * (lane & 31);
-  const int nav = (G.nang - subset + nsub - 1) / nsub;
-  const int ag = a0 + a;
-  const int it = subset + ag * nsub;
-  if (a0 + 2 * ap >= nav) return;  // whole block: no angle of the pair in the subset
-  const bool aok = a < na && ag < nav;
-  double ll = 0.0;
-  if (s0 < G.nsinogs) {
-    const int ns = min(SG, G.nsinogs - s0);
-    // Lanes of an angle past the chunk read past r_bytes: zeros, unused.
-    const __amdgpu_buffer_rsrc_t rr = rsrc(R, r_bytes);
-    const unsigned rowb = (unsigned)G.nrad * 4u;
-    const unsigned planeb = rowb * (unsigned)G.nzs;
-    const unsigned voff = (unsigned)a * (unsigned)nl * planeb + (unsigned)r * 4u;
-    float4 acc[SG];
+// N <= 4 consecutive bins r .. of sinogram s, angle it (ag of the subset).
+template <int S, bool RATIO, bool LLH>
+__device__ __forceinline__ void emit(const DevGeom& G, const FwdArgs& o, int s, int ag, int it,
+                                     int r, int N, const float (&p)[4], double& ll) {
+  const size_t bin0 = ((size_t)s * G.nang + it) * G.nrad + r;
+  float c[4];
+  bool valid[4];
 #pragma unroll
-    for (int i = 0; i < SG; i++) acc[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-    unsigned soff = 0;
-    // z-table entries of sample li, loaded one sample ahead
-    uint2 en[SG];
-#pragma unroll
-    for (int i = 0; i < SG; i++) en[i] = G.ztab[s0 + (i < ns ? i : ns - 1)];
-    for (int li = 0; li < nl; li++, soff += planeb) {
-      uint2 e[SG];
-#pragma unroll
-      for (int i = 0; i < SG; i++) e[i] = en[i];
-      if (li + 1 < nl) {
-        const uint2* zt = G.ztab + (size_t)(li + 1) * G.nsinogs + s0;
-#pragma unroll
-        for (int i = 0; i < SG; i++) en[i] = zt[i < ns ? i : ns - 1];
-      }
-      const unsigned z00 = e[0].x & 0xFFFFu;
-      bool reg = true;
-#pragma unroll
-      for (int i = 0; i < SG; i++)
-        reg = reg && (e[i].x == ((z00 + i) | ((z00 + i + 1) << 16)));
-      if (reg) {
-        float4 row[SG + 1];
-#pragma unroll
-        for (int k = 0; k <= SG; k++) row[k] = ld_f4(rr, voff, soff + (z00 + k) * rowb);
-#pragma unroll
-        for (int i = 0; i < SG; i++) {
-          const float al = __uint_as_float(e[i].y);
-          acc[i].x += lerp1(row[i].x, row[i + 1].x, al);
-          acc[i].y += lerp1(row[i].y, row[i + 1].y, al);
-          acc[i].z += lerp1(row[i].z, row[i + 1].z, al);
-          acc[i].w += lerp1(row[i].w, row[i + 1].w, al);
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < SG; i++) {
-          const float al = __uint_as_float(e[i].y);
-          const float4 v0 = ld_f4(rr, voff, soff + (e[i].x & 0xFFFFu) * rowb);
-          const float4 v1 = ld_f4(rr, voff, soff + (e[i].x >> 16) * rowb);
-          acc[i].x += lerp1(v0.x, v1.x, al);
-          acc[i].y += lerp1(v0.y, v1.y, al);
-          acc[i].z += lerp1(v0.z, v1.z, al);
-          acc[i].w += lerp1(v0.w, v1.w, al);
-        }
-      }
-    }
-    if (aok) {
-#pragma unroll
-      for (int i = 0; i < SG; i++) {
-        if (i >= ns) break;
-        const int s = s0 + i;
-        const float av[4] = {acc[i].x, acc[i].y, acc[i].z, acc[i].w};
-        const int N = min(4, G.nrad - r);
-        const size_t bin0 = ((size_t)s * G.nang + it) * G.nrad + r;
-        float c[4];
-        bool valid[4];
-#pragma unroll
-        for (int h = 0; h < 4; h++) {
-          c[h] = 0.f;
-          valid[h] = true;
-          if (h >= N) continue;
-          const size_t bin = bin0 + h;
-          const float accv = av[h];
-          if (o.proj) o.proj[bin] = accv;
-          if constexpr (RATIO) {
-            const float yv = o.yscale * load_store<S>(o.y, bin);
-            float bv = o.bg ? o.yscale * load_store<S>(o.bg, bin) : 0.f;
-            if (bv < 0.f) bv = 0.f;
-            const float den = accv + bv;
-            c[h] = (den >= 0.01f) ? yv / den : -1000.f;
-            if (o.mask) valid[h] = o.mask[bin] != 0;
-            if (o.corr) o.corr[bin] = c[h];
-            if (o.corr4)
-              store_packed4(G, o.corr4, ag, s, r + h, o.chan, c[h], valid[h] ? 1.f : -1000.f);
-            if constexpr (LLH) {
-              // Poisson log-likelihood in count units over the bins whose
-              // ratio enters the backprojection: model mean den/RES, counts
-              // yv/RES (yv and den as the ratio sees them).
-              if (den >= 0.01f && valid[h]) {
-                const double m = (double)den / (double)o.yscale;
-                ll += ((double)yv / (double)o.yscale) * log(m) - m;
-              }
-            }
-          }
-        }
-        if constexpr (RATIO) {
-          if (o.rows.v && N > 0) store_packed(G, o.rows, ag, s, r, N, c, valid);
+  for (int h = 0; h < 4; h++) {
+    c[h] = 0.f;
+    valid[h] = true;
+    if (h >= N) continue;
+    const size_t bin = bin0 + h;
+    if (o.proj) o.proj[bin] = p[h];
+    if constexpr (RATIO) {
+      const float yv = o.yscale * load_store<S>(o.y, bin);
+      float bv = o.bg ? o.yscale * load_store<S>(o.bg, bin) : 0.f;
+      if (bv < 0.f) bv = 0.f;
+      const float den = p[h] + bv;
+      c[h] = (den >= 0.01f) ? yv / den : -1000.f;
+      if (o.mask) valid[h] = o.mask[bin] != 0;
+      if (o.corr) o.corr[bin] = c[h];
+      if (o.corr4)
+        store_packed4(G, o.corr4, ag, s, r + h, o.chan, c[h], valid[h] ? 1.f : -1000.f);
+      if constexpr (LLH) {
+        // Poisson log-likelihood in count units over the bins whose ratio
+        // enters the backprojection: model mean den/RES, counts yv/RES (yv
+        // and den as the ratio sees them).
+        if (den >= 0.01f && valid[h]) {
+          const double m = (double)den / (double)o.yscale;
+          ll += ((double)yv / (double)o.yscale) * log(m) - m;
         }
       }
     }
   }
+  if constexpr (RATIO) {
+    if (o.rows.v && N > 0) store_packed(G, o.rows, ag, s, r, N, c, valid);
+  }
+}
+
+template <bool LLH>
+__device__ __forceinline__ void block_llh(double ll, double* part) {
   if constexpr (LLH) {
     __shared__ double red[256];
     const int t = threadIdx.x;
@@ -322,8 +236,177 @@ __global__ __launch_bounds__(256) void k_zsum(DevGeom G, const float* __restrict
       if (t < w) red[t] += red[t + w];
       __syncthreads();
     }
-    if (t == 0) o.llh_part[llh_off + b] = red[0];
+    if (t == 0) *part = red[0];
   }
+}
+
+// Wide waves: one wave per (64 quads of bins, group of SG planes of a segment).
+// Its lanes are consecutive (angle, 4 bins) items, so a row load is one 16-byte
+// access per lane and a wave is full whatever the bin count; the SG LORs of a
+// lane share SG + 1 rows. The waves of an angle walk the samples together and
+// are the first to touch a sample's rows, so a load waits for memory and not
+// for L2: the rows of the next sample are requested before the current one is
+// summed. Row and weights of a sample are wave-uniform (scalar loads, further
+// ahead). Samples whose LORs do not blend consecutive rows (at the volume's
+// ends) load each LOR's two rows.
+template <int S, bool RATIO, bool LLH, int SG>
+__global__ __launch_bounds__(256) void k_zsum_wide(DevGeom G, const float* __restrict__ R,
+                                                   unsigned r_bytes, FwdArgs o, int subset,
+                                                   int nsub, const int* __restrict__ dsub, int a0,
+                                                   int na, int nl, unsigned llh_off) {
+  if (dsub) subset = *dsub;
+  const ZGroups zg = G.zg[zg_index(SG)];
+  const unsigned b = xcd_remap(blockIdx.x, gridDim.x);
+  const int nq = (G.nrad + 3) / 4, ngb = (zg.n + 3) / 4;
+  const int ib = (int)(b / (unsigned)ngb), gb = (int)(b % (unsigned)ngb);
+  const int nav = (G.nang - subset + nsub - 1) / nsub;
+  if (a0 + ib * 64 / nq >= nav) return;  // whole block: no angle of the subset
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int item = ib * 64 + (int)(threadIdx.x & 63);
+  const int a = item / nq, r = 4 * (item - a * nq);
+  const int ag = a0 + a, it = subset + ag * nsub;
+  const int gi = gb * 4 + wv;
+  double ll = 0.0;
+  const int2 grp = zg.s[gi];  // zg.n is a multiple of 4
+  const int ng = grp.y < 0 ? -grp.y : grp.y;
+  if (ng > 0) {
+    const __amdgpu_buffer_rsrc_t rr = rsrc(R, r_bytes);
+    const unsigned rowb = (unsigned)G.nrad * 4u;
+    const unsigned planeb = rowb * (unsigned)G.nzs;
+    // Lanes past the chunk's angles read past r_bytes: zeros, unused.
+    const unsigned voff = (unsigned)a * (unsigned)nl * planeb + (unsigned)r * 4u;
+    float4 acc[SG];
+#pragma unroll
+    for (int i = 0; i < SG; i++) acc[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    auto add = [&](float4& c, const float4& v0, const float4& v1, float al) {
+      c.x += lerp1(v0.x, v1.x, al);
+      c.y += lerp1(v0.y, v1.y, al);
+      c.z += lerp1(v0.z, v1.z, al);
+      c.w += lerp1(v0.w, v1.w, al);
+    };
+    const uint32_t* rows = zg.row + gi;
+    const float* wts = G.za + grp.x;
+    unsigned soff = 0;
+    if (grp.y > 0) {
+      float e[SG];
+      uint32_t z = rows[0];
+#pragma unroll
+      for (int i = 0; i < SG; i++) e[i] = wts[i];
+      for (int li = 0; li < nl; li++, soff += planeb) {
+        const unsigned base = soff + (z & ~kZReg) * rowb;
+        float4 row[SG + 1];
+#pragma unroll
+        for (int k = 0; k <= SG; k++) row[k] = ld_f4(rr, voff, base + (unsigned)k * rowb);
+        float en[SG];
+        if (li + 1 < nl) {  // the next sample's, while the rows come
+          rows += zg.n;
+          wts += G.nsinogs;
+        }
+        z = rows[0];
+#pragma unroll
+        for (int i = 0; i < SG; i++) en[i] = wts[i];
+#pragma unroll
+        for (int i = 0; i < SG; i++) add(acc[i], row[i], row[i + 1], e[i]);
+#pragma unroll
+        for (int i = 0; i < SG; i++) e[i] = en[i];
+      }
+    } else {
+      for (int li = 0; li < nl; li++, soff += planeb) {
+        const uint2* t = G.ztab + (size_t)li * G.nsinogs + grp.x;
+#pragma unroll
+        for (int i = 0; i < SG; i++) {
+          const uint2 q = t[i < ng ? i : 0];
+          add(acc[i], ld_f4(rr, voff, soff + (q.x & 0xffffu) * rowb),
+              ld_f4(rr, voff, soff + (q.x >> 16) * rowb), __uint_as_float(q.y));
+        }
+      }
+    }
+    if (a < na && ag < nav) {
+      const int N = min(4, G.nrad - r);
+#pragma unroll
+      for (int i = 0; i < SG; i++) {
+        if (i >= ng) break;
+        const float p[4] = {acc[i].x, acc[i].y, acc[i].z, acc[i].w};
+        emit<S, RATIO, LLH>(G, o, grp.x + i, ag, it, r, N, p, ll);
+      }
+    }
+  }
+  block_llh<LLH>(ll, o.llh_part + llh_off + b);
+}
+
+// Narrow waves for small sinograms, where a few hundred wide waves would each
+// walk the samples one memory round trip at a time: one wave per (64 bins of
+// consecutive angles, 2 sinograms), the rows of 4 samples requested together.
+template <int S, bool RATIO, bool LLH>
+__global__ __launch_bounds__(256) void k_zsum_narrow(DevGeom G, const float* __restrict__ R,
+                                                     unsigned r_bytes, FwdArgs o, int subset,
+                                                     int nsub, const int* __restrict__ dsub,
+                                                     int a0, int na, int nl, unsigned llh_off) {
+  constexpr int LA = 4;
+  if (dsub) subset = *dsub;
+  const unsigned b = xcd_remap(blockIdx.x, gridDim.x);
+  const int ngb = (G.nsinogs + 7) / 8;
+  const int ib = (int)(b / (unsigned)ngb), gb = (int)(b % (unsigned)ngb);
+  const int nav = (G.nang - subset + nsub - 1) / nsub;
+  if (a0 + ib * 64 / G.nrad >= nav) return;  // whole block: no angle of the subset
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int item = ib * 64 + (int)(threadIdx.x & 63);
+  const int a = item / G.nrad, r = item - a * G.nrad;
+  const int ag = a0 + a, it = subset + ag * nsub;
+  const int s0 = 2 * (gb * 4 + wv);
+  double ll = 0.0;
+  if (s0 < G.nsinogs) {
+    const int s1 = min(s0 + 1, G.nsinogs - 1);
+    const __amdgpu_buffer_rsrc_t rr = rsrc(R, r_bytes);
+    const unsigned rowb = (unsigned)G.nrad * 4u;
+    const unsigned planeb = rowb * (unsigned)G.nzs;
+    const unsigned voff = (unsigned)a * (unsigned)nl * planeb + (unsigned)r * 4u;
+    float p0 = 0.f, p1 = 0.f;
+    uint2 e0[LA], e1[LA];
+    auto entries = [&](int l0) {
+#pragma unroll
+      for (int u = 0; u < LA; u++) {
+        const uint2* t = G.ztab + (size_t)min(l0 + u, nl - 1) * G.nsinogs;
+        e0[u] = t[s0];
+        e1[u] = t[s1];
+      }
+    };
+    float v[LA][4];
+    auto load = [&](int l0) {
+#pragma unroll
+      for (int u = 0; u < LA; u++) {
+        const unsigned so = (unsigned)min(l0 + u, nl - 1) * planeb;
+        v[u][0] = ld_f1(rr, voff, so + (e0[u].x & 0xffffu) * rowb);
+        v[u][1] = ld_f1(rr, voff, so + (e0[u].x >> 16) * rowb);
+        v[u][2] = ld_f1(rr, voff, so + (e1[u].x & 0xffffu) * rowb);
+        v[u][3] = ld_f1(rr, voff, so + (e1[u].x >> 16) * rowb);
+      }
+    };
+    entries(0);
+    for (int l0 = 0; l0 < nl; l0 += LA) {
+      load(l0);
+      float w0[LA], w1[LA];
+#pragma unroll
+      for (int u = 0; u < LA; u++) {
+        w0[u] = __uint_as_float(e0[u].y);
+        w1[u] = __uint_as_float(e1[u].y);
+      }
+      if (l0 + LA < nl) entries(l0 + LA);
+#pragma unroll
+      for (int u = 0; u < LA; u++) {
+        if (l0 + u < nl) {
+          p0 += lerp1(v[u][0], v[u][1], w0[u]);
+          p1 += lerp1(v[u][2], v[u][3], w1[u]);
+        }
+      }
+    }
+    if (a < na && ag < nav) {
+      const float q0[4] = {p0, 0.f, 0.f, 0.f}, q1[4] = {p1, 0.f, 0.f, 0.f};
+      emit<S, RATIO, LLH>(G, o, s0, ag, it, r, 1, q0, ll);
+      if (s0 + 1 < G.nsinogs) emit<S, RATIO, LLH>(G, o, s0 + 1, ag, it, r, 1, q1, ll);
+    }
+  }
+  block_llh<LLH>(ll, o.llh_part + llh_off + b);
 }
 
 // Full-layout ratio + byte mask -> packed rows of a subset.
@@ -747,38 +830,75 @@ size_t rotate_floats_per_angle(const DevGeom& G) {
   return (size_t)(G.l1 - G.l0 + 1) * G.nzs * G.nrad;
 }
 
-// z-sum blocks (= log-likelihood partials) per pair of angles, and in all
-int zsum_blocks_per_pair(const DevGeom& G, int sg) {
-  return ((G.nrad + 127) / 128) * ((G.nsinogs + 4 * sg - 1) / (4 * sg));
-}
-
-int forward_llh_blocks(const DevGeom& G, int subset, int nsub, int sg) {
-  return zsum_blocks_per_pair(G, sg) * ((nav_of(G, subset, nsub) + 1) / 2);
-}
-
 namespace {
 
-template <int SG>
-hipError_t zsum_launch(const DevGeom& G, const float* R, unsigned rbytes, const FwdArgs& o,
-                       bool ratio, int storage, int subset, int nsub, const int* dsub, int a0,
-                       int na, int nl, hipStream_t st) {
-  // a0 is even (chunks hold whole pairs of angles)
-  const unsigned per = (unsigned)zsum_blocks_per_pair(G, SG);
-  const unsigned gz = per * (unsigned)((na + 1) / 2);
-  const unsigned off = per * (unsigned)(a0 / 2);
-  if (!ratio) {
-    hipLaunchKernelGGL((k_zsum<GFR_STORE_F32, false, false, SG>), dim3(gz), dim3(256), 0, st, G,
-                       R, rbytes, o, subset, nsub, dsub, a0, na, nl, off);
-    return hipGetLastError();
+// z-sum blocks (= log-likelihood partials): along the sinograms, and for na
+// angles of a chunk.
+__host__ __device__ inline int zsum_ngb(bool wide, int ngroups, int nsinogs) {
+  return wide ? (ngroups + 3) / 4 : (nsinogs + 7) / 8;  // 4 waves a block
+}
+__host__ __device__ inline int zsum_nib(bool wide, int nrad, int na) {
+  return (na * (wide ? (nrad + 3) / 4 : nrad) + 63) / 64;
+}
+
+// Blocks (partials) of a pass over nav angles in chunks of kRotChunk.
+inline int zsum_blocks(bool wide, int ngroups, int nsinogs, int nrad, int nav) {
+  return zsum_ngb(wide, ngroups, nsinogs) *
+         (nav / kRotChunk * zsum_nib(wide, nrad, kRotChunk) + zsum_nib(wide, nrad, nav % kRotChunk));
+}
+// The narrow kernel serves passes up to this many of its blocks (measured,
+// narrow / best wide, us of a whole projection: 368 blocks 26 / 60, 750 40 / 79,
+// 1472 53 / 66, 2016 89 / 98, 2466 104 / 107, 2745 94 / 85, 4575 141 / 98).
+constexpr int kNarrowBlocks = 2400;
+
+// Which kernel a pass over nav angles takes: sinograms per wave, or 0 for the
+// narrow one. Where no measurement says: the narrow one where it serves, 4
+// sinograms where 6 leave too few waves (3.3M LORs a pass 150 us with 4, 163
+// with 6; 4.8M 202 and 170).
+int zsum_kind(const DevGeom& G, const Tune& tune, int nav) {
+  const bool fits = zsum_blocks(false, 0, G.nsinogs, G.nrad, nav) <= kNarrowBlocks;
+  if (fits && tune.zsum_narrow != 0) return 0;
+  if (tune.tuned) return tune.zsum_sg;
+  return (long long)G.nsinogs * nav * G.nrad < 3800000 ? 4 : 6;
+}
+
+// Angles per rotation chunk for nav angles.
+int forward_chunk(const DevGeom& G, int nav, size_t r_cap_floats) {
+  const size_t per = rotate_floats_per_angle(G);
+  size_t chunk = r_cap_floats / per;
+  if (chunk > (size_t)nav) chunk = nav;
+  if (chunk * per * sizeof(float) >= 0xFFFFFFF0u) chunk = 0xFFFFFFF0u / (per * 4);
+  return (int)chunk;
+}
+
+int zsum_ngb_of(const DevGeom& G, int kind) {
+  return zsum_ngb(kind != 0, kind ? G.zg[zg_index(kind)].n : 0, G.nsinogs);
+}
+
+hipError_t zsum_launch(const DevGeom& G, int kind, const float* R, unsigned rbytes,
+                       const FwdArgs& o, bool ratio, int storage, int subset, int nsub,
+                       const int* dsub, int a0, int na, int nl, unsigned llh_off, hipStream_t st) {
+  const unsigned blocks =
+      (unsigned)zsum_ngb_of(G, kind) * (unsigned)zsum_nib(kind != 0, G.nrad, na);
+#define GFR_ZK(K)                                                                             \
+  hipLaunchKernelGGL(K, dim3(blocks), dim3(256), 0, st, G, R, rbytes, o, subset, nsub, dsub, \
+                     a0, na, nl, llh_off)
+#define GFR_ZL(S, RT, LL)                                      \
+  switch (kind) {                                              \
+    case 0: GFR_ZK((k_zsum_narrow<S, RT, LL>)); break;         \
+    case 4: GFR_ZK((k_zsum_wide<S, RT, LL, 4>)); break;        \
+    case 6: GFR_ZK((k_zsum_wide<S, RT, LL, 6>)); break;        \
+    default: GFR_ZK((k_zsum_wide<S, RT, LL, 8>)); break;       \
   }
-#define GFR_ZS(S)                                                                             \
-  if (o.llh_part)                                                                             \
-    hipLaunchKernelGGL((k_zsum<S, true, true, SG>), dim3(gz), dim3(256), 0, st, G, R, rbytes, \
-                       o, subset, nsub, dsub, a0, na, nl, off);                                   \
-  else                                                                                        \
-    hipLaunchKernelGGL((k_zsum<S, true, false, SG>), dim3(gz), dim3(256), 0, st, G, R,       \
-                       rbytes, o, subset, nsub, dsub, a0, na, nl, off);
-  if (storage == GFR_STORE_F16) {
+#define GFR_ZS(S)              \
+  if (o.llh_part) {            \
+    GFR_ZL(S, true, true)      \
+  } else {                     \
+    GFR_ZL(S, true, false)     \
+  }
+  if (!ratio) {
+    GFR_ZL(GFR_STORE_F32, false, false)
+  } else if (storage == GFR_STORE_F16) {
     GFR_ZS(GFR_STORE_F16)
   } else if (storage == GFR_STORE_BF16) {
     GFR_ZS(GFR_STORE_BF16)
@@ -786,15 +906,20 @@ hipError_t zsum_launch(const DevGeom& G, const float* R, unsigned rbytes, const 
     GFR_ZS(GFR_STORE_F32)
   }
 #undef GFR_ZS
+#undef GFR_ZL
+#undef GFR_ZK
   return hipGetLastError();
 }
 
-// Deterministic sum of the first n(subset) partials; with dsub the count
-// follows the device-side subset index.
-__global__ void k_llh_sum(const double* __restrict__ part, int per_pair, int nang, int subset,
-                          int nsub, const int* __restrict__ dsub, double* __restrict__ out) {
+// Deterministic sum of the partials of the subset's angles (full chunks of
+// `full` partials each, then the last one's); with dsub the count follows the
+// device-side subset index.
+__global__ void k_llh_sum(const double* __restrict__ part, int wide, int ngb, int nrad, int chunk,
+                          int nang, int subset, int nsub, const int* __restrict__ dsub,
+                          double* __restrict__ out) {
   if (dsub) subset = *dsub;
-  const int n = per_pair * (((nang - subset + nsub - 1) / nsub + 1) / 2);
+  const int nav = (nang - subset + nsub - 1) / nsub;
+  const int n = ngb * (nav / chunk * zsum_nib(wide, nrad, chunk) + zsum_nib(wide, nrad, nav % chunk));
   __shared__ double red[256];
   double acc = 0.0;
   for (int i = threadIdx.x; i < n; i += 256) acc += part[i];
@@ -816,14 +941,11 @@ hipError_t launch_forward(const DevGeom& G, const float* img, float* R, size_t r
   const int nav = dsub ? nav_of(G, 0, nsub) : nav_of(G, subset, nsub);
   const int nl = G.l1 - G.l0 + 1;
   const size_t per = rotate_floats_per_angle(G);
-  int chunk = (int)(r_cap_floats / per);
+  const int chunk = forward_chunk(G, nav, r_cap_floats);
   if (chunk < 1) return hipErrorInvalidValue;
-  if (chunk > nav) chunk = nav;
-  if ((size_t)chunk * per * sizeof(float) >= 0xFFFFFFF0u) chunk = (int)(0xFFFFFFF0u / (per * 4));
-  if (chunk < nav && chunk > 1) chunk &= ~1;  // the z-sum takes angles in pairs
-  if (chunk < 1) return hipErrorInvalidValue;
-  // log-likelihood partials are indexed by pair: chunks must hold whole pairs
-  if (out.llh_part && chunk < nav && (chunk & 1)) return hipErrorInvalidValue;
+  const int kind = zsum_kind(G, tune, nav);
+  const unsigned llh_per_chunk =
+      (unsigned)zsum_ngb_of(G, kind) * (unsigned)zsum_nib(kind != 0, G.nrad, chunk);
   if (out.corr4 && (out.chan < 0 || out.chan >= kMaxGroup)) return hipErrorInvalidValue;
   FwdArgs o{out.proj, out.corr,  out.rows,   out.corr4,   out.chan,
             out.mask, out.y,     out.bg,     out.yscale,  out.llh_part};
@@ -846,20 +968,22 @@ hipError_t launch_forward(const DevGeom& G, const float* img, float* R, size_t r
                          img, R, subset, nsub, dsub, a0, nl, zouter);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    switch (tune.zsum_sg) {
-      case 4: e = zsum_launch<4>(G, R, rbytes, o, ratio, out.storage, subset, nsub, dsub, a0, na, nl, st); break;
-      case 6: e = zsum_launch<6>(G, R, rbytes, o, ratio, out.storage, subset, nsub, dsub, a0, na, nl, st); break;
-      default: e = zsum_launch<8>(G, R, rbytes, o, ratio, out.storage, subset, nsub, dsub, a0, na, nl, st); break;
-    }
+    e = zsum_launch(G, kind, R, rbytes, o, ratio, out.storage, subset, nsub, dsub, a0, na, nl,
+                    llh_per_chunk * (unsigned)(a0 / chunk), st);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
 }
 
 hipError_t launch_llh_sum(const DevGeom& G, const double* part, int subset, int nsub,
-                          const int* dsub, int sg, double* out, hipStream_t st) {
-  hipLaunchKernelGGL(k_llh_sum, dim3(1), dim3(256), 0, st, part, zsum_blocks_per_pair(G, sg),
-                     G.nang, subset, nsub, dsub, out);
+                          const int* dsub, size_t r_cap_floats, const Tune& tune, double* out,
+                          hipStream_t st) {
+  const int nav = nav_of(G, dsub ? 0 : subset, nsub);
+  const int chunk = forward_chunk(G, nav, r_cap_floats);
+  if (chunk < 1) return hipErrorInvalidValue;
+  const int kind = zsum_kind(G, tune, nav);
+  hipLaunchKernelGGL(k_llh_sum, dim3(1), dim3(256), 0, st, part, kind != 0, zsum_ngb_of(G, kind),
+                     G.nrad, chunk, G.nang, subset, nsub, dsub, out);
   return hipGetLastError();
 }
 
@@ -925,7 +1049,12 @@ hipError_t launch_sensitivity(const DevGeom& G, const uint8_t* mask, float2* c2,
 
 int llh_capacity(const GeomHost& h, int nsub) {
   const int nav = (h.g.nang + nsub - 1) / nsub;
-  return ((h.g.nrad + 127) / 128) * ((h.info.nsinogs + 15) / 16) * ((nav + 1) / 2);  // zsum_sg = 4
+  const int wide = zsum_blocks(true, (int)h.zgrp[0].size(), h.info.nsinogs, h.g.nrad, nav);
+  const int narrow = zsum_blocks(false, 0, h.info.nsinogs, h.g.nrad, nav);
+  int most = ((h.g.nrad + 127) / 128) * ((h.info.nsinogs + 15) / 16) * ((nav + 1) / 2);
+  if (wide > most) most = wide;
+  if (narrow <= kNarrowBlocks && narrow > most) most = narrow;
+  return most;
 }
 
 hipError_t tune_shapes(const DevGeom& G, int nsub, const FwdOut& fo, const float* img, float* R,
@@ -952,17 +1081,20 @@ hipError_t tune_shapes(const DevGeom& G, int nsub, const FwdOut& fo, const float
     return best;
   };
   Tune t;
-  const int cand[3] = {4, 6, 8};
+  t.tuned = true;
+  const int cand[4] = {4, 6, 8, 0};  // 0: narrow waves
   float bz = 1e30f, bb = 1e30f;
   for (int c : cand) {
     Tune tt = t;
-    tt.zsum_sg = c;
+    tt.zsum_narrow = c == 0;
+    if (c) tt.zsum_sg = c;
     const float ms = time_it([&] {
       return launch_forward(G, img, R, r_floats, fo, 0, nsub, nullptr, tt, st);
     });
     if (ms < bz) {
       bz = ms;
-      t.zsum_sg = c;
+      t.zsum_sg = tt.zsum_sg;
+      t.zsum_narrow = tt.zsum_narrow;
     }
   }
   const int rcand[3] = {4, 16, 32};  // planes per rotation block

@@ -489,7 +489,7 @@ int gfr_recon_step(gfr_recon* r) {
       fo.llh_part = llh_part;
       GFR_HIP(ctx, launch_forward(G, xb, R, r->r_floats, fo, s, S, nullptr, r->tune, st));
     }
-    GFR_HIP(ctx, launch_llh_sum(G, llh_part, s, S, nullptr, r->tune.zsum_sg, d_llh, st));
+    GFR_HIP(ctx, launch_llh_sum(G, llh_part, s, S, nullptr, r->r_floats, r->tune, d_llh, st));
     r->llh_valid = 1;
     r->llh_chain = tc ? 1 : 0;
   }
