@@ -30,33 +30,47 @@ namespace {
 // ---------------------------------------------------------------------------
 // k_rotate_tile: R[a][l][z][r], the bilinear sample of image plane z at the
 // position of (bin r, sample l) of angle a. A block takes one angle, a tile
-// of 32 bins x 32 samples and ZC planes (autotuned). The tile's sample
+// of 32 bins x up to 40 samples and ZC planes (autotuned). The tile's sample
 // points fall in a rotated rectangle of the image; since x and y (and then
 // the clamped texel indices) are monotone in r and l, the texels the tile
-// touches lie in the bounding box of its four corner samples. Per plane
-// the block copies that box into LDS with coalesced row loads (the next
-// plane's rows are in flight while the current one is used) and every
-// output reads its four texels from LDS. A box larger than the LDS tile
-// (coarse geometries) falls back to gathers from global memory.
+// touches lie in the bounding box of its four corner samples. Per pair of
+// planes the block copies that box into LDS with coalesced row loads, the two
+// planes side by side (the next pair's rows are in flight while the current
+// one is used), and every output reads its four texels of both planes from
+// LDS. A box larger than the LDS tile (coarse geometries) falls back to
+// gathers from global memory.
+// What bounds it: the loads and barriers of a plane, not bytes or arithmetic;
+// two planes a turn halve them, and tiles of equal height (129 samples in four
+// tiles of 33 instead of 32 + 32 + 32 + 32 + 1) save a fifth of the blocks:
+// 10 angles at 128x128x159 59 -> 35 us, 16 at 147x147x239 84 -> 55 us (write
+// floors at the rate of a large copy, 16 and 32 us).
 // ---------------------------------------------------------------------------
-constexpr int kRotTile = 64;         // LDS box capacity: texels per row and rows
-constexpr int kRotStride = kRotTile + 1;  // LDS row stride (odd: rows on different banks)
+constexpr int kRotTile = 64;  // largest LDS box: texels per row and rows
+constexpr int kRotOut = 5;    // samples per thread: tiles of up to 40
+
+// Samples per tile: as few tiles as tiles of up to 40 give, of equal height.
+__host__ __device__ inline int rot_tile_samples(int nl) {
+  const int n = (nl + 8 * kRotOut - 1) / (8 * kRotOut);
+  return (nl + n - 1) / n;
+}
 
 template <int ZC>
 __global__ __launch_bounds__(256) void k_rotate_tile(DevGeom G, const float* __restrict__ img,
                                                      float* __restrict__ R, int subset, int nsub,
                                                      const int* __restrict__ dsub, int a0,
-                                                     int nl, int zouter) {
-  __shared__ float box[kRotTile * kRotStride];
+                                                     int nl, int zouter, int side) {
+  extern __shared__ float2 box[];  // side rows of side | 1 texels (odd: rows on different banks)
+  const int stride = side | 1;
   if (dsub) subset = *dsub;
   // Logical order: bin tile, sample tile, then angle and plane chunk; every
   // XCD walks one contiguous range of logical blocks. With zouter the plane
   // chunk is outermost: an XCD rotates a few plane chunks for every angle
   // and reads each image plane once into its L2 (rotation outputs larger than
-  // an L2). Otherwise the angle is: an XCD writes the angles whose pairs its
-  // z-sum blocks read next, while they are still in its L2.
+  // an L2). Otherwise the angle is: an XCD writes the angles whose z-sum blocks
+  // it reads next, while they are still in its L2.
   const unsigned b = xcd_remap(blockIdx.x, gridDim.x);
-  const unsigned nrt = (G.nrad + 31) / 32, nlt = (nl + 31) / 32;
+  const int tl = rot_tile_samples(nl);
+  const unsigned nrt = (G.nrad + 31) / 32, nlt = (nl + tl - 1) / tl;
   const unsigned nzc = (G.nzs + ZC - 1) / ZC;
   const unsigned na = gridDim.x / (nrt * nlt * nzc);
   const unsigned rt = b % nrt;
@@ -80,7 +94,7 @@ __global__ __launch_bounds__(256) void k_rotate_tile(DevGeom G, const float* __r
     axis(fmaf(fl, -ct, yc), G.res, y0i, y1i, ay);  // dy = -cos(theta) (:82)
   };
   const int rlo = (int)rt * 32, rhi = min(rlo + 31, G.nrad - 1);
-  const int llo = (int)lt * 32, lhi = min(llo + 31, nl - 1);
+  const int llo = (int)lt * tl, lhi = min(llo + tl, nl) - 1;
   int bx0 = G.res, bx1 = -1, by0 = G.res, by1 = -1;
 #pragma unroll
   for (int c = 0; c < 4; c++) {
@@ -93,27 +107,22 @@ __global__ __launch_bounds__(256) void k_rotate_tile(DevGeom G, const float* __r
     by1 = max(by1, y1i);
   }
   const int bw = bx1 - bx0 + 1, bh = by1 - by0 + 1;
-  const bool staged = bw <= kRotTile && bh <= kRotTile;
-  // this thread's four outputs: bin rlo + (tid & 31), samples llo + (tid >> 5) + 8k
+  const bool staged = bw <= side && bh <= side;
+  // this thread's outputs: bin rlo + (tid & 31), samples llo + (tid >> 5) + 8k
   const int r = rlo + (tid & 31);
-  int o00[4], dx[4], dy[4];
-  float ax[4], ay[4];
-  bool ok[4];
+  int o00[kRotOut], dx[kRotOut], dy[kRotOut];
+  float ax[kRotOut], ay[kRotOut];
+  bool ok[kRotOut];
 #pragma unroll
-  for (int k = 0; k < 4; k++) {
+  for (int k = 0; k < kRotOut; k++) {
     const int li = llo + (tid >> 5) + 8 * k;
-    ok[k] = r < G.nrad && li < nl;
+    ok[k] = r < G.nrad && li <= lhi;
     int x0i, x1i, y0i, y1i;
-    texels(r, li, x0i, x1i, ax[k], y0i, y1i, ay[k]);
-    if (staged) {
-      o00[k] = (y0i - by0) * kRotStride + (x0i - bx0);
-      dx[k] = x1i - x0i;
-      dy[k] = (y1i - y0i) * kRotStride;
-    } else {
-      o00[k] = y0i * G.res + x0i;
-      dx[k] = x1i - x0i;
-      dy[k] = (y1i - y0i) * G.res;
-    }
+    texels(r, min(li, lhi), x0i, x1i, ax[k], y0i, y1i, ay[k]);
+    const int w = staged ? stride : G.res;
+    o00[k] = staged ? (y0i - by0) * w + (x0i - bx0) : y0i * w + x0i;
+    dx[k] = x1i - x0i;
+    dy[k] = (y1i - y0i) * w;
   }
   const size_t plane = (size_t)G.res * G.res;
   const int nz = min(ZC, G.nzs - zc);
@@ -123,7 +132,7 @@ __global__ __launch_bounds__(256) void k_rotate_tile(DevGeom G, const float* __r
     for (int zi = 0; zi < nz; zi++) {
       const float* pk = img + (size_t)(zc + zi) * plane;
 #pragma unroll
-      for (int k = 0; k < 4; k++) {
+      for (int k = 0; k < kRotOut; k++) {
         if (ok[k]) {
           const float* p = pk + o00[k];
           out[k * lstep + (size_t)zi * G.nrad] =
@@ -137,27 +146,35 @@ __global__ __launch_bounds__(256) void k_rotate_tile(DevGeom G, const float* __r
   const int lc = tid & 63, lr = tid >> 6;
   const int nj = (bh + 3) >> 2;
   const float* src = img + (size_t)(by0 + lr) * G.res + bx0 + lc;
-  float pre[kRotTile / 4];
-  auto fetch = [&](int z) {
-    const float* pz = src + (size_t)z * plane;
+  float2 pre[kRotTile / 4];
+  auto fetch = [&](int z) {  // planes z and z + 1 (the last one again past the end)
+    const float* p0 = src + (size_t)z * plane;
+    const float* p1 = src + (size_t)min(z + 1, G.nzs - 1) * plane;
 #pragma unroll
     for (int j = 0; j < kRotTile / 4; j++)
-      if (j < nj && lc < bw && lr + 4 * j < bh) pre[j] = pz[(size_t)(4 * j) * G.res];
+      if (j < nj && lc < bw && lr + 4 * j < bh) {
+        const size_t o = (size_t)(4 * j) * G.res;
+        pre[j] = make_float2(p0[o], p1[o]);
+      }
   };
   fetch(zc);
-  for (int zi = 0; zi < nz; zi++) {
-    __syncthreads();  // the previous plane's reads are done
+  for (int zi = 0; zi < nz; zi += 2) {
+    __syncthreads();  // the previous planes' reads are done
 #pragma unroll
     for (int j = 0; j < kRotTile / 4; j++)
-      if (j < nj && lc < bw && lr + 4 * j < bh) box[(lr + 4 * j) * kRotStride + lc] = pre[j];
+      if (j < nj && lc < bw && lr + 4 * j < bh) box[(lr + 4 * j) * stride + lc] = pre[j];
     __syncthreads();
-    if (zi + 1 < nz) fetch(zc + zi + 1);
+    if (zi + 2 < nz) fetch(zc + zi + 2);
+    const bool two = zi + 1 < nz;
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
+    for (int k = 0; k < kRotOut; k++) {
       if (ok[k]) {
-        const float* p = box + o00[k];
-        out[k * lstep + (size_t)zi * G.nrad] =
-            lerp1(lerp1(p[0], p[dx[k]], ax[k]), lerp1(p[dy[k]], p[dy[k] + dx[k]], ax[k]), ay[k]);
+        const float2* p = box + o00[k];
+        const float2 v00 = p[0], v01 = p[dx[k]], v10 = p[dy[k]], v11 = p[dy[k] + dx[k]];
+        float* w = out + k * lstep + (size_t)zi * G.nrad;
+        w[0] = lerp1(lerp1(v00.x, v01.x, ax[k]), lerp1(v10.x, v11.x, ax[k]), ay[k]);
+        if (two)
+          w[G.nrad] = lerp1(lerp1(v00.y, v01.y, ax[k]), lerp1(v10.y, v11.y, ax[k]), ay[k]);
       }
     }
   }
@@ -953,19 +970,25 @@ hipError_t launch_forward(const DevGeom& G, const float* img, float* R, size_t r
   for (int a0 = 0; a0 < nav; a0 += chunk) {
     const int na = min(chunk, nav - a0);
     const unsigned rbytes = (unsigned)((size_t)na * per * sizeof(float));
-    const unsigned gxy = ((G.nrad + 31) / 32) * ((nl + 31) / 32) * na;
+    const int tl = rot_tile_samples(nl);
+    const unsigned gxy = ((G.nrad + 31) / 32) * ((nl + tl - 1) / tl) * na;
     // plane chunks outermost when an angle pair's rotation exceeds an XCD's
     // 4 MiB L2 (the z-sum cannot find it there anyway)
     const int zouter = 2 * per * sizeof(float) > ((size_t)4 << 20);
-    if (tune.rot_z == 4)
-      hipLaunchKernelGGL(k_rotate_tile<4>, dim3(gxy * ((G.nzs + 3) / 4)), dim3(256), 0, st, G, img,
-                         R, subset, nsub, dsub, a0, nl, zouter);
-    else if (tune.rot_z == 32)
-      hipLaunchKernelGGL(k_rotate_tile<32>, dim3(gxy * ((G.nzs + 31) / 32)), dim3(256), 0, st, G,
-                         img, R, subset, nsub, dsub, a0, nl, zouter);
-    else
-      hipLaunchKernelGGL(k_rotate_tile<16>, dim3(gxy * ((G.nzs + 15) / 16)), dim3(256), 0, st, G,
-                         img, R, subset, nsub, dsub, a0, nl, zouter);
+    // texels a tile can touch: its diagonal's span, the interpolation partner and rounding
+    const float diag = sqrtf(31.f * G.fxf * 31.f * G.fxf + (float)((tl - 1) * (tl - 1)));
+    const int side = min(kRotTile, min((int)diag + 4, G.res));
+    const unsigned lds = (unsigned)(side * (side | 1) * sizeof(float2));
+    // planes per block: 16, or 4 where that alone makes enough blocks (64 angles
+    // at 64x64x32: the pass 53 us with 16, 49 with 4)
+    const int rz = tune.tuned ? tune.rot_z : kind == 0 ? 4 : 16;
+#define GFR_RT(ZC)                                                                                \
+  hipLaunchKernelGGL(k_rotate_tile<ZC>, dim3(gxy * ((G.nzs + ZC - 1) / ZC)), dim3(256), lds, st, G, \
+                     img, R, subset, nsub, dsub, a0, nl, zouter, side)
+    if (rz == 4) GFR_RT(4);
+    else if (rz == 32) GFR_RT(32);
+    else GFR_RT(16);
+#undef GFR_RT
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     e = zsum_launch(G, kind, R, rbytes, o, ratio, out.storage, subset, nsub, dsub, a0, na, nl,
