@@ -178,123 +178,193 @@ __global__ __launch_bounds__(256) void k_jbf(int res, int nzs, const float* __re
   out[iV] = ((double)norm > 1e-8) ? sum / norm : 0.f;
 }
 
-// The reference's radius (4, GFIRST.cu:512) with the neighbour offsets as
-// loop counters: offsets and the spatial-weight index are the same for every
-// lane (scalar), a row's nine texels are read by buffer loads from one 32-bit
-// row offset (texels past the volume's end read 0 and are not summed), and
-// each voxel still sums its neighbours in the reference's order (z, then y,
-// then x), skipping those past the volume's upper faces.
+// The reference's radius (4, GFIRST.cu:512). Lanes are consecutive voxels of
+// the interior columns, so a wave is full whatever the image side; each walks
+// its neighbours in the reference's order (z, then y, then x), skipping those
+// past the volume's upper faces.
 //
-// Each intensity weight H = (float)exp(-(double)di2 / kI) is first computed
-// on a fast path whose result is provably the same float:
-//  - tq = (g - rv) / mref by a reciprocal and two FMA corrections with
-//    y = RN(1/mref) (Markstein's theorem: the second correction of a
-//    faithful quotient is the correctly rounded one). It holds while nothing
-//    underflows or overflows: for mref in [2^-20, 2^20) and a first quotient
-//    q0 of magnitude in [2^-60, 2^90). Outside that range the weight is the
-//    same on both paths when kI is in [2^-80, 2^40]: |q0| < 2^-60 gives
-//    |x| < 2^-40 and H = 1; |q0| >= 2^90 gives di2 = inf (H = 0) or a NaN,
-//    which the range test below sends to the reference expression. With
-//    mref or kI outside those bounds every weight takes that expression.
-//  - x' = di2 * (-1/kI) instead of the division (|x' - x| <= 3 ulp(x)), and
-//    exp(x') = 2^(n/1024) * p(r): n rounded by the 1.5 * 2^52 shift (its low
-//    word is n), r = x' - n ln2/1024 in one FMA, a 1024-entry table of
-//    2^(j/1024) and a cubic on |r| <= ln2/2048. For x' >= -87 (a normal
-//    float result) the relative error is below 2^-44.
-//  - the float rounding of E drops its 29 low mantissa bits; if they are
-//    more than 2^13 units (2^-40 relative) away from the halfway point, the
-//    library's exp of the exact x rounds to the same float. Below x' = -104.5
-//    the float is 0 either way.
-// A weight near a rounding midpoint (about 3e-5 of them) or with x' in
-// [-104.5, -87) (a denormal float) is recomputed by the reference's
-// expression; the row's weights are then summed in order.
+// Each intensity weight H = (float)exp(-(double)di2 / kI) is first computed in
+// pairs of floats, with a result that is kept only if it is provably the same
+// float:
+//  - tq = (g - rv) / mref from y = RN(1/mref) and the rest yl of 1/mref:
+//    q = RN(a y + a yl) is a faithful quotient, and its correction by the exact
+//    remainder is the correctly rounded one (Markstein). It holds while
+//    nothing underflows or overflows: for mref in [2^-20, 2^20) and |q| in
+//    [2^-60, 2^90). Outside that range the weight is the same either way when
+//    kI is in [2^-80, 2^40]: |q| < 2^-60 gives x < 2^-40 and H = 1; |q| >= 2^90
+//    gives H = 0 or a NaN, which takes the reference expression. With mref or
+//    kI outside those bounds every weight takes that expression.
+//  - t = -di2 / kI * 8192 / ln2 is split as n + 1/2 + f, f in (-0.38, 0.63), by
+//    a sum with 2^22 - 1/4, whose bits hold 4 n: f = di2 (nh + nl) - (n + 1/2)
+//    in two FMAs, where nh + nl is the factor to 2^-48.
+//  - H = 2^(n >> 13) |T + s|, s = RN(T p + Tl), with the table's T + Tl =
+//    -2^((j + 1/2)/8192), j = n mod 8192, and p = exp(f ln2/8192) - 1 as a
+//    quadratic. T + s is within 2^-35 of the exact value (0.82 of that at most
+//    over all floats di2), so its rounding to 24 bits is that of the exact one
+//    unless the rest e of that rounding lies within 2^-35 of half a unit.
+//  - Rare rows of neighbours hold more: x >= 104.5 gives 0, a value below
+//    2^-125 is rounded again to a multiple of 2^-149, and one that may lie at a
+//    rounding midpoint (2e-4 of them) takes the reference expression.
+//
+// What bounds it: VALU issue, 29 full-rate instructions a weight with its sums
+// (about 50 with the exponential in FP64, which issues at half the rate). One
+// pass at 128x128x159: 1.37 -> 0.87 ms. A table of 8192 entries in 64 KB leaves
+// 16 waves per CU, which is enough: the loop has no other long wait. Two rows
+// per thread would share their loads but last twice as long: a few waves whose
+// every row is rare end late, 1.00 ms.
 namespace jbfx {
-constexpr int kBits = 10, kTab = 1 << kBits;
-constexpr double kCN = 1477.3197218702985;                  // 1024 / ln2
-constexpr double kShift = 0x1.8p52;                          // ulp 1
-constexpr double kLn2N = 0x1.62e42fefa39efp-1 / kTab;
-constexpr unsigned kHalf = 1u << 28, kBand = 1u << 13;
+constexpr int kTab = 8192;
+constexpr double kLn2 = 0x1.62e42fefa39efp-1;
+constexpr float kS = 0x1p22f - 0.25f, kM = 0x1p22f - 0.5f;
+constexpr float kC1 = (float)(kLn2 / kTab);
+constexpr float kC2 = (float)(kLn2 / kTab * (kLn2 / kTab) / 2);
+constexpr float kKeep = 0x1p-24f - 0x1p-35f;                        // largest |e| kept
+constexpr float kFar = (float)(0x1p22 - 87.0 / kLn2 * kTab);        // H below 2^-125
+constexpr float kUnder = (float)(0x1p22 - 104.5 / kLn2 * kTab);     // H = 0
+struct Table { float v[2 * kTab]; };
+// -2^((j + 1/2)/8192) as float + float, by the series of exp in double
+constexpr Table table() {
+  Table t{};
+  for (int j = 0; j < kTab; j++) {
+    const double u = kLn2 * (j + 0.5) / kTab;
+    double e = 1.0;
+    for (int i = 17; i > 0; i--) e = 1.0 + e * u / i;
+    t.v[j] = (float)-e;
+    t.v[kTab + j] = (float)((float)e - e);
+  }
+  return t;
+}
+__device__ const Table kT = table();
+constexpr int kThreads = 512;
+
+// The weight of a neighbour between 2^-151 and 2^-125, from the sum sh, the
+// weight v = 2^k |h| as if exponents had no end, and the rest e of h: |h|
+// rounded to a multiple of 2^-149. False if sh is not in that range or the
+// value may lie at a rounding midpoint.
+__device__ inline bool low_weight(float sh, float v, float e, float* w) {
+  const unsigned n = (__float_as_uint(sh) & ~(4u * kTab - 1u)) << 8, x = n & 0x7f800000u;
+  const float h = __uint_as_float(__float_as_uint(v) - n);
+  *w = h * -0x1p-64f * __uint_as_float(x - (65u << 23));  // x: 256 + k, in place
+  const float rest = h + *w * 0x1p64f * __uint_as_float((319u << 23) - x) + e;
+  const float half = __uint_as_float((233u << 23) - x);
+  return (sh < kFar) & (sh >= kUnder) & (fabsf(rest) <= fmaf(half, 1 - 0x1p-20f, -0x1p-35f));
+}
 }  // namespace jbfx
 
-__global__ __launch_bounds__(256) void k_jbf_r4(int res, int nzs, const float* __restrict__ in,
-                                                const float* __restrict__ guide,
-                                                const float* __restrict__ d_max, float max_ref,
-                                                double kI, double nki, GTab gt,
-                                                float* __restrict__ out) {
-  constexpr int R = 4;
-  __shared__ double p2[jbfx::kTab];  // 2^(j/1024)
-  for (int j = threadIdx.y * kWave + threadIdx.x; j < jbfx::kTab; j += 4 * kWave)
-    p2[j] = exp2((double)j * (1.0 / jbfx::kTab));
-  __syncthreads();
-  const int ix = blockIdx.x * kWave + threadIdx.x;
-  const int iy = blockIdx.y * 4 + threadIdx.y;
-  const int iz = blockIdx.z;
-  if (ix >= res || iy >= res) return;
-  const int r2 = res * res;
-  const int iV = (iz * res + iy) * res + ix;
-  if (ix < R || iy < R || iz < R) {
-    out[iV] = 0.f;
+__global__ __launch_bounds__(jbfx::kThreads, 4) void k_jbf_r4(
+    int res, int nzs, const float* __restrict__ in, const float* __restrict__ guide,
+    const float* __restrict__ d_max, float max_ref, double kI, float nh_, float nl_, GTab gt,
+    float* __restrict__ out) {
+  using namespace jbfx;
+  constexpr int R = 4, W = 2 * R + 1;
+  __shared__ __align__(16) float tab[2 * kTab];
+  const int r2 = res * res, iz = blockIdx.y, side = res - R;  // columns R..res-1
+  const int i = blockIdx.x * kThreads + threadIdx.x, n = gridDim.x * kThreads;
+  // the low borders are zero
+  if (iz < R || side <= 0) {
+    for (int j = i; j < r2; j += n) out[(size_t)iz * r2 + j] = 0.f;
     return;
   }
+  for (int j = i; j < R * res + R * side; j += n) {
+    const int k = j - R * res;
+    out[(size_t)iz * r2 + (k < 0 ? j : (R + k / R) * res + k % R)] = 0.f;
+  }
+  for (int j = threadIdx.x; j < kTab / 2; j += kThreads)
+    ((float4*)tab)[j] = ((const float4*)kT.v)[j];
+  __syncthreads();
+  const int iy = R + i / side, ix = R + i % side;
+  if (iy >= res) return;
   const unsigned vbytes = (unsigned)(r2 * nzs) * 4u;
   const __amdgpu_buffer_rsrc_t rg = rsrc(guide, vbytes), ri = rsrc(in, vbytes);
-  const float mref = d_max ? __uint_as_float(*(const unsigned int*)d_max) : max_ref;
-  const float ym = 1.0f / mref;
-  const unsigned allslow =
-      (mref >= 0x1p-20f && mref < 0x1p20f && kI >= 0x1p-80 && kI <= 0x1p40) ? 0u : 0x1ffu;
-  const float rv = guide[iV];
+  float mref = d_max ? __uint_as_float(*(const unsigned int*)d_max) : max_ref;
+  const bool all = !(mref >= 0x1p-20f && mref < 0x1p20f && kI >= 0x1p-80 && kI <= 0x1p40);
+  // constants in vector registers: an instruction with a scalar operand issues
+  // at half the rate
+  float yh = 1.0f / mref;
+  float yl = fmaf(-mref, yh, 1.0f) * yh, nh = nh_, nl = nl_, S = kS, M = kM, C1 = kC1, C2 = kC2;
+  asm volatile("" : "+v"(mref), "+v"(yh), "+v"(yl), "+v"(nh), "+v"(nl));
+  asm volatile("" : "+v"(S), "+v"(M), "+v"(C1), "+v"(C2));
+  const int iV = (iz * res + iy) * res + ix;
+  const float rv = ld_f1(rg, 4u * iV, 0);
   float norm = 0.f, sum = 0.f;
-  for (int dz = -R; dz <= R; dz++) {
+  // bit k: neighbour ix + k - R lies inside the volume
+  const unsigned vmask = 0x1ffu >> max(0, ix + R - (res - 1));
+  for (int dz = -R; dz <= min(R, nzs - 1 - iz); dz++) {
     for (int dy = -R; dy <= R; dy++) {
-      const bool vzy = iz + dz <= nzs - 1 && iy + dy <= res - 1;
-      // bit k: neighbour ix + k - R lies inside the volume
-      const unsigned vmask = vzy ? (0x1ffu >> max(0, ix + R - (res - 1))) : 0u;
+      if (iy + dy > res - 1) continue;
       unsigned voff = (unsigned)(iV + dz * r2 + dy * res - R) * 4u;
       asm volatile("" : "+v"(voff));  // row start as the base: texel k at immediate 4k
-      float gv[2 * R + 1], iv[2 * R + 1], H[2 * R + 1];
+      float gv[W], iv[W], H[W], e[W], sh[W];
 #pragma unroll
-      for (int k = 0; k <= 2 * R; k++) {
+      for (int k = 0; k < W; k++) {
         gv[k] = ld_f1(rg, voff + 4u * k, 0);
         iv[k] = ld_f1(ri, voff + 4u * k, 0);
       }
-      unsigned slow = 0;
+      float emax = 0.f, smin = 0x1p22f;
 #pragma unroll
-      for (int k = 0; k <= 2 * R; k++) {
+      for (int k = 0; k < W; k++) {
         const float a = gv[k] - rv;
-        const float q0 = a * ym;
-        const float q1 = fmaf(fmaf(-q0, mref, a), ym, q0);
-        const float tq = fmaf(fmaf(-q1, mref, a), ym, q1);
+        const float q = fmaf(a, yh, a * yl);
+        const float tq = fmaf(fmaf(-q, mref, a), yh, q);
         const float di2 = tq * tq;
-        const double x = (double)di2 * nki;
-        const double sh = fma(x, jbfx::kCN, jbfx::kShift);
-        const int n = __double2loint(sh);
-        const double r = fma(-(sh - jbfx::kShift), jbfx::kLn2N, x);
-        double p = fma(r, 1.0 / 6, 0.5);
-        p = fma(p, r, 1.0);
-        p = fma(p, r, 1.0);
-        const double E = ldexp(p2[n & (jbfx::kTab - 1)] * p, n >> jbfx::kBits);
-        const unsigned low = (unsigned)__double2loint(E) & 0x1fffffffu;
-        const bool amb = low - (jbfx::kHalf - jbfx::kBand) < 2u * jbfx::kBand;
-        const bool under = x < -104.5;
-        H[k] = under ? 0.f : (float)E;
-        const bool bad = !under & (!(x >= -87.0) | amb);
-        slow |= bad ? 1u << k : 0u;
+        sh[k] = fmaf(di2, nh, S);
+        const unsigned b = __float_as_uint(sh[k]);
+        const float* T = (const float*)((const char*)tab + (b & (4u * kTab - 4u)));
+        float f = fmaf(di2, nh, M - __uint_as_float(b & ~3u));
+        f = fmaf(di2, nl, f);
+        const float p = f * fmaf(f, C2, C1);
+        const float s = fmaf(T[0], p, T[kTab]);
+        const float h = T[0] + s;
+        e[k] = s - (h - T[0]);
+        unsigned m = b & ~(4u * kTab - 1u);
+        asm("" : "+v"(m));  // shift and add in one instruction
+        H[k] = __uint_as_float((m << 8) + __float_as_uint(h));
+        emax = fmaxf(emax, fabsf(e[k]));
+        smin = __builtin_elementwise_minimum(smin, sh[k]);  // a NaN stays
       }
-      slow = (slow | allslow) & vmask;
-      if (slow) {
-        for (int k = 0; k <= 2 * R; k++) {
-          if ((slow >> k) & 1u) {
-            const float tq = (gv[k] - rv) / mref;
-            const float di2 = tq * tq;
-            H[k] = (float)exp(-(double)di2 / kI);
+      if (emax > kKeep || !(smin >= kFar) || all) {
+        unsigned left = 0;
+        bool mid = false;
+#pragma unroll
+        for (int k = 0; k < W; k++) {
+          const bool under = sh[k] < kUnder, low = !(sh[k] >= kFar) & !under;
+          left |= (low | ((fabsf(e[k]) > kKeep) & !under)) ? 1u << k : 0u;
+          mid |= low;
+          H[k] = under ? 0.f : H[k];
+        }
+        if (__builtin_amdgcn_ballot_w64(mid)) {
+#pragma unroll
+          for (int k = 0; k < W; k++) {
+            float w;
+            const bool low = low_weight(sh[k], H[k], e[k], &w);
+            H[k] = low ? w : H[k];
+            left &= low ? ~(1u << k) : ~0u;
+          }
+        }
+        // every lane takes its own next neighbour, and with it all that have
+        // the same value (a flat background)
+        left = (all ? 0x1ffu : left) & vmask;
+        while (left) {
+          const int k = __builtin_ctz(left);
+          const float g = ld_f1(rg, voff + 4u * k, 0);
+          const float tq = (g - rv) / mref;
+          const float di2 = tq * tq;
+          const float w = (float)exp(-(double)di2 / kI);
+#pragma unroll
+          for (int j = 0; j < W; j++) {
+            const bool same = (j == k) | (gv[j] == g);
+            H[j] = same ? w : H[j];
+            left &= same ? ~(1u << j) : ~0u;
           }
         }
       }
-      const int d2yz = dz * dz + dy * dy;
+      const int d2 = dz * dz + dy * dy;
+      float gk[R + 1] = {gt.g[d2], gt.g[d2 + 1], gt.g[d2 + 4], gt.g[d2 + 9], gt.g[d2 + 16]};
+      asm("" : "+v"(gk[0]), "+v"(gk[1]), "+v"(gk[2]), "+v"(gk[3]), "+v"(gk[4]));
 #pragma unroll
-      for (int k = 0; k <= 2 * R; k++) {
-        if ((vmask >> k) & 1u) {
-          const float hg = H[k] * gt.g[d2yz + (k - R) * (k - R)];
+      for (int k = 0; k < W; k++) {
+        if (k <= R || (vmask >> k) & 1u) {
+          const float hg = H[k] * gk[k < R ? R - k : k - R];
           norm += hg;
           sum = fmaf(hg, iv[k], sum);
         }
@@ -614,11 +684,17 @@ hipError_t launch_jbf(const DevGeom& G, const float* in, const float* guide,
   const double kI = (2.0 * (double)sI) * (2.0 * (double)sI);
   // the radius-4 kernel addresses the volume with 32-bit byte offsets
   if (r == 4 && G.nvox < (1ll << 29))
-    hipLaunchKernelGGL(k_jbf_r4, grid_img(G, G.nzs), dim3(kWave, 4), 0, st, G.res, G.nzs, in,
-                       guide, d_max_ref, max_ref, kI, -1.0 / kI, gt, out);
-  else
+  {
+    const long long items = (long long)(G.res - 4) * (G.res - 4);
+    const unsigned gx = G.res > 4 ? (unsigned)((items + jbfx::kThreads - 1) / jbfx::kThreads) : 1u;
+    const double nki = -jbfx::kTab / jbfx::kLn2 / kI;
+    const float nh = (float)nki;
+    hipLaunchKernelGGL(k_jbf_r4, dim3(gx, G.nzs), dim3(jbfx::kThreads), 0, st, G.res, G.nzs, in,
+                       guide, d_max_ref, max_ref, kI, nh, (float)(nki - nh), gt, out);
+  } else {
     hipLaunchKernelGGL(k_jbf, grid_img(G, G.nzs), dim3(kWave, 4), 0, st, G.res, G.nzs, in,
                        guide, d_max_ref, max_ref, r, kI, gt, out);
+  }
   return hipGetLastError();
 }
 
