@@ -522,7 +522,8 @@ int gfr_back_project(gfr_ctx* ctx, const gfr_geometry* g, const float* d_corr,
         packed_rows(gd->dev, buf, subset, nsub, ctx->d_scratch_u32 + 128, ++ctx->pack_epoch);
     if (buf) e = launch_pack(gd->dev, d_corr, d_mask, P, subset, nsub, st);
     if (buf && e == hipSuccess)
-      e = launch_back_packed(gd->dev, P, d_numer, d_denom, subset, nsub, nullptr, gd->tune[nsub], st);
+      e = launch_back_packed(gd->dev, {{P}, {d_numer}, {d_denom}}, 1, subset, nsub, nullptr,
+                             gd->tune[nsub], st);
     if (buf) scratch_release(ctx->pack, st);
   }
   if (e != hipSuccess) return hip_err(ctx, e, "back projection");

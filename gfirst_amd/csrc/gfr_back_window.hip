@@ -124,8 +124,8 @@ __device__ __forceinline__ void exact_view(const DevGeom& G, __amdgpu_buffer_rsr
 // geometries whose tiles need wider windows.
 template <int ZB, int NV, bool TAB, bool WIN>
 __global__ __launch_bounds__(256, ZB * NV <= 8 ? 5 : 3) void k_back_window(
-    DevGeom G, PackedRows P, float* __restrict__ numer, float* __restrict__ denom, int subset,
-    int nsub, const int* __restrict__ dsub, int tabf, int wrows) {
+    DevGeom G, BackFrames F, int nf, int subset, int nsub, const int* __restrict__ dsub, int tabf,
+    int wrows) {
   // [angle][3][64]: yr, au, entry offset in bytes; then per wave NV windows of
   // wrows rows
   extern __shared__ __align__(16) float tab[];
@@ -135,6 +135,9 @@ __global__ __launch_bounds__(256, ZB * NV <= 8 ? 5 : 3) void k_back_window(
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   int bx, by, bz;
   xcd_region(bx, by, bz);
+  const int fr = __builtin_amdgcn_readfirstlane(bz % nf);  // every frame's heavy slabs first
+  bz /= nf;
+  const PackedRows P = F.rows[fr];
   // The four waves of a block take the same columns and neighbouring slabs,
   // counted from the middle of the volume outwards: the middle slabs see the
   // most views, so the heaviest blocks start first and the last ones are light.
@@ -470,8 +473,8 @@ __global__ __launch_bounds__(256, ZB * NV <= 8 ? 5 : 3) void k_back_window(
     const int iz = zb + j;
     if (iz < G.nzs) {
       const size_t iV = ((size_t)iz * G.res + iy) * G.res + ix;
-      numer[iV] = n[j];
-      denom[iV] = d[j];
+      F.numer[fr][iV] = n[j];
+      F.denom[fr][iV] = d[j];
     }
   }
 }
@@ -486,19 +489,19 @@ int window_rows(const DevGeom& G, int zb) {
 }
 
 template <int ZB, int NV, bool WIN>
-hipError_t launch_zb(const DevGeom& G, const PackedRows& P, float* numer, float* denom, int subset,
-                     int nsub, const int* dsub, int nav, hipStream_t st) {
+hipError_t launch_zb(const DevGeom& G, const BackFrames& F, int nf, int subset, int nsub,
+                     const int* dsub, int nav, hipStream_t st) {
   const unsigned nt = (G.res + 7) / 8, ns = (G.nzs + ZB - 1) / ZB;
-  const dim3 grid(nt, nt, (ns + 3) / 4);
+  const dim3 grid(nt, nt, (ns + 3) / 4 * nf);
   const int rows = WIN ? max(16, window_rows(G, ZB)) : 0;
   const int tabf = nav <= kTabAngles ? nav * 192 : 0;
   const unsigned lds = (unsigned)(tabf + 4 * NV * rows * kWinStride) * 4u;
   if (tabf)
-    hipLaunchKernelGGL((k_back_window<ZB, NV, true, WIN>), grid, dim3(256), lds, st, G, P, numer,
-                       denom, subset, nsub, dsub, tabf, rows);
+    hipLaunchKernelGGL((k_back_window<ZB, NV, true, WIN>), grid, dim3(256), lds, st, G, F, nf,
+                       subset, nsub, dsub, tabf, rows);
   else
-    hipLaunchKernelGGL((k_back_window<ZB, NV, false, WIN>), grid, dim3(256), lds, st, G, P, numer,
-                       denom, subset, nsub, dsub, tabf, rows);
+    hipLaunchKernelGGL((k_back_window<ZB, NV, false, WIN>), grid, dim3(256), lds, st, G, F, nf,
+                       subset, nsub, dsub, tabf, rows);
   return hipGetLastError();
 }
 
@@ -528,14 +531,14 @@ static Tune untuned_shape(const DevGeom& G) {
   return t;
 }
 
-hipError_t launch_back_packed(const DevGeom& G, const PackedRows& P, float* numer, float* denom,
-                              int subset, int nsub, const int* dsub, const Tune& asked,
-                              hipStream_t st) {
+hipError_t launch_back_packed(const DevGeom& G, const BackFrames& F, int nf, int subset, int nsub,
+                              const int* dsub, const Tune& asked, hipStream_t st) {
+  if (nf < 1 || nf > kMaxGroup) return hipErrorInvalidValue;
   const Tune tune = asked.tuned ? asked : untuned_shape(G);
   if (packed_bytes(G, dsub ? 0 : subset, nsub) >= 0xFFFFFFF0u) return hipErrorInvalidValue;
   const int nav = (G.nang - (dsub ? 0 : subset) + nsub - 1) / nsub;
 #define GFR_BW(ZB, NV, WIN) \
-  return launch_zb<ZB, NV, WIN>(G, P, numer, denom, subset, nsub, dsub, nav, st)
+  return launch_zb<ZB, NV, WIN>(G, F, nf, subset, nsub, dsub, nav, st)
   const int zb = tune.back_zb;
   if (zb == 1 && tune.back_ahead > 1 && back_window_fits(G, 1) && window_rows(G, 1) <= 16) {  // NV > 1
     if (tune.back_ahead == 2) GFR_BW(1, 2, true);

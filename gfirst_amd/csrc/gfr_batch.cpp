@@ -15,10 +15,11 @@
 // the reference's (GFIRST.cu:324-340 blur, 341-469 forward/ratio/backward,
 // 482-502 update), identical kernel for kernel to gfr_recon_step in mode 1,
 // except that frames at the same subset of the same subset count share their
-// backprojection: up to `group` of them write their ratios into one set of
-// interleaved rows and one launch backprojects them all (the per-view
-// geometry, calibration interpolation and row loads are shared; each frame's
-// sums keep their bits).
+// backprojection launch: up to `group` of them at a time, each from its own
+// packed rows, which fills the chip at subsets of a few angles. Six Inveon-size
+// frames of 8, 16 and 24 subsets, one iteration each: 64 ms (one kernel for
+// three interleaved frames, gathering 16 bytes a bin, and the projector of that
+// time: 91 ms).
 #include <math.h>
 #include <stdlib.h>
 #include <string.h>
@@ -35,12 +36,11 @@ namespace {
 struct Lane {
   hipStream_t st = nullptr;
   hipEvent_t join = nullptr;
-  float *xb = nullptr, *num = nullptr, *den = nullptr, *work = nullptr, *R = nullptr;
-  float* rows = nullptr;                 // packed rows of a lone frame
+  float *xb = nullptr, *work = nullptr, *R = nullptr;
   unsigned* bad = nullptr;               // PackedRows::bad
-  float* corr4 = nullptr;                // interleaved rows of a frame group
-  float* num_g[kMaxGroup] = {};          // numerators / denominators of a group
-  float* den_g[kMaxGroup] = {};          // ([0] = num / den)
+  float* rows[kMaxGroup] = {};           // per frame of a group: packed rows,
+  float* num[kMaxGroup] = {};            // numerator,
+  float* den[kMaxGroup] = {};            // denominator
   double* llh_part = nullptr;
   size_t r_floats = 0;
 };
@@ -63,7 +63,7 @@ size_t store_bytes(int storage) { return storage == GFR_STORE_F32 ? 4 : 2; }
 int group_of(const gfr_batch_params* p) { return p->group == 0 ? kMaxGroup : p->group; }
 
 struct Sizes {
-  size_t img, rows, corr4, rot, llh, frame_nobg, frame_bg, shared;
+  size_t img, rows, rot, llh, frame_nobg, frame_bg, shared;
 };
 
 Sizes sizes_of(const GeomHost& h, const gfr_batch_params* p) {
@@ -73,7 +73,6 @@ Sizes sizes_of(const GeomHost& h, const gfr_batch_params* p) {
   z.rows = 2 * sizeof(float) * nav * ((size_t)h.info.nsinogs + 2 * (size_t)h.g.nseg) *
             ((size_t)h.g.nrad + 2);  // packed rows: NRAD + 2 entries
   const int grp = group_of(p);
-  z.corr4 = grp > 1 ? 2 * z.rows : 0;
   z.rot = sizeof(float) * (size_t)(h.info.lambda1 - h.info.lambda0 + 1) * h.g.nzs * h.g.nrad *
           std::min(nav, (size_t)kRotChunk);
   z.llh = sizeof(double) * (size_t)llh_capacity(h, p->min_nsub) + 64;
@@ -81,7 +80,7 @@ Sizes sizes_of(const GeomHost& h, const gfr_batch_params* p) {
   z.frame_nobg = z.img + sino;
   z.frame_bg = z.img + 2 * sino;
   const size_t per_lane =
-      (4 + 2 * (size_t)(grp - 1)) * z.img + z.rows + z.corr4 + z.rot + z.llh;
+      (2 + 2 * (size_t)grp) * z.img + (size_t)grp * z.rows + z.rot + z.llh;
   const size_t slots = (size_t)p->max_frames * (3 * sizeof(int) + sizeof(double)) + 256;
   z.shared = (size_t)p->lanes * per_lane + (size_t)h.info.ndata /* mask */ + slots;
   return z;
@@ -129,9 +128,8 @@ void drop_graph(gfr_batch* b) {
 }
 
 // Enqueues the blur and forward projection of frame f on lane L (kernels
-// read the subset index from d_sub[f]); the ratio goes to the lane's packed
-// rows (chan < 0) or to channel chan of its interleaved group rows.
-hipError_t enqueue_forward(gfr_batch* b, int f, const Lane& L, int chan) {
+// read the subset index from d_sub[f]); the ratio goes to `rows`.
+hipError_t enqueue_forward(gfr_batch* b, int f, const Lane& L, const PackedRows& rows) {
   const DevGeom& G = b->gd->dev;
   const Frame& fr = b->frames[f];
   const int* dsub = b->d_sub + f;
@@ -139,12 +137,7 @@ hipError_t enqueue_forward(gfr_batch* b, int f, const Lane& L, int chan) {
   psf_taps(b->p.psf_fw, tf.g);
   hipError_t e = launch_blur_xy(G, tf, fr.x, L.xb, L.st);
   FwdOut fo;
-  if (chan < 0) {
-    fo.rows = packed_rows(G, L.rows, 0, fr.nsub, L.bad, 1);
-  } else {
-    fo.corr4 = L.corr4;
-    fo.chan = chan;
-  }
+  fo.rows = rows;
   fo.mask = b->mask;
   fo.y = fr.y;
   fo.bg = fr.bg;
@@ -173,31 +166,26 @@ hipError_t enqueue_update(gfr_batch* b, int f, const float* num, const float* de
 hipError_t enqueue_group(gfr_batch* b, const std::vector<int>& grp, const Lane& L) {
   const DevGeom& G = b->gd->dev;
   const Frame& f0 = b->frames[grp[0]];
+  BackFrames F{};
   hipError_t e = hipSuccess;
-  if (grp.size() == 1) {
-    e = enqueue_forward(b, grp[0], L, -1);
-    if (e == hipSuccess)
-      e = launch_back_packed(G, packed_rows(G, L.rows, 0, f0.nsub, L.bad, 1), L.num, L.den, 0, f0.nsub, b->d_sub + grp[0], f0.tune,
-                             L.st);
-    if (e == hipSuccess) e = enqueue_update(b, grp[0], L.num, L.den, L);
-    return e;
+  for (size_t i = 0; i < grp.size() && e == hipSuccess; i++) {
+    F.rows[i] = packed_rows(G, L.rows[i], 0, f0.nsub, L.bad, 1);
+    F.numer[i] = L.num[i];
+    F.denom[i] = L.den[i];
+    e = enqueue_forward(b, grp[i], L, F.rows[i]);
   }
-  for (size_t i = 0; i < grp.size() && e == hipSuccess; i++)
-    e = enqueue_forward(b, grp[i], L, (int)i);
   if (e == hipSuccess)
-    e = launch_back_multi(G, L.corr4, L.num_g, L.den_g, (int)grp.size(), 0, f0.nsub,
-                          b->d_sub + grp[0], f0.tune.multi_zb == 6 ? 6 : 4, L.st);
+    e = launch_back_packed(G, F, (int)grp.size(), 0, f0.nsub, b->d_sub + grp[0], f0.tune, L.st);
   for (size_t i = 0; i < grp.size() && e == hipSuccess; i++)
-    e = enqueue_update(b, grp[i], L.num_g[i], L.den_g[i], L);
+    e = enqueue_update(b, grp[i], F.numer[i], F.denom[i], L);
   return e;
 }
 
-// Work of one pass of a group, for spreading groups over lanes (a shared
-// backprojection costs about 0.7 of the separate ones per frame).
+// Work of one pass of a group, for spreading groups over lanes.
 double group_cost(const gfr_batch* b, const std::vector<int>& grp) {
   const int S = b->frames[grp[0]].nsub;
   const double one = (double)((b->g.nang + S - 1) / S) + 2.0;
-  return grp.size() == 1 ? one : 0.7 * one * (double)grp.size();
+  return one * (double)grp.size();
 }
 
 // Frames at the same subset of the same subset count (their subset indices
@@ -283,29 +271,6 @@ int rebuild(gfr_batch* b) {
   return GFR_OK;
 }
 
-// Best of two timed group backprojections (after a warm-up) of subset 0.
-float time_group_back(gfr_batch* b, Lane& L, int nsub, int zb, hipError_t* err) {
-  hipEvent_t e0 = nullptr, e1 = nullptr;
-  hipError_t e = hipEventCreate(&e0);
-  if (e == hipSuccess) e = hipEventCreate(&e1);
-  float best = 1e30f;
-  for (int rep = 0; rep < 3 && e == hipSuccess; rep++) {
-    e = hipEventRecord(e0, b->st);
-    if (e == hipSuccess)
-      e = launch_back_multi(b->gd->dev, L.corr4, L.num_g, L.den_g, group_of(&b->p), 0, nsub,
-                            nullptr, zb, b->st);
-    if (e == hipSuccess) e = hipEventRecord(e1, b->st);
-    if (e == hipSuccess) e = hipEventSynchronize(e1);
-    float ms = 0.f;
-    if (e == hipSuccess) e = hipEventElapsedTime(&ms, e0, e1);
-    if (e == hipSuccess && rep > 0 && ms < best) best = ms;
-  }
-  if (e0) (void)hipEventDestroy(e0);
-  if (e1) (void)hipEventDestroy(e1);
-  *err = e;
-  return best;
-}
-
 bool any_positive(const float* v, long long n) {
   for (long long i = 0; i < n; i++)
     if (!(v[i] <= 0.f)) return true;
@@ -383,18 +348,11 @@ int gfr_batch_create(gfr_ctx* ctx, const gfr_geometry* g, const gfr_batch_params
     L.bad = b->d_bad + (&L - b->lanes.data());  // at most 16 lanes
     ok = hipStreamCreateWithFlags(&L.st, hipStreamNonBlocking) == hipSuccess &&
          hipEventCreateWithFlags(&L.join, hipEventDisableTiming) == hipSuccess &&
-         A((void**)&L.xb, z.img) && A((void**)&L.num, z.img) && A((void**)&L.den, z.img) &&
-         A((void**)&L.work, z.img) && A((void**)&L.rows, z.rows) && A((void**)&L.R, z.rot) &&
+         A((void**)&L.xb, z.img) && A((void**)&L.work, z.img) && A((void**)&L.R, z.rot) &&
          A((void**)&L.llh_part, z.llh);
-    L.num_g[0] = L.num;
-    L.den_g[0] = L.den;
-    if (ok && z.corr4) {
-      ok = A((void**)&L.corr4, z.corr4);
-      for (int i = 1; i < group_of(p) && ok; i++)
-        ok = A((void**)&L.num_g[i], z.img) && A((void**)&L.den_g[i], z.img);
-      // defined contents for the first timing of the group backprojector
-      if (ok) ok = launch_zero(L.corr4, z.corr4, b->st) == hipSuccess;
-    }
+    for (int i = 0; i < group_of(p) && ok; i++)
+      ok = A((void**)&L.rows[i], z.rows) && A((void**)&L.num[i], z.img) &&
+           A((void**)&L.den[i], z.img);
     L.r_floats = z.rot / sizeof(float);
   }
   if (!ok) return bfail(b, set_err(ctx, GFR_ENOMEM, "batch allocation failed"));
@@ -511,32 +469,17 @@ int gfr_batch_add(gfr_batch* b, int niter, int nsub, const float* prompts, const
   if (!t.tuned && !(env && env[0] == '0')) {
     Lane& L = b->lanes[0];
     FwdOut fo;
-    fo.rows = packed_rows(G, L.rows, 0, nsub, L.bad, 1);
+    fo.rows = packed_rows(G, L.rows[0], 0, nsub, L.bad, 1);
     fo.mask = b->mask;
     fo.y = fr.y;
     fo.bg = fr.bg;
     fo.storage = b->p.storage;
     fo.yscale = (float)b->g.res;
     fo.llh_part = L.llh_part;
-    e = tune_shapes(G, nsub, fo, fr.x, L.R, L.r_floats, L.num, L.den, st, &t);
+    e = tune_shapes(G, nsub, fo, fr.x, L.R, L.r_floats, L.num[0], L.den[0], st, &t);
     if (e != hipSuccess) return undo(hip_err(ctx, e, "gfr_batch_add tuning"));
     std::lock_guard<std::mutex> lk(ctx->mu);
     b->gd->tune[nsub] = t;
-  }
-  // Slices of the group backprojector, measured once per subset count.
-  if (t.multi_zb == 0 && group_of(&b->p) > 1 && !(env && env[0] == '0')) {
-    Lane& L = b->lanes[0];
-    float best = 1e30f;
-    for (int zb : {4, 6}) {
-      const float ms = time_group_back(b, L, nsub, zb, &e);
-      if (e != hipSuccess) return undo(hip_err(ctx, e, "gfr_batch_add tuning"));
-      if (ms < best) {
-        best = ms;
-        t.multi_zb = zb;
-      }
-    }
-    std::lock_guard<std::mutex> lk(ctx->mu);
-    b->gd->tune[nsub].multi_zb = t.multi_zb;
   }
   (void)hipFree(stage);
   stage = nullptr;

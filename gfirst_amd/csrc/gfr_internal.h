@@ -80,7 +80,6 @@ struct Tune {
   int rot_z = 16;         // planes per rotation block: 4, 16 or 32
   int back_bw = 4;        // waves per direct backprojector block: 4 (16x16) or 1 (8x8)
   int back_ahead = 1;     // 1-slice shapes: views whose rows are loaded ahead (1, 2, 4)
-  int multi_zb = 0;       // slices of the multi-frame backprojector: 4 or 6 (0: not measured)
   bool tuned = false;
   float ms_back = 0.f, ms_zsum = 0.f;
 };
@@ -220,8 +219,6 @@ struct FwdOut {
   float* proj = nullptr;          // projection, full sinogram layout
   float* corr = nullptr;          // ratio, full layout
   PackedRows rows{};              // packed rows of the subset (v NULL: not written)
-  float* corr4 = nullptr;         // or: channel `chan` of interleaved 3-frame rows
-  int chan = 0;
   const uint8_t* mask = nullptr;  // calibration mask (needed with rows)
   const void* y = nullptr;        // measured prompts (storage format, unscaled)
   const void* bg = nullptr;       // background or NULL
@@ -238,19 +235,18 @@ size_t rotate_floats_per_angle(const DevGeom& G);
 hipError_t launch_forward(const DevGeom& G, const float* img, float* R, size_t r_cap_floats,
                           const FwdOut& out, int subset, int nsub, const int* dsub,
                           const Tune& tune, hipStream_t st);
-hipError_t launch_back_packed(const DevGeom& G, const PackedRows& P, float* numer, float* denom,
-                              int subset, int nsub, const int* dsub, const Tune& tune,
-                              hipStream_t st);
+// Backprojection of the packed rows of nf frames (same geometry, subset and
+// mask) into their numerators and denominators, in one launch.
+constexpr int kMaxGroup = 3;
+struct BackFrames {
+  PackedRows rows[kMaxGroup];
+  float* numer[kMaxGroup];
+  float* denom[kMaxGroup];
+};
+hipError_t launch_back_packed(const DevGeom& G, const BackFrames& F, int nf, int subset, int nsub,
+                              const int* dsub, const Tune& tune, hipStream_t st);
 // Whether a wave's window of zb slices holds every read of a tile.
 bool back_window_fits(const DevGeom& G, int zb);
-// Multi-frame backprojection: nf (2 or 3) frames' interleaved rows
-// (packed4_bytes) -> numer[f], denom[f]; the sums of launch_back_packed on
-// each frame's own rows, bit for bit. zb: 4 or 6 slices per thread.
-constexpr int kMaxGroup = 3;
-size_t packed4_bytes(const DevGeom& G, int subset, int nsub);
-hipError_t launch_back_multi(const DevGeom& G, const float* corr4, float* const* numer,
-                             float* const* denom, int nf, int subset, int nsub, const int* dsub,
-                             int zb, hipStream_t st);
 // Sensitivity of a subset: the backprojector's denominator half in FP64
 // ({1, calib} pairs, packed_bytes of scratch, so only calibration gaps apply).
 hipError_t launch_sensitivity(const DevGeom& G, const uint8_t* mask, float2* c2, double* sens,

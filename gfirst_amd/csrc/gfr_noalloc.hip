@@ -84,7 +84,7 @@ extern "C" int gfr_back_project_noalloc(gfr_ctx* ctx, const gfr_geometry* g, con
                                    ++epoch);
   hipError_t e = launch_pack(gd->dev, d_corr, d_mask, P, subset, nsub, st);
   if (e == hipSuccess)
-    e = launch_back_packed(gd->dev, P, d_numer, d_denom, subset, nsub, nullptr, t, st);
+    e = launch_back_packed(gd->dev, {{P}, {d_numer}, {d_denom}}, 1, subset, nsub, nullptr, t, st);
   if (e != hipSuccess) return hip_err(ctx, e, "gfr_back_project_noalloc");
   return GFR_OK;
 }

@@ -496,7 +496,7 @@ int gfr_recon_step(gfr_recon* r) {
   // Backprojection of the subset (GFIRST.cu:436-469) and update (:482-502).
   {
     PhaseMark pm(r, GFR_PHASE_BACK, st);
-    GFR_HIP(ctx, launch_back_packed(G, rows, num, den, s, S, nullptr, r->tune, st));
+    GFR_HIP(ctx, launch_back_packed(G, {{rows}, {num}, {den}}, 1, s, S, nullptr, r->tune, st));
   }
   {
     PhaseMark pm(r, GFR_PHASE_UPDATE, st);
