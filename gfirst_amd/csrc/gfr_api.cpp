@@ -608,8 +608,8 @@ int gfr_image_max(gfr_ctx* ctx, const gfr_geometry* g, const float* d_x, float* 
 
 // ---------------------------------------------------------------------------
 // VLOR: the static part of the soft assignment (valid records, BLANKT and the
-// bin -> record lists) is built once; each pass recomputes 1/(s1+s2) per
-// record and sums each touched bin's contributions in record order.
+// bin -> record lists) is built once; each pass sums the contributions of its
+// own touched bins in record order.
 // ---------------------------------------------------------------------------
 int gfr_vlor_create(gfr_ctx* ctx, const gfr_geometry* g, const int32_t* rec, long long nrec,
                     const float* d_yT, gfr_vlor** out) {
@@ -626,11 +626,8 @@ int gfr_vlor_assign(gfr_ctx* ctx, gfr_vlor* v, const float* d_proj, float* d_dv,
   GFR_GEOM(ctx, &v->g, gd);
   if (bad_subset(ctx, gd, subset, nsub)) return GFR_EINVAL;
   hipStream_t st = stream_of(ctx, stream);
-  GFR_HIP(ctx, launch_vlor_event(v->d_i1, v->d_i2, v->d_blankt, d_proj, v->d_sinv, v->d_valor,
-                                 v->nev, 0, st));
-  GFR_HIP(ctx, launch_vlor_zero_subset(gd->dev, d_dv, subset, nsub, st));
-  GFR_HIP(ctx, launch_vlor_bins(gd->dev, v->d_bins, v->d_start, v->d_ev, v->nbins, d_proj,
-                                v->d_sinv, v->d_valor, d_dv, subset, nsub, st));
+  GFR_HIP(ctx, launch_vlor_assign(gd->dev, v->d_bins, v->d_start, v->d_ent, v->d_first, d_proj,
+                                  d_dv, subset, nsub, st));
   return GFR_OK;
 }
 
@@ -640,8 +637,7 @@ int gfr_vlor_destroy(gfr_vlor* v) {
     std::lock_guard<std::mutex> lk(v->ctx->mu);
     if (v->ctx->in_use >= v->bytes) v->ctx->in_use -= v->bytes;
   }
-  void* ps[] = {v->d_i1, v->d_i2, v->d_blankt, v->d_sinv, v->d_valor, v->d_bins, v->d_start, v->d_ev};
-  for (void* p : ps)
+  for (void* p : {(void*)v->d_bins, (void*)v->d_start, (void*)v->d_ent, (void*)v->d_first})
     if (p) (void)hipFree(p);
   delete v;
   return GFR_OK;
@@ -735,24 +731,25 @@ int vlor_create_on(gfr_ctx* ctx, const gfr_geometry* g, const int32_t* rec, long
     v->bytes += b;
     return hipMalloc(p, b ? b : 4);
   };
-  float* d_v0 = nullptr;
-  int* d_rec = nullptr;
-  hipError_t e = hipSuccess;
-  if (e == hipSuccess) e = dalloc((void**)&v->d_i1, sizeof(int) * nrec);
-  if (e == hipSuccess) e = dalloc((void**)&v->d_i2, sizeof(int) * nrec);
-  if (e == hipSuccess) e = dalloc((void**)&v->d_blankt, sizeof(float) * nd);
-  if (e == hipSuccess) e = dalloc((void**)&v->d_sinv, sizeof(float) * nrec);
-  if (e == hipSuccess) e = dalloc((void**)&v->d_valor, sizeof(float) * nrec);
-  if (e == hipSuccess) e = dalloc((void**)&v->d_bins, sizeof(long long) * ne);
+  float *d_v0 = nullptr, *d_blankt = nullptr;
+  int *d_rec = nullptr, *d_i1 = nullptr, *d_i2 = nullptr, *d_ev = nullptr;
+  auto talloc = [](void** p, size_t b) { return hipMalloc(p, b ? b : 4); };
+  hipError_t e = dalloc((void**)&v->d_bins, sizeof(unsigned) * ne);
   if (e == hipSuccess) e = dalloc((void**)&v->d_start, sizeof(int) * (ne + 1));
-  if (e == hipSuccess) e = dalloc((void**)&v->d_ev, sizeof(int) * ne);
-  if (e == hipSuccess) e = hipMalloc((void**)&d_v0, sizeof(float) * nd);
+  if (e == hipSuccess) e = dalloc((void**)&v->d_ent, sizeof(int2) * ne);
+  if (e == hipSuccess)
+    e = dalloc((void**)&v->d_first, sizeof(int) * ((size_t)g->nang * vlor_chunks(gd->dev) + 1));
+  if (e == hipSuccess) e = talloc((void**)&d_i1, sizeof(int) * nrec);
+  if (e == hipSuccess) e = talloc((void**)&d_i2, sizeof(int) * nrec);
+  if (e == hipSuccess) e = talloc((void**)&d_ev, sizeof(int) * ne);
+  if (e == hipSuccess) e = talloc((void**)&d_blankt, sizeof(float) * nd);
+  if (e == hipSuccess) e = talloc((void**)&d_v0, sizeof(float) * nd);
   if (e == hipSuccess && nrec) e = hipMalloc((void**)&d_rec, 2 * sizeof(int) * nrec);
   if (e == hipSuccess && nrec)
     e = hipMemcpyAsync(d_rec, rec, 2 * sizeof(int) * nrec, hipMemcpyHostToDevice, st);
   if (e == hipSuccess) {
     long long nev = 0, nbins = 0;
-    e = build_vlor_lists(d_rec, nrec, nd, v->d_i1, v->d_i2, v->d_bins, v->d_start, v->d_ev, &nev,
+    e = build_vlor_lists(gd->dev, d_rec, nrec, d_i1, d_i2, v->d_bins, v->d_start, d_ev, &nev,
                          &nbins, st);
     v->nev = nev;
     v->nbins = nbins;
@@ -766,15 +763,15 @@ int vlor_create_on(gfr_ctx* ctx, const gfr_geometry* g, const int32_t* rec, long
   }
   // datos_v0 counts on the device (GFIRST.cu:238-239)
   if (e == hipSuccess) e = launch_zero(d_v0, sizeof(float) * nd, st);
-  if (e == hipSuccess) e = launch_vlor_count(v->d_i1, v->d_i2, nev, d_v0, st);
+  if (e == hipSuccess) e = launch_vlor_count(d_i1, d_i2, nev, d_v0, st);
   // BLANKT = T/(RES*v0) where v0 > 0.01 (GFIRST.cu:244-247); T already x RES.
-  if (e == hipSuccess) e = launch_vlor_blankt(d_yT, d_v0, (float)g->res, v->d_blankt, nd, st);
-  // valor per record is static: BLANKT[i1] + BLANKT[i2].
+  if (e == hipSuccess) e = launch_vlor_blankt(d_yT, d_v0, (float)g->res, d_blankt, nd, st);
   if (e == hipSuccess)
-    e = launch_vlor_event(v->d_i1, v->d_i2, v->d_blankt, v->d_blankt, v->d_sinv, v->d_valor, nev,
-                          1, st);
+    e = launch_vlor_lists(gd->dev, v->d_bins, v->d_start, d_ev, d_i1, d_i2, d_blankt, v->nbins,
+                          v->d_ent, v->d_first, st);
   if (e == hipSuccess) e = hipStreamSynchronize(st);
-  if (d_v0) (void)hipFree(d_v0);
+  for (void* p : {(void*)d_v0, (void*)d_i1, (void*)d_i2, (void*)d_blankt, (void*)d_ev})
+    if (p) (void)hipFree(p);
   if (e != hipSuccess) {
     v->ctx = nullptr;  // its bytes were never counted in the context
     gfr_vlor_destroy(v);

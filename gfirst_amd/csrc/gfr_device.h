@@ -204,4 +204,14 @@ __device__ __forceinline__ void store_calib(const DevGeom& G, float2* c2, int ag
   if (k == nz - 1) put(row0 + nz + 1, edge);
 }
 
+// Sinogram bin b in angle-major order, and back.
+__device__ __forceinline__ unsigned vlor_key(const DevGeom& G, int b) {
+  const int row = b / G.nrad, s = row / G.nang;
+  return (unsigned)(((row - s * G.nang) * G.nsinogs + s) * G.nrad + b - row * G.nrad);
+}
+__device__ __forceinline__ int vlor_bin(const DevGeom& G, unsigned key) {
+  const int row = (int)key / G.nrad, it = row / G.nsinogs;
+  return ((row - it * G.nsinogs) * G.nang + it) * G.nrad + (int)key - row * G.nrad;
+}
+
 }  // namespace gfr

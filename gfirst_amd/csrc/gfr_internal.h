@@ -304,21 +304,26 @@ hipError_t launch_vlor_count(const int* i1, const int* i2, long long nev, float*
                              hipStream_t st);
 hipError_t launch_vlor_blankt(const float* yT, const float* v0, float res, float* blankt,
                               long long nd, hipStream_t st);
-hipError_t launch_vlor_event(const int* i1, const int* i2, const float* blankt,
-                             const float* proj, float* sinv, float* valor, long long nev,
-                             int want_valor, hipStream_t st);
-hipError_t launch_vlor_zero_subset(const DevGeom& G, float* dv, int subset, int nsub,
-                                   hipStream_t st);
+// Touched bins are kept by angle, then sinogram, then radial bin (vlor_key), so
+// that the bins of a subset are whole runs; a run is cut into chunks.
+constexpr int kVlorChunk = 1024;
+inline int vlor_chunks(const DevGeom& G) {
+  return (G.nsinogs * G.nrad + kVlorChunk - 1) / kVlorChunk;
+}
 // Valid events and bin -> event lists from raw records (device, `d_rec` holds
-// nrec pairs of 1-based bins); sizes: i1/i2 nrec, bins/ev 2*nrec, start
-// 2*nrec+1. Synchronises `st` and returns the counts.
-hipError_t build_vlor_lists(const int* d_rec, long long nrec, long long nd, int* d_i1, int* d_i2,
-                            long long* d_bins, int* d_start, int* d_ev, long long* nev_out,
+// nrec pairs of 1-based bins); sizes: i1/i2 nrec, bins (vlor_key, ascending)
+// and ev 2*nrec, start 2*nrec+1. Synchronises `st` and returns the counts.
+hipError_t build_vlor_lists(const DevGeom& G, const int* d_rec, long long nrec, int* d_i1,
+                            int* d_i2, unsigned* d_bins, int* d_start, int* d_ev, long long* nev_out,
                             long long* nbins_out, hipStream_t st);
-hipError_t launch_vlor_bins(const DevGeom& G, const long long* bins, const int* start,
-                            const int* ev, long long nbins, const float* proj,
-                            const float* sinv, const float* valor, float* dv, int subset,
-                            int nsub, hipStream_t st);
+// ent: [2*nev] entries of the lists; first: [nang * vlor_chunks + 1].
+hipError_t launch_vlor_lists(const DevGeom& G, const unsigned* bins, const int* start,
+                             const int* ev, const int* i1, const int* i2, const float* blankt,
+                             long long nbins, int2* ent, int* first, hipStream_t st);
+// The subset's bins of dv, touched or not.
+hipError_t launch_vlor_assign(const DevGeom& G, const unsigned* bins, const int* start,
+                              const int2* ent, const int* first, const float* proj, float* dv,
+                              int subset, int nsub, hipStream_t st);
 
 }  // namespace gfr
 
@@ -333,13 +338,9 @@ struct gfr_vlor {
   gfr_geometry g;
   long long nev = 0;      // valid records
   long long nbins = 0;    // touched bins
-  int* d_i1 = nullptr;    // [nev] 0-based
-  int* d_i2 = nullptr;
-  float* d_blankt = nullptr;  // [ndata]
-  float* d_sinv = nullptr;    // [nev]
-  float* d_valor = nullptr;   // [nev]
-  long long* d_bins = nullptr;  // [nbins] bin ids, ascending
-  int* d_start = nullptr;       // [nbins+1] offsets into d_ev
-  int* d_ev = nullptr;          // [2*nev] event ids per bin, record order
+  unsigned* d_bins = nullptr;  // [nbins] vlor_key, ascending
+  int* d_start = nullptr;      // [nbins+1] offsets into d_ent
+  int2* d_ent = nullptr;       // [2*nev] {other bin, valor} per bin, record order
+  int* d_first = nullptr;      // [nang * vlor_chunks + 1] first touched bin of a chunk
   size_t bytes = 0;
 };

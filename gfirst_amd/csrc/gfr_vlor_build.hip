@@ -13,7 +13,7 @@
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
-#include "gfr_internal.h"
+#include "gfr_device.h"
 
 namespace gfr {
 
@@ -32,8 +32,9 @@ __global__ void k_vrec_fill(unsigned* __restrict__ key, long long n, unsigned v)
   if (k < n) key[k] = v;
 }
 
-__global__ void k_vrec_compact(const int* __restrict__ rec, const int* __restrict__ flag,
-                               const int* __restrict__ pos, long long nrec,
+__global__ void k_vrec_compact(DevGeom G, const int* __restrict__ rec,
+                               const int* __restrict__ flag, const int* __restrict__ pos,
+                               long long nrec,
                                int* __restrict__ i1, int* __restrict__ i2,
                                unsigned* __restrict__ key, int* __restrict__ val) {
   const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -42,8 +43,8 @@ __global__ void k_vrec_compact(const int* __restrict__ rec, const int* __restric
   const int a = rec[2 * e] - 1, b = rec[2 * e + 1] - 1;
   i1[p] = a;
   i2[p] = b;
-  key[2 * p] = (unsigned)a;
-  key[2 * p + 1] = (unsigned)b;
+  key[2 * p] = vlor_key(G, a);
+  key[2 * p + 1] = vlor_key(G, b);
   val[2 * p] = p;
   val[2 * p + 1] = p;
 }
@@ -58,10 +59,10 @@ __global__ void k_vrec_runs(const unsigned* __restrict__ key, long long n, unsig
 
 __global__ void k_vrec_starts(const unsigned* __restrict__ key, const int* __restrict__ first,
                               const int* __restrict__ bpos, long long n,
-                              long long* __restrict__ bins, int* __restrict__ start) {
+                              unsigned* __restrict__ bins, int* __restrict__ start) {
   const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n || !first[k]) return;
-  bins[bpos[k]] = (long long)key[k];
+  bins[bpos[k]] = key[k];
   start[bpos[k]] = (int)k;
 }
 
@@ -82,12 +83,12 @@ inline unsigned blocks(long long n) { return (unsigned)((n + 255) / 256); }
 
 }  // namespace
 
-hipError_t build_vlor_lists(const int* d_rec, long long nrec, long long nd, int* d_i1, int* d_i2,
-                            long long* d_bins, int* d_start, int* d_ev, long long* nev_out,
+hipError_t build_vlor_lists(const DevGeom& G, const int* d_rec, long long nrec, int* d_i1,
+                            int* d_i2, unsigned* d_bins, int* d_start, int* d_ev, long long* nev_out,
                             long long* nbins_out, hipStream_t st) {
   *nev_out = *nbins_out = 0;
   if (nrec == 0) return hipSuccess;
-  const long long n = 2 * nrec;
+  const long long n = 2 * nrec, nd = G.ndata;
   int nbits = 1;
   while (nbits < 32 && ((unsigned long long)nd >> nbits) != 0) nbits++;  // nd < 2^nbits
   int *flag = nullptr, *pos = nullptr, *val = nullptr, *first = nullptr, *bpos = nullptr;
@@ -116,8 +117,8 @@ hipError_t build_vlor_lists(const int* d_rec, long long nrec, long long nd, int*
   if (e == hipSuccess) e = hipcub::DeviceScan::ExclusiveSum(tmp, t_scan1, flag, pos, nrec, st);
   if (e == hipSuccess) {
     hipLaunchKernelGGL(k_vrec_fill, dim3(blocks(n)), dim3(256), 0, st, key, n, (unsigned)nd);
-    hipLaunchKernelGGL(k_vrec_compact, dim3(blocks(nrec)), dim3(256), 0, st, d_rec, flag, pos,
-                       nrec, d_i1, d_i2, key, val);
+    hipLaunchKernelGGL(k_vrec_compact, dim3(blocks(nrec)), dim3(256), 0, st, G, d_rec, flag,
+                       pos, nrec, d_i1, d_i2, key, val);
     e = hipGetLastError();
   }
   if (e == hipSuccess)
