@@ -21,10 +21,11 @@ int set_err(gfr_ctx* ctx, int code, const std::string& msg) {
   return code;
 }
 
-bool is_device_ptr(const void* p) {
+bool is_device_ptr(const void* p, int device) {
   if (!p) return false;
   hipPointerAttribute_t at{};
-  const bool dev = hipPointerGetAttributes(&at, p) == hipSuccess && at.type == hipMemoryTypeDevice;
+  const bool dev = hipPointerGetAttributes(&at, p) == hipSuccess && at.type == hipMemoryTypeDevice &&
+                   (device < 0 || at.device == device);
   (void)hipGetLastError();  // a pageable host pointer reports an error: not sticky
   return dev;
 }
@@ -614,7 +615,7 @@ int gfr_image_max(gfr_ctx* ctx, const gfr_geometry* g, const float* d_x, float* 
 int gfr_vlor_create(gfr_ctx* ctx, const gfr_geometry* g, const int32_t* rec, long long nrec,
                     const float* d_yT, gfr_vlor** out) {
   GFR_CHECK_CTX(ctx);
-  return vlor_create_on(ctx, g, rec, nrec, d_yT, ctx->stream, out);
+  return vlor_create_on(ctx, g, rec, nrec, d_yT, 1.f, ctx->stream, out);
 }
 
 int gfr_vlor_assign(gfr_ctx* ctx, gfr_vlor* v, const float* d_proj, float* d_dv, int subset,
@@ -710,7 +711,7 @@ int gfr_tuning_set(gfr_ctx* ctx, const gfr_geometry* g, int nsub, const gfr_tuni
 namespace gfr {
 
 int vlor_create_on(gfr_ctx* ctx, const gfr_geometry* g, const int32_t* rec, long long nrec,
-                   const float* d_yT, hipStream_t st, gfr_vlor** out) {
+                   const float* d_yT, float scale, hipStream_t st, gfr_vlor** out) {
   GFR_GEOM(ctx, g, gd);
   GFR_NONNULL(ctx, out, "out");
   GFR_NONNULL(ctx, d_yT, "d_yT");
@@ -731,7 +732,7 @@ int vlor_create_on(gfr_ctx* ctx, const gfr_geometry* g, const int32_t* rec, long
     v->bytes += b;
     return hipMalloc(p, b ? b : 4);
   };
-  float *d_v0 = nullptr, *d_blankt = nullptr;
+  float* d_v0 = nullptr;
   int *d_rec = nullptr, *d_i1 = nullptr, *d_i2 = nullptr, *d_ev = nullptr;
   auto talloc = [](void** p, size_t b) { return hipMalloc(p, b ? b : 4); };
   hipError_t e = dalloc((void**)&v->d_bins, sizeof(unsigned) * ne);
@@ -742,7 +743,6 @@ int vlor_create_on(gfr_ctx* ctx, const gfr_geometry* g, const int32_t* rec, long
   if (e == hipSuccess) e = talloc((void**)&d_i1, sizeof(int) * nrec);
   if (e == hipSuccess) e = talloc((void**)&d_i2, sizeof(int) * nrec);
   if (e == hipSuccess) e = talloc((void**)&d_ev, sizeof(int) * ne);
-  if (e == hipSuccess) e = talloc((void**)&d_blankt, sizeof(float) * nd);
   if (e == hipSuccess) e = talloc((void**)&d_v0, sizeof(float) * nd);
   if (e == hipSuccess && nrec) e = hipMalloc((void**)&d_rec, 2 * sizeof(int) * nrec);
   if (e == hipSuccess && nrec)
@@ -755,22 +755,16 @@ int vlor_create_on(gfr_ctx* ctx, const gfr_geometry* g, const int32_t* rec, long
     v->nbins = nbins;
   }
   if (d_rec) (void)hipFree(d_rec);
-  const long long nev = v->nev;
   if (e == hipSuccess && nrec == 0) {
     const int zero = 0;
     e = hipMemcpyAsync(v->d_start, &zero, sizeof(int), hipMemcpyHostToDevice, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
   }
-  // datos_v0 counts on the device (GFIRST.cu:238-239)
-  if (e == hipSuccess) e = launch_zero(d_v0, sizeof(float) * nd, st);
-  if (e == hipSuccess) e = launch_vlor_count(d_i1, d_i2, nev, d_v0, st);
-  // BLANKT = T/(RES*v0) where v0 > 0.01 (GFIRST.cu:244-247); T already x RES.
-  if (e == hipSuccess) e = launch_vlor_blankt(d_yT, d_v0, (float)g->res, d_blankt, nd, st);
   if (e == hipSuccess)
-    e = launch_vlor_lists(gd->dev, v->d_bins, v->d_start, d_ev, d_i1, d_i2, d_blankt, v->nbins,
-                          v->d_ent, v->d_first, st);
+    e = launch_vlor_lists(gd->dev, v->d_bins, v->d_start, d_ev, d_i1, d_i2, d_yT, scale,
+                          (float)g->res, d_v0, v->nbins, v->d_ent, v->d_first, st);
   if (e == hipSuccess) e = hipStreamSynchronize(st);
-  for (void* p : {(void*)d_v0, (void*)d_i1, (void*)d_i2, (void*)d_blankt, (void*)d_ev})
+  for (void* p : {(void*)d_v0, (void*)d_i1, (void*)d_i2, (void*)d_ev})
     if (p) (void)hipFree(p);
   if (e != hipSuccess) {
     v->ctx = nullptr;  // its bytes were never counted in the context

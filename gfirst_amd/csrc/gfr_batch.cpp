@@ -440,14 +440,16 @@ int gfr_batch_add(gfr_batch* b, int niter, int nsub, const float* prompts, const
   // A NaN or infinite count fails the frame (as gfr_recon_create).
   unsigned int* bad = (unsigned int*)(stage + nd_al);
   hipError_t e = launch_zero(bad, sizeof(unsigned int), st);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(stage, prompts, sizeof(float) * (size_t)nd, hipMemcpyDefault, st);
-  if (e == hipSuccess) e = launch_any_nonfinite(stage, nd, bad, st);
-  if (e == hipSuccess) e = launch_convert_store(stage, fr.y, b->p.storage, nd, st);
-  if (e == hipSuccess && has_bg)
-    e = hipMemcpyAsync(stage, bg, sizeof(float) * (size_t)nd, hipMemcpyDefault, st);
-  if (e == hipSuccess && has_bg) e = launch_any_nonfinite(stage, nd, bad, st);
-  if (e == hipSuccess && has_bg) e = launch_convert_store(stage, fr.bg, b->p.storage, nd, st);
+  auto upload = [&](const float* src, void* dst) -> hipError_t {
+    hipError_t ee = hipSuccess;
+    if (!is_device_ptr(src, ctx->device)) {
+      ee = hipMemcpyAsync(stage, src, sizeof(float) * (size_t)nd, hipMemcpyDefault, st);
+      src = stage;
+    }
+    return ee == hipSuccess ? launch_store_checked(src, dst, b->p.storage, nd, bad, st) : ee;
+  };
+  if (e == hipSuccess) e = upload(prompts, fr.y);
+  if (e == hipSuccess && has_bg) e = upload(bg, fr.bg);
   if (e == hipSuccess) e = launch_fill_cylinder(G, 1.f, fr.x, st);
   const int cur[2] = {0, nsub};  // host source of the two copies, alive until the sync
   if (e == hipSuccess) e = hipMemcpyAsync(b->d_sub + f, &cur[0], sizeof(int), hipMemcpyHostToDevice, st);

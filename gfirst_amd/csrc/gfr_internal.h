@@ -186,7 +186,7 @@ namespace gfr {
 int set_err(gfr_ctx* ctx, int code, const std::string& msg);
 int hip_err(gfr_ctx* ctx, hipError_t e, const char* where);
 // True for device memory (host and NULL pointers: false).
-bool is_device_ptr(const void* p);
+bool is_device_ptr(const void* p, int device = -1);
 #define GFR_HIP(ctx, call)                                   \
   do {                                                       \
     hipError_t _e = (call);                                  \
@@ -276,15 +276,13 @@ hipError_t launch_jbf(const DevGeom& G, const float* in, const float* guide,
 hipError_t launch_blend(const DevGeom& G, float coef, const float* filt, float* x,
                         hipStream_t st);
 hipError_t launch_max(const DevGeom& G, const float* x, unsigned int* d_bits, hipStream_t st);
-hipError_t launch_scale_copy(const float* in, float s, float* out, long long n, hipStream_t st);
-hipError_t launch_convert_store(const float* in, void* out, int storage, long long n,
-                                hipStream_t st);
 hipError_t launch_llh_final(const double* part, int n, double* out, hipStream_t st);
 // *flag = 1 if some v[i] is not <= 0 (NaN counts); *flag must start at 0.
 hipError_t launch_any_positive(const float* v, long long n, unsigned int* flag, hipStream_t st);
-// *flag = 1 if some v[i] is NaN or infinite; *flag must start at 0.
-hipError_t launch_any_nonfinite(const float* v, long long n, unsigned int* flag,
-                                hipStream_t st);
+// n counts into the storage format; *flag = 1 if one is NaN or infinite (*flag
+// must start at 0).
+hipError_t launch_store_checked(const float* in, void* out, int storage, long long n,
+                                unsigned int* flag, hipStream_t st);
 // sub[slots[i]] = (sub[slots[i]] + 1) mod nsub[slots[i]] for i < n.
 hipError_t launch_advance(int* sub, const int* nsub, const int* slots, int n, hipStream_t st);
 // Synthetic measurements (gfr_synth.hip).
@@ -300,10 +298,6 @@ hipError_t tune_shapes(const DevGeom& G, int nsub, const FwdOut& fo, const float
                        size_t r_floats, float* num, float* den, hipStream_t st, Tune* out);
 
 // VLOR.
-hipError_t launch_vlor_count(const int* i1, const int* i2, long long nev, float* v0,
-                             hipStream_t st);
-hipError_t launch_vlor_blankt(const float* yT, const float* v0, float res, float* blankt,
-                              long long nd, hipStream_t st);
 // Touched bins are kept by angle, then sinogram, then radial bin (vlor_key), so
 // that the bins of a subset are whole runs; a run is cut into chunks.
 constexpr int kVlorChunk = 1024;
@@ -316,10 +310,11 @@ inline int vlor_chunks(const DevGeom& G) {
 hipError_t build_vlor_lists(const DevGeom& G, const int* d_rec, long long nrec, int* d_i1,
                             int* d_i2, unsigned* d_bins, int* d_start, int* d_ev, long long* nev_out,
                             long long* nbins_out, hipStream_t st);
-// ent: [2*nev] entries of the lists; first: [nang * vlor_chunks + 1].
+// T = yT * scale; v0: ndata floats of scratch; ent: [2*nev] entries of the lists; first: [nang * vlor_chunks + 1].
 hipError_t launch_vlor_lists(const DevGeom& G, const unsigned* bins, const int* start,
-                             const int* ev, const int* i1, const int* i2, const float* blankt,
-                             long long nbins, int2* ent, int* first, hipStream_t st);
+                             const int* ev, const int* i1, const int* i2, const float* yT,
+                             float scale, float res, float* v0, long long nbins, int2* ent,
+                             int* first, hipStream_t st);
 // The subset's bins of dv, touched or not.
 hipError_t launch_vlor_assign(const DevGeom& G, const unsigned* bins, const int* start,
                               const int2* ent, const int* first, const float* proj, float* dv,
@@ -330,7 +325,7 @@ hipError_t launch_vlor_assign(const DevGeom& G, const unsigned* bins, const int*
 namespace gfr {
 // gfr_vlor_create with its device work ordered on stream st.
 int vlor_create_on(gfr_ctx* ctx, const gfr_geometry* g, const int32_t* rec, long long nrec,
-                   const float* d_yT, hipStream_t st, gfr_vlor** out);
+                   const float* d_yT, float scale, hipStream_t st, gfr_vlor** out);
 }  // namespace gfr
 
 struct gfr_vlor {

@@ -346,7 +346,8 @@ int gfr_recon_create(gfr_ctx* ctx, const gfr_geometry* g, const gfr_recon_params
   const DevGeom& G = gd->dev;
   r->r_floats = pl.rot / sizeof(float);
   hipError_t e = hipSuccess;
-  // Host arrays reach the device through a transient staging buffer.
+  // Host arrays reach the device through a transient staging buffer; arrays in
+  // this device's memory are read where they are.
   float* stage = nullptr;
   if (dev_alloc(ctx, (void**)&stage, pl.sino_f32) != hipSuccess)
     return rfail(r, set_err(ctx, GFR_ENOMEM, "reconstruction staging allocation failed"));
@@ -356,10 +357,15 @@ int gfr_recon_create(gfr_ctx* ctx, const gfr_geometry* g, const gfr_recon_params
   // selects the calibration mask through its > 0.01 test, where NaN masks
   // the bin and +inf keeps it, as there.
   unsigned int* bad = r->d_maxbits;
-  auto upload = [&](const float* host, void* dst) -> hipError_t {
-    hipError_t ee = hipMemcpyAsync(stage, host, pl.sino_f32, hipMemcpyDefault, st);
-    if (ee == hipSuccess) ee = launch_any_nonfinite(stage, nd, bad, st);
-    if (ee == hipSuccess) ee = launch_convert_store(stage, dst, p->storage, nd, st);
+  auto on_device = [&](const float* src, float* buf, const float** out) -> hipError_t {
+    *out = is_device_ptr(src, ctx->device) ? src : buf;
+    return *out == src ? hipSuccess
+                       : hipMemcpyAsync(buf, src, pl.sino_f32, hipMemcpyDefault, st);
+  };
+  auto upload = [&](const float* src, void* dst) -> hipError_t {
+    const float* v = nullptr;
+    hipError_t ee = on_device(src, stage, &v);
+    if (ee == hipSuccess) ee = launch_store_checked(v, dst, p->storage, nd, bad, st);
     if (ee == hipSuccess) ee = hipStreamSynchronize(st);
     return ee;
   };
@@ -371,8 +377,9 @@ int gfr_recon_create(gfr_ctx* ctx, const gfr_geometry* g, const gfr_recon_params
     e = geom_sino(r, false, 0.f, &pb);
     r->pb = const_cast<float*>(pb);
   }
-  if (e == hipSuccess) e = hipMemcpyAsync(stage, norm, pl.sino_f32, hipMemcpyDefault, st);
-  if (e == hipSuccess) e = launch_calib_mask(G, r->pb, stage, r->mask, st);
+  const float* dnorm = nullptr;
+  if (e == hipSuccess) e = on_device(norm, stage, &dnorm);
+  if (e == hipSuccess) e = launch_calib_mask(G, r->pb, dnorm, r->mask, st);
   if (e == hipSuccess) e = hipStreamSynchronize(st);
   // Measured data, stored unscaled; kernels scale by RES on load (GFIRST.cu:224-260).
   if (e == hipSuccess) e = launch_zero(bad, 64, st);
@@ -396,12 +403,12 @@ int gfr_recon_create(gfr_ctx* ctx, const gfr_geometry* g, const gfr_recon_params
   dev_free(ctx, stage, pl.sino_f32);
   if (e != hipSuccess) return rfail(r, hip_err(ctx, e, "gfr_recon_create"));
   if (p->mode == 3) {
-    // BLANKT needs T x RES (GFIRST.cu:225-226, 246): scale a float copy.
-    e = hipMemcpyAsync(r->ptc, t2, pl.sino_f32, hipMemcpyDefault, st);
-    if (e == hipSuccess) e = launch_scale_copy(r->ptc, (float)g->res, r->dv, nd, st);
+    // BLANKT needs T x RES (GFIRST.cu:225-226, 246).
+    const float* dT = nullptr;
+    e = on_device(t2, r->ptc, &dT);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     if (e != hipSuccess) return rfail(r, hip_err(ctx, e, "gfr_recon_create vlor"));
-    int rc = vlor_create_on(ctx, g, rec, nrec, r->dv, st, &r->vl);
+    int rc = vlor_create_on(ctx, g, rec, nrec, dT, (float)g->res, st, &r->vl);
     if (rc != GFR_OK) return rfail(r, rc);
     // Projection cache of the triples estimate (bins outside the current
     // subset keep their last projection): it starts as the projection of the
