@@ -473,8 +473,12 @@ __global__ __launch_bounds__(256, ZB * NV <= 8 ? 5 : 3) void k_back_window(
     const int iz = zb + j;
     if (iz < G.nzs) {
       const size_t iV = ((size_t)iz * G.res + iy) * G.res + ix;
-      F.numer[fr][iV] = n[j];
-      F.denom[fr][iV] = d[j];
+      if (F.denom[fr]) {
+        F.numer[fr][iV] = n[j];
+        F.denom[fr][iV] = d[j];
+      } else {
+        F.numer[fr][iV] = update_ratio(n[j], d[j]);
+      }
     }
   }
 }

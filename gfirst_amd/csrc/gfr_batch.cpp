@@ -39,8 +39,7 @@ struct Lane {
   float *xb = nullptr, *work = nullptr, *R = nullptr;
   unsigned* bad = nullptr;               // PackedRows::bad
   float* rows[kMaxGroup] = {};           // per frame of a group: packed rows,
-  float* num[kMaxGroup] = {};            // numerator,
-  float* den[kMaxGroup] = {};            // denominator
+  float* num[kMaxGroup] = {};            // update ratio
   double* llh_part = nullptr;
   size_t r_floats = 0;
 };
@@ -80,7 +79,7 @@ Sizes sizes_of(const GeomHost& h, const gfr_batch_params* p) {
   z.frame_nobg = z.img + sino;
   z.frame_bg = z.img + 2 * sino;
   const size_t per_lane =
-      (2 + 2 * (size_t)grp) * z.img + (size_t)grp * z.rows + z.rot + z.llh;
+      (2 + (size_t)grp) * z.img + (size_t)grp * z.rows + z.rot + z.llh;
   const size_t slots = (size_t)p->max_frames * (3 * sizeof(int) + sizeof(double)) + 256;
   z.shared = (size_t)p->lanes * per_lane + (size_t)h.info.ndata /* mask */ + slots;
   return z;
@@ -152,13 +151,12 @@ hipError_t enqueue_forward(gfr_batch* b, int f, const Lane& L, const PackedRows&
   return e;
 }
 
-hipError_t enqueue_update(gfr_batch* b, int f, const float* num, const float* den,
-                          const Lane& L) {
+hipError_t enqueue_update(gfr_batch* b, int f, const float* ratio, const Lane& L) {
   Taps9 tb;
   Taps5 tz;
   psf_taps(b->p.psf_bw, tb.g);
   gz_taps(tz.g);
-  return launch_update(b->gd->dev, tb, tz, num, den, b->frames[f].x, L.work, L.st);
+  return launch_update(b->gd->dev, tb, tz, ratio, nullptr, b->frames[f].x, L.work, L.st);
 }
 
 // Enqueues one subset pass of the frames of a group on lane L: every
@@ -171,13 +169,12 @@ hipError_t enqueue_group(gfr_batch* b, const std::vector<int>& grp, const Lane& 
   for (size_t i = 0; i < grp.size() && e == hipSuccess; i++) {
     F.rows[i] = packed_rows(G, L.rows[i], 0, f0.nsub, L.bad, 1);
     F.numer[i] = L.num[i];
-    F.denom[i] = L.den[i];
     e = enqueue_forward(b, grp[i], L, F.rows[i]);
   }
   if (e == hipSuccess)
     e = launch_back_packed(G, F, (int)grp.size(), 0, f0.nsub, b->d_sub + grp[0], f0.tune, L.st);
   for (size_t i = 0; i < grp.size() && e == hipSuccess; i++)
-    e = enqueue_update(b, grp[i], F.numer[i], F.denom[i], L);
+    e = enqueue_update(b, grp[i], F.numer[i], L);
   return e;
 }
 
@@ -351,8 +348,7 @@ int gfr_batch_create(gfr_ctx* ctx, const gfr_geometry* g, const gfr_batch_params
          A((void**)&L.xb, z.img) && A((void**)&L.work, z.img) && A((void**)&L.R, z.rot) &&
          A((void**)&L.llh_part, z.llh);
     for (int i = 0; i < group_of(p) && ok; i++)
-      ok = A((void**)&L.rows[i], z.rows) && A((void**)&L.num[i], z.img) &&
-           A((void**)&L.den[i], z.img);
+      ok = A((void**)&L.rows[i], z.rows) && A((void**)&L.num[i], z.img);
     L.r_floats = z.rot / sizeof(float);
   }
   if (!ok) return bfail(b, set_err(ctx, GFR_ENOMEM, "batch allocation failed"));
@@ -478,7 +474,7 @@ int gfr_batch_add(gfr_batch* b, int niter, int nsub, const float* prompts, const
     fo.storage = b->p.storage;
     fo.yscale = (float)b->g.res;
     fo.llh_part = L.llh_part;
-    e = tune_shapes(G, nsub, fo, fr.x, L.R, L.r_floats, L.num[0], L.den[0], st, &t);
+    e = tune_shapes(G, nsub, fo, fr.x, L.R, L.r_floats, L.num[0], st, &t);
     if (e != hipSuccess) return undo(hip_err(ctx, e, "gfr_batch_add tuning"));
     std::lock_guard<std::mutex> lk(ctx->mu);
     b->gd->tune[nsub] = t;

@@ -86,6 +86,11 @@ __device__ __forceinline__ void xcd_region(int& bx, int& by, int& bz) {
   }
 }
 
+// divVxVGPU (GFIRST_GPU_Kernels.cu:173-182)
+__device__ __forceinline__ float update_ratio(float num, float den) {
+  return (den < 0.001f) ? 1.0f : num / den;
+}
+
 // Lanes of one wave exchange values through LDS: orders what the wave wrote
 // before what it reads, without a barrier (DS operations of a wave are in
 // order).

@@ -236,7 +236,8 @@ hipError_t launch_forward(const DevGeom& G, const float* img, float* R, size_t r
                           const FwdOut& out, int subset, int nsub, const int* dsub,
                           const Tune& tune, hipStream_t st);
 // Backprojection of the packed rows of nf frames (same geometry, subset and
-// mask) into their numerators and denominators, in one launch.
+// mask) into their numerators and denominators, in one launch; without a
+// denominator array (null), numer takes the update ratio of the two.
 constexpr int kMaxGroup = 3;
 struct BackFrames {
   PackedRows rows[kMaxGroup];
@@ -268,6 +269,7 @@ PackedRows packed_rows(const DevGeom& G, void* buf, int subset, int nsub, unsign
                        unsigned epoch);
 hipError_t launch_pack(const DevGeom& G, const float* corr, const uint8_t* mask,
                        const PackedRows& P, int subset, int nsub, hipStream_t st);
+// (denom null: numer is the update ratio)
 hipError_t launch_update(const DevGeom& G, const Taps9& t9, const Taps5& t5, const float* numer,
                          const float* denom, float* x, float* work, hipStream_t st);
 hipError_t launch_jbf(const DevGeom& G, const float* in, const float* guide,
@@ -295,7 +297,7 @@ int llh_capacity(const GeomHost& h, int nsub);
 // Times each tile shape of the two projectors on the given buffers (subset 0)
 // and returns the fastest; any shape gives identical results.
 hipError_t tune_shapes(const DevGeom& G, int nsub, const FwdOut& fo, const float* img, float* R,
-                       size_t r_floats, float* num, float* den, hipStream_t st, Tune* out);
+                       size_t r_floats, float* num, hipStream_t st, Tune* out);
 
 // VLOR.
 // Touched bins are kept by angle, then sinogram, then radial bin (vlor_key), so

@@ -12,127 +12,188 @@ namespace gfr {
 
 namespace {
 
-// Ratio alone (GFIRST.cu:415-430) over the subset's bins; the background is
-// in storage format S.
+__device__ __forceinline__ Float4u load4(const float* p, int m) {
+  if (m == 4) return *(const Float4u*)p;
+  return Float4u{p[0], m > 1 ? p[1] : 0.f, m > 2 ? p[2] : 0.f, 0.f};
+}
+
+// Ratio alone (GFIRST.cu:415-430) over the subset's bins, 4 of a row a thread;
+// the background is in storage format S. One subset of 16 at 128x160x4319 bins
+// with packed rows: 29 -> 21 us (one bin a thread before).
 template <int S>
-__global__ void k_ratio(DevGeom G, const float* __restrict__ proj, const float* __restrict__ y,
-                        const void* __restrict__ bg, float yscale, float* __restrict__ corr,
-                        PackedRows P, const uint8_t* __restrict__ mask, int subset, int nsub) {
-  const int r = blockIdx.x * kWave + threadIdx.x;
-  const int s = blockIdx.y * 4 + threadIdx.y;
-  const int it = subset + (int)blockIdx.z * nsub;
-  if (r >= G.nrad || s >= G.nsinogs) return;
+__global__ __launch_bounds__(256) void k_ratio(DevGeom G, const float* __restrict__ proj,
+                                               const float* __restrict__ y,
+                                               const void* __restrict__ bg, float yscale,
+                                               float* __restrict__ corr, PackedRows P,
+                                               const uint8_t* __restrict__ mask, int subset,
+                                               int nsub) {
+  const int quads = (G.nrad + 3) / 4;
+  const int i = blockIdx.x * 256 + threadIdx.x, s = i / quads, r = (i - s * quads) * 4;
+  const int it = subset + (int)blockIdx.y * nsub;
+  if (s >= G.nsinogs) return;
+  const int m = min(4, G.nrad - r);
   const size_t bin = ((size_t)s * G.nang + it) * G.nrad + r;
-  const float p = proj[bin];
-  const float yv = yscale * y[bin];
-  float bv = bg ? yscale * load_store<S>(bg, bin) : 0.f;
-  if (bv < 0.f) bv = 0.f;
-  const float den = p + bv;
-  const float c = (den >= 0.01f) ? yv / den : -1000.f;
-  if (corr) corr[bin] = c;
-  if (P.v) {
-    const float c4[4] = {c, 0.f, 0.f, 0.f};
-    const bool valid[4] = {mask[bin] != 0, true, true, true};
-    store_packed(G, P, blockIdx.z, s, r, 1, c4, valid);
+  const Float4u pv = load4(proj + bin, m), yy = load4(y + bin, m);
+  const float p[4] = {pv.x, pv.y, pv.z, pv.w}, yv[4] = {yy.x, yy.y, yy.z, yy.w};
+  float c[4];
+  bool valid[4];
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    float bv = bg && k < m ? yscale * load_store<S>(bg, bin + k) : 0.f;
+    if (bv < 0.f) bv = 0.f;
+    const float den = p[k] + bv;
+    c[k] = (den >= 0.01f) ? yscale * yv[k] / den : -1000.f;
+    valid[k] = P.v && k < m ? mask[bin + k] != 0 : true;
+    if (corr && k < m) corr[bin + k] = c[k];
   }
+  if (P.v) store_packed(G, P, blockIdx.y, s, r, m, c, valid);
 }
 
 // ---------------------------------------------------------------------------
-// XY blur (convolutionXY_GPU, GFIRST_GPU_Kernels.cu:332-358). One block per
-// (plane, 4 rows); the plane's rows y-4..y+4 go through LDS once. SRC reads
-// the input value (plain load, or the update ratio NUMER/DENOM).
+// XY blur (convolutionXY_GPU, GFIRST_GPU_Kernels.cu:332-358). SRC reads the
+// input value (plain load, or the update ratio NUMER/DENOM).
 // ---------------------------------------------------------------------------
 struct SrcPlain {
+  static constexpr bool kStage = false;
   const float* p;
   __device__ __forceinline__ float operator()(size_t i) const { return p[i]; }
 };
 struct SrcRatio {  // divVxVGPU (GFIRST_GPU_Kernels.cu:173-182)
+  static constexpr bool kStage = true;  // a division per element: once, in LDS
   const float* num;
   const float* den;
   __device__ __forceinline__ float operator()(size_t i) const {
     const float b = den[i];
-    return (b < 0.001f) ? 1.0f : num[i] / b;
+    return update_ratio(num[i], b);
   }
 };
 
-// One block per (plane, kBlurRows output rows): the input rows y-4..y+kBlurRows+3
-// are loaded once into LDS (zero outside the plane), y-filtered in LDS, then
-// x-filtered; the SRC functor is evaluated once per loaded element.
-constexpr int kBlurRows = 16;
+// One block per (plane, kBlurRows output rows). A thread loads the rows that
+// kBlurCol outputs of one column need (zero outside the plane), y-filters them in registers and leaves them in LDS;
+// then a thread x-filters four neighbouring columns from three 16-byte reads.
+// What bounds it: the chain of loads, barrier and LDS reads, at about twice the
+// time its bytes take. 128x128x159: 13 -> 8.7 us; with the ratio, whose divisions are
+// done once in LDS, 18 -> 13 us (all through LDS by single words before).
+constexpr int kBlurRows = 16, kBlurCol = 8;
+__host__ __device__ inline int blur_stride(int res) { return (res + 3) / 4 * 4; }
 
 template <class Src>
 __global__ __launch_bounds__(256) void k_blur_xy(int res, int nzs, Taps9 t, Src src,
                                                  float* __restrict__ out) {
-  extern __shared__ float lds[];
-  float* in = lds;                           // (kBlurRows + 8) x res
-  float* yc = lds + (kBlurRows + 8) * res;   // kBlurRows x res
-  const int z = blockIdx.y;
+  extern __shared__ __align__(16) float yc[];  // kBlurRows rows of blur_stride(res)
+  const int z = blockIdx.y, stride = blur_stride(res);
   const int y0 = blockIdx.x * kBlurRows;
   const int nrows = min(kBlurRows, res - y0);
   const size_t pb = (size_t)z * res * res;
   const int tid = threadIdx.x;
-  const int nin = (nrows + 8) * res;
-  for (int i = tid; i < nin; i += 256) {
-    const int row = i / res, col = i - row * res;
-    const int y = y0 + row - 4;
-    in[i] = (y >= 0 && y < res) ? src(pb + (size_t)y * res + col) : 0.f;
-  }
-  __syncthreads();
-  const int nout = nrows * res;
-  for (int i = tid; i < nout; i += 256) {
-    const int row = i / res, col = i - row * res;
-    float acc = in[row * res + col] * t.g[0];
-#pragma unroll
-    for (int j = 1; j < 9; j++) acc = fmaf(in[(row + j) * res + col], t.g[j], acc);
-    yc[i] = acc;
-  }
-  __syncthreads();
-  for (int i = tid; i < nout; i += 256) {
-    const int row = i / res, x = i - row * res;
-    float o;
-    if (x > 3 && x < res - 4) {
-      const float* yr = yc + row * res + x - 4;
-      o = yr[0] * t.g[0];
-#pragma unroll
-      for (int k = 1; k < 9; k++) o = fmaf(yr[k], t.g[k], o);
-    } else {
-      o = in[(row + 4) * res + x];  // raw input at the x borders
+  float* const staged = yc + kBlurRows * stride;  // kBlurRows + 8 rows
+  if constexpr (Src::kStage) {
+    for (int i = tid; i < (nrows + 8) * res; i += 256) {
+      const int y = y0 - 4 + i / res;
+      staged[i] = (y >= 0 && y < res) ? src(pb + (size_t)(y0 * res) + i - 4 * res) : 0.f;
     }
-    out[pb + (size_t)(y0 + row) * res + x] = o;
+    __syncthreads();
+  }
+  for (int i = tid; i < (kBlurRows / kBlurCol) * res; i += 256) {
+    const int g = i / res, x = i - g * res, r0 = g * kBlurCol, ya = y0 + r0 - 4;
+    if (r0 >= nrows) break;
+    float in[kBlurCol + 8];
+#pragma unroll
+    for (int j = 0; j < kBlurCol + 8; j++) {
+      const int y = ya + j;
+      if constexpr (Src::kStage)
+        in[j] = staged[(r0 + j) * res + x];
+      else
+        in[j] = (y >= 0 && y < res) ? src(pb + (size_t)y * res + x) : 0.f;
+    }
+    const bool border = x < 4 || x >= res - 4;  // raw input at the x borders
+#pragma unroll
+    for (int k = 0; k < kBlurCol; k++) {
+      float acc = in[k] * t.g[0];
+#pragma unroll
+      for (int j = 1; j < 9; j++) acc = fmaf(in[k + j], t.g[j], acc);
+      yc[(r0 + k) * stride + x] = acc;
+      if (border && r0 + k < nrows) out[pb + (size_t)(y0 + r0 + k) * res + x] = in[k + 4];
+    }
+  }
+  __syncthreads();
+  const int quads = (res + 3) / 4;
+  for (int i = tid; i < nrows * quads; i += 256) {
+    const int row = i / quads, x = (i - row * quads) * 4;
+    if (x < 4 || x >= res - 4) continue;
+    const float* yr = yc + row * stride + x - 4;
+    float v[12];
+#pragma unroll
+    for (int k = 0; k < 3; k++) *(float4*)(v + 4 * k) = ((const float4*)yr)[k];
+    float o[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      o[c] = v[c] * t.g[0];
+#pragma unroll
+      for (int k = 1; k < 9; k++) o[c] = fmaf(v[c + k], t.g[k], o[c]);
+    }
+    float* p = out + pb + (size_t)(y0 + row) * res + x;
+    if (x + 4 <= res - 4) {
+      *(Float4u*)p = Float4u{o[0], o[1], o[2], o[3]};
+    } else {
+#pragma unroll
+      for (int c = 0; c < 4; c++)
+        if (x + c < res - 4) p[c] = o[c];
+    }
   }
 }
 
 // Gz with the reference's index shift, multiply, slice copies
-// (GFIRST_CPU_Kernels.cpp:174-186; GFIRST.cu:491-502). One thread per voxel
-// of slices 1..NZS-2; slices 0 and NZS-1 receive copies of slices 1 and
-// NZS-2, so each voxel is read and written by one thread only (in place).
+// (GFIRST_CPU_Kernels.cpp:174-186; GFIRST.cu:491-502), for slices 1..NZS-2, 4
+// voxels a thread; slices 0 and NZS-1 receive copies of slices 1 and NZS-2, so
+// each voxel is read and written by one thread only (in place). The reference
+// takes the slice of voxel n as K = (n - 1) / RES^2: that is z, except for a
+// slice's first voxel. 128x128x159: 10.7 -> 9.7 us (single voxels and a
+// 64-bit division each before).
 __global__ __launch_bounds__(256) void k_gz_mul(int res, int nzs, Taps5 t,
                                                 const float* __restrict__ f1,
                                                 float* __restrict__ x) {
-  const int ix = blockIdx.x * kWave + threadIdx.x;
-  const int iy = blockIdx.y * 4 + threadIdx.y;
-  const int z = blockIdx.z + 1;
-  if (ix >= res || iy >= res || z > nzs - 2) return;
-  const long long r2 = (long long)res * res;
-  const long long nv = r2 * nzs;
-  const long long n = z * r2 + (long long)iy * res + ix;
-  const int K = (int)((n - 1) / r2);
-  auto rd = [&](long long j) -> float { return (j >= 0 && j < nv) ? f1[j] : 0.f; };
-  float v;
-  if (K == 0) {
-    v = 0.5f * rd(n) + 0.5f * rd(n + r2);
-  } else if (K == nzs - 1) {
-    v = 0.5f * rd(n - r2) + 0.5f * rd(n);
-  } else if (K == 1 || K == nzs - 2) {
-    v = 0.333f * rd(n - r2) + 0.333f * rd(n) + 0.333f * rd(n + r2);
-  } else {
-    v = t.g[0] * rd(n - 2 * r2) + t.g[1] * rd(n - r2) + t.g[2] * rd(n) + t.g[3] * rd(n + r2) +
-        t.g[4] * rd(n + 2 * r2);
+  const int q = (blockIdx.x * 256 + threadIdx.x) * 4, r2 = res * res;
+  const int z = blockIdx.y + 1, m = min(4, r2 - q);
+  if (m <= 0) return;
+  const size_t n = (size_t)z * r2 + q;
+  // slices z - 2 .. z + 2 (zero outside the volume)
+  float s[5][4];
+#pragma unroll
+  for (int k = 0; k < 5; k++) {
+    const int zz = z + k - 2;
+    const Float4u v = zz >= 0 && zz < nzs ? load4(f1 + (size_t)zz * r2 + q, m)
+                                          : Float4u{0.f, 0.f, 0.f, 0.f};
+    s[k][0] = v.x, s[k][1] = v.y, s[k][2] = v.z, s[k][3] = v.w;
   }
-  const float nx = x[n] * v;
-  x[n] = nx;
-  if (z == 1) x[n - r2] = nx;
-  if (z == nzs - 2) x[n + r2] = nx;
+  const Float4u xv = load4(x + n, m);
+  const float xi[4] = {xv.x, xv.y, xv.z, xv.w};
+  float o[4];
+#pragma unroll
+  for (int c = 0; c < 4; c++) {
+    const int K = q + c == 0 ? z - 1 : z;
+    float v;
+    if (K == 0)
+      v = 0.5f * s[2][c] + 0.5f * s[3][c];
+    else if (K == 1 || K == nzs - 2)
+      v = 0.333f * s[1][c] + 0.333f * s[2][c] + 0.333f * s[3][c];
+    else
+      v = t.g[0] * s[0][c] + t.g[1] * s[1][c] + t.g[2] * s[2][c] + t.g[3] * s[3][c] +
+          t.g[4] * s[4][c];
+    o[c] = xi[c] * v;
+  }
+  auto put = [&](float* p) {
+    if (m == 4) {
+      *(Float4u*)p = Float4u{o[0], o[1], o[2], o[3]};
+    } else {
+#pragma unroll
+      for (int c = 0; c < 3; c++)
+        if (c < m) p[c] = o[c];
+    }
+  };
+  put(x + n);
+  if (z == 1) put(x + n - r2);
+  if (z == nzs - 2) put(x + n + r2);
 }
 
 // ---------------------------------------------------------------------------
@@ -382,21 +443,25 @@ __global__ void k_blend(long long nv, float coef, const float* __restrict__ filt
 }
 
 // max(0, max x): non-negative floats order like their bit patterns.
-__global__ void k_max(long long nv, const float* __restrict__ x, unsigned int* bits) {
+// 128x128x159: 17 -> 9 us (single words from 1024 blocks before).
+__global__ __launch_bounds__(256) void k_max(long long nv, const float* __restrict__ x,
+                                             unsigned int* bits) {
   __shared__ unsigned int red[256];
-  unsigned int m = 0;
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < nv;
-       i += (long long)gridDim.x * blockDim.x) {
-    const float v = x[i];
-    if (v > 0.f) m = max(m, __float_as_uint(v));
+  float m4 = 0.f;
+#pragma unroll 4
+  for (long long i = ((long long)blockIdx.x * 256 + threadIdx.x) * 4; i < nv;
+       i += (long long)gridDim.x * 1024) {
+    const Float4u v = load4(x + i, (int)min(4ll, nv - i));
+    m4 = fmaxf(fmaxf(fmaxf(m4, v.x), v.y), fmaxf(v.z, v.w));  // a NaN is passed over
   }
+  const unsigned int m = m4 > 0.f ? __float_as_uint(m4) : 0;
   red[threadIdx.x] = m;
   __syncthreads();
   for (int w = 128; w > 0; w >>= 1) {
     if ((int)threadIdx.x < w) red[threadIdx.x] = max(red[threadIdx.x], red[threadIdx.x + w]);
     __syncthreads();
   }
-  if (threadIdx.x == 0) atomicMax(bits, red[0]);
+  if (threadIdx.x == 0 && red[0]) atomicMax(bits, red[0]);
 }
 
 __global__ void k_fill_cylinder(int res, int nzs, float val, float* __restrict__ img) {
@@ -434,11 +499,6 @@ __device__ __forceinline__ void each_item(long long n, Fn fn) {
     if (i < n) fn(i, (int)min(4ll, n - i));
   }
 }
-__device__ __forceinline__ Float4u load4(const float* p, int m) {
-  if (m == 4) return *(const Float4u*)p;
-  return Float4u{p[0], m > 1 ? p[1] : 0.f, m > 2 ? p[2] : 0.f, 0.f};
-}
-
 // Calibration mask (GFIRST.cu:453-458). The reference compares in double; a
 // float is above 0.01 exactly where it is above the float nearest to it, which
 // is smaller.
@@ -674,8 +734,9 @@ hipError_t launch_zero(void* p, size_t bytes, hipStream_t st) {
 
 template <class Src>
 hipError_t blur_launch(const DevGeom& G, const Taps9& t, Src src, float* out, hipStream_t st) {
-  const size_t lds = sizeof(float) * (size_t)(2 * kBlurRows + 8) * G.res;
-  if (lds > 160 * 1024) return hipErrorInvalidValue;
+  const size_t lds = sizeof(float) * ((size_t)kBlurRows * blur_stride(G.res) +
+                                     (Src::kStage ? (size_t)(kBlurRows + 8) * G.res : 0));
+  if (sizeof(float) * (size_t)(2 * kBlurRows + 8) * G.res > 160 * 1024) return hipErrorInvalidValue;
   dim3 grid((G.res + kBlurRows - 1) / kBlurRows, G.nzs);
   hipLaunchKernelGGL(k_blur_xy<Src>, grid, dim3(256), lds, st, G.res, G.nzs, t, src, out);
   return hipGetLastError();
@@ -690,15 +751,15 @@ hipError_t launch_ratio(const DevGeom& G, const float* proj, const float* y, con
                         int storage, float yscale, float* corr, const PackedRows& P,
                         const uint8_t* mask, int subset, int nsub, hipStream_t st) {
   const int nav = nav_of(G, subset, nsub);
-  dim3 grid((G.nrad + kWave - 1) / kWave, (G.nsinogs + 3) / 4, nav);
+  const dim3 grid((unsigned)((G.nsinogs * ((G.nrad + 3) / 4) + 255) / 256), nav);
   if (storage == GFR_STORE_F16)
-    hipLaunchKernelGGL(k_ratio<GFR_STORE_F16>, grid, dim3(kWave, 4), 0, st, G, proj, y, bg,
+    hipLaunchKernelGGL(k_ratio<GFR_STORE_F16>, grid, dim3(256), 0, st, G, proj, y, bg,
                        yscale, corr, P, mask, subset, nsub);
   else if (storage == GFR_STORE_BF16)
-    hipLaunchKernelGGL(k_ratio<GFR_STORE_BF16>, grid, dim3(kWave, 4), 0, st, G, proj, y, bg,
+    hipLaunchKernelGGL(k_ratio<GFR_STORE_BF16>, grid, dim3(256), 0, st, G, proj, y, bg,
                        yscale, corr, P, mask, subset, nsub);
   else
-    hipLaunchKernelGGL(k_ratio<GFR_STORE_F32>, grid, dim3(kWave, 4), 0, st, G, proj, y, bg,
+    hipLaunchKernelGGL(k_ratio<GFR_STORE_F32>, grid, dim3(256), 0, st, G, proj, y, bg,
                        yscale, corr, P, mask, subset, nsub);
   return hipGetLastError();
 }
@@ -712,11 +773,12 @@ hipError_t launch_calib_mask(const DevGeom& G, const float* pb, const float* nor
 
 hipError_t launch_update(const DevGeom& G, const Taps9& t9, const Taps5& t5, const float* numer,
                          const float* denom, float* x, float* work, hipStream_t st) {
-  hipError_t e = blur_launch(G, t9, SrcRatio{numer, denom}, work, st);
+  hipError_t e = denom ? blur_launch(G, t9, SrcRatio{numer, denom}, work, st)
+                       : blur_launch(G, t9, SrcPlain{numer}, work, st);
   if (e != hipSuccess) return e;
   if (G.nzs >= 3)
-    hipLaunchKernelGGL(k_gz_mul, grid_img(G, G.nzs - 2), dim3(kWave, 4), 0, st, G.res, G.nzs, t5,
-                       work, x);
+    hipLaunchKernelGGL(k_gz_mul, dim3((G.res * G.res + 1023) / 1024, G.nzs - 2), dim3(256), 0, st,
+                       G.res, G.nzs, t5, work, x);
   return hipGetLastError();
 }
 
@@ -754,7 +816,7 @@ hipError_t launch_blend(const DevGeom& G, float coef, const float* filt, float* 
 hipError_t launch_max(const DevGeom& G, const float* x, unsigned int* d_bits, hipStream_t st) {
   hipError_t e = launch_zero(d_bits, 4, st);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_max, dim3(1024), dim3(256), 0, st, G.nvox, x, d_bits);
+  hipLaunchKernelGGL(k_max, dim3(512), dim3(256), 0, st, G.nvox, x, d_bits);
   return hipGetLastError();
 }
 

@@ -858,7 +858,7 @@ int llh_capacity(const GeomHost& h, int nsub) {
 }
 
 hipError_t tune_shapes(const DevGeom& G, int nsub, const FwdOut& fo, const float* img, float* R,
-                       size_t r_floats, float* num, float* den, hipStream_t st, Tune* out) {
+                       size_t r_floats, float* num, hipStream_t st, Tune* out) {
   hipEvent_t e0, e1;
   if (hipEventCreate(&e0) != hipSuccess) return hipErrorUnknown;
   if (hipEventCreate(&e1) != hipSuccess) {
@@ -926,7 +926,7 @@ hipError_t tune_shapes(const DevGeom& G, int nsub, const FwdOut& fo, const float
     tt.back_ahead = c[2];
     tt.tuned = true;
     const float ms = time_it([&] {
-      return launch_back_packed(G, {{fo.rows}, {num}, {den}}, 1, 0, nsub, nullptr, tt, st);
+      return launch_back_packed(G, {{fo.rows}, {num}}, 1, 0, nsub, nullptr, tt, st);
     });
     if (ms < bb) {
       bb = ms;

@@ -34,7 +34,7 @@ struct gfr_recon {
   hipStream_t st = nullptr;
   int ntypes = 1;
   // image-sized
-  float *xD = nullptr, *xT = nullptr, *xb = nullptr, *num = nullptr, *den = nullptr,
+  float *xD = nullptr, *xT = nullptr, *xb = nullptr, *num = nullptr,
         *work = nullptr, *jo = nullptr;
   // sinogram-sized
   float *pb = nullptr, *ptc = nullptr, *dv = nullptr;
@@ -50,7 +50,7 @@ struct gfr_recon {
   int llh_valid = 0;
   // triples chain (modes 2-3): stream, scratch, the doubles snapshot
   hipStream_t stT = nullptr;
-  float *xbT = nullptr, *numT = nullptr, *denT = nullptr, *workT = nullptr, *xDs = nullptr;
+  float *xbT = nullptr, *numT = nullptr, *workT = nullptr, *xDs = nullptr;
   float* rowsT = nullptr;
   float* RT = nullptr;
   double *llh_partT = nullptr, *d_llhT = nullptr;
@@ -103,9 +103,9 @@ Plan plan_of(const GeomHost& h, const gfr_recon_params* p, bool bgD, bool bgT) {
            std::min(nav, (size_t)kRotChunk);
   const bool two = p->mode >= 2;
   pl.two = two;
-  // xD num den work xb (+ xT jo, and the triples chain's xb num den work and
+  // xD num work xb and one more (+ xT jo, and the triples chain's xb num work and
   // the doubles snapshot)
-  pl.nimg = 6 + (two ? 7 : 0);
+  pl.nimg = 5 + (two ? 6 : 0);
   pl.nsino_f32 = p->mode == 3 ? 2 : 0;              // ptc dv (PROJ_BLANK is per geometry)
   pl.nsino_store = 1 + (bgD ? 1 : 0) + (two ? 1 + (bgT ? 1 : 0) : 0);
   return pl;
@@ -182,7 +182,7 @@ hipError_t autotune(gfr_recon* r) {
   fo.yscale = (float)r->g.res;
   fo.llh_part = r->llh_part;
   Tune t;
-  hipError_t e = tune_shapes(gd->dev, S, fo, r->xb, r->R, r->r_floats, r->num, r->den, r->st, &t);
+  hipError_t e = tune_shapes(gd->dev, S, fo, r->xb, r->R, r->r_floats, r->num, r->st, &t);
   if (e != hipSuccess) return e;
   r->tune = t;
   std::lock_guard<std::mutex> lk(r->ctx->mu);
@@ -321,7 +321,7 @@ int gfr_recon_create(gfr_ctx* ctx, const gfr_geometry* g, const gfr_recon_params
     r->owned.push_back({*ptr, nb});
     return true;
   };
-  bool ok = A((void**)&r->xD, pl.img) && A((void**)&r->num, pl.img) && A((void**)&r->den, pl.img) &&
+  bool ok = A((void**)&r->xD, pl.img) && A((void**)&r->num, pl.img) &&
             A((void**)&r->work, pl.img) && A((void**)&r->xb, pl.img) &&
             A((void**)&r->rows, pl.rows) && A((void**)&r->R, pl.rot) &&
             A((void**)&r->mask, pl.mask) && A((void**)&r->yD, pl.sino_store) &&
@@ -331,7 +331,7 @@ int gfr_recon_create(gfr_ctx* ctx, const gfr_geometry* g, const gfr_recon_params
   if (ok && r->ntypes == 2)
     ok = A((void**)&r->xT, pl.img) && A((void**)&r->jo, pl.img) && A(&r->yT, pl.sino_store) &&
          (!hasBgT || A(&r->bT, pl.sino_store)) && A((void**)&r->xbT, pl.img) &&
-         A((void**)&r->numT, pl.img) && A((void**)&r->denT, pl.img) &&
+         A((void**)&r->numT, pl.img) &&
          A((void**)&r->workT, pl.img) && A((void**)&r->xDs, pl.img) &&
          A((void**)&r->rowsT, pl.rows) && A((void**)&r->RT, pl.rot) && A((void**)&r->llh_partT, pl.llh) &&
          A((void**)&r->d_llhT, 64);
@@ -442,7 +442,6 @@ int gfr_recon_step(gfr_recon* r) {
   float* R = tc ? r->RT : r->R;
   const PackedRows rows = packed_rows(G, tc ? r->rowsT : r->rows, s, S, r->d_maxbits + 8 + (tc ? 1 : 0), 1);
   float* num = tc ? r->numT : r->num;
-  float* den = tc ? r->denT : r->den;
   float* work = tc ? r->workT : r->work;
   double* llh_part = tc ? r->llh_partT : r->llh_part;
   double* d_llh = tc ? r->d_llhT : r->d_llh;
@@ -503,11 +502,11 @@ int gfr_recon_step(gfr_recon* r) {
   // Backprojection of the subset (GFIRST.cu:436-469) and update (:482-502).
   {
     PhaseMark pm(r, GFR_PHASE_BACK, st);
-    GFR_HIP(ctx, launch_back_packed(G, {{rows}, {num}, {den}}, 1, s, S, nullptr, r->tune, st));
+    GFR_HIP(ctx, launch_back_packed(G, {{rows}, {num}}, 1, s, S, nullptr, r->tune, st));
   }
   {
     PhaseMark pm(r, GFR_PHASE_UPDATE, st);
-    GFR_HIP(ctx, launch_update(G, tb, tz, num, den, x, work, st));
+    GFR_HIP(ctx, launch_update(G, tb, tz, num, nullptr, x, work, st));
   }
   if (tc) {
     // Joint bilateral filter of triples guided by doubles + blend (:504-526).
