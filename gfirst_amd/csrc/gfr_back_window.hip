@@ -23,8 +23,9 @@
 // (exactly rounded like the additions they stand for).
 //
 // Measured (pack and backprojection of one subset, before and after): 128x128x
-// 159 voxels, 530 views of 128 bins: 602 -> 292 us; the same image, 210 views of
-// 147 bins with detector gaps: 255 -> 206 us; 64x64x32, 176 views: 189 -> 59 us.
+// 159 voxels, 530 views of 128 bins: 604 -> 289 us; the same image, 210 views of
+// 147 bins with detector gaps: 254 -> 202 us; 64x64x32, 176 views: 190 -> 45 us
+// (57 with one wave per tile and slice).
 //
 // Where the calibration went: the calibration of a bin is 1 or -1000, and the
 // interpolated calibration B of four valid bins is exactly 1. Rows therefore
@@ -115,14 +116,18 @@ __device__ __forceinline__ void exact_view(const DevGeom& G, __amdgpu_buffer_rsr
   }
 }
 
-// NV views are taken at a time: their windows are loaded together and the next
-// NV are in flight meanwhile (small images, where a wave's walk over the views,
-// a chain of memory round trips, sets the time; windows of at most 16 rows).
+// One slice per wave, for small images, where a wave's walk over the views, a
+// chain of instructions and round trips, sets the time (windows of at most 16
+// rows). NV views are taken at a time: their windows are loaded together and
+// the next NV are in flight meanwhile.
+// SPLIT: the four waves of a block share a tile and slice and take NV views each
+// a turn. They leave their samples in LDS, and one wave after the other adds a
+// turn's samples to the sums in the order of the views.
 // TAB: the radial part of every angle of the subset is kept in LDS (few
 // angles), else it is computed per view.
 // WIN false: the same sums with every pair gathered from the rows, for
 // geometries whose tiles need wider windows.
-template <int ZB, int NV, bool TAB, bool WIN>
+template <int ZB, int NV, bool TAB, bool WIN, bool SPLIT>
 __global__ __launch_bounds__(256, ZB * NV <= 8 ? 5 : 3) void k_back_window(
     DevGeom G, BackFrames F, int nf, int subset, int nsub, const int* __restrict__ dsub, int tabf,
     int wrows) {
@@ -141,7 +146,8 @@ __global__ __launch_bounds__(256, ZB * NV <= 8 ? 5 : 3) void k_back_window(
   // The four waves of a block take the same columns and neighbouring slabs,
   // counted from the middle of the volume outwards: the middle slabs see the
   // most views, so the heaviest blocks start first and the last ones are light.
-  const int ns = (G.nzs + ZB - 1) / ZB, sk = bz * 4 + wv;
+  // (the waves of a split block take one slab)
+  const int ns = (G.nzs + ZB - 1) / ZB, sk = SPLIT ? bz : bz * 4 + wv;
   const int zb = ((sk & 1) ? (ns - 1) / 2 + (sk + 1) / 2 : (ns - 1) / 2 - sk / 2) * ZB;
   const int ix = bx * 8 + (lane & 7), iy = by * 8 + (lane >> 3);
   const bool act = ix < G.res && iy < G.res;
@@ -159,7 +165,7 @@ __global__ __launch_bounds__(256, ZB * NV <= 8 ? 5 : 3) void k_back_window(
     }
     __syncthreads();
   }
-  if (sk >= ns) return;  // no barrier follows
+  if (sk >= ns) return;  // of four slabs: no barrier follows
   const bool bad = *P.bad == P.epoch;
   const unsigned rowb = (unsigned)packed_row_len(G.nrad) * 4u;
   const unsigned nr = (unsigned)(G.nsinogs + 2 * G.nseg);
@@ -224,6 +230,21 @@ __global__ __launch_bounds__(256, ZB * NV <= 8 ? 5 : 3) void k_back_window(
       d[j] += e;
     }
   };
+
+  // split blocks: samples of two turns, what they count where that is not 1 or
+  // 0, sums, and per wave the views of a turn that have such samples
+  constexpr int kTurn = 4 * NV;
+  float* const smp = win + 4 * NV * wrows * kWinStride;
+  float* const cts = smp + 2 * kTurn * 64;
+  float* const sums = cts + 2 * kTurn * 64;
+  int* const rare = (int*)(sums + 128);
+  int turn = 0;
+  if constexpr (SPLIT) {
+    if (wv == 0) {
+      sums[lane] = sums[64 + lane] = 0.f;
+    }
+    __syncthreads();
+  }
 
   const int nviews = G.nseg * nav;  // view v: segment v / nav, angle v % nav
   for (int c0 = 0; c0 < nviews; c0 += 64) {
@@ -329,12 +350,10 @@ __global__ __launch_bounds__(256, ZB * NV <= 8 ? 5 : 3) void k_back_window(
         }
       }
     };
-    // one view of the chunk, window u
-    auto one_view = [&](int k, int u) {
-      const int fl = lane_of(r_view, k);
-      const float fzb = lane_of(r_fzb, k);
-      const unsigned row = WIN ? 0 : lane_of(r_base, k), clamp = WIN ? 0 : lane_of(r_clamp, k);
-      float yr, au, col, A[ZB], c[ZB + 1];
+    // samples of one view of the chunk, window u
+    auto sample = [&](int k, int u, int fl, float fzb, unsigned row, unsigned clamp, float& yr,
+                      float& au, float& col, float (&A)[ZB]) {
+      float c[ZB + 1];
       column(k, u, fl, yr, au, col);
       const float s0 = fmaf(yr, fzb, fz0);
       if (fl & 1) {
@@ -369,6 +388,13 @@ __global__ __launch_bounds__(256, ZB * NV <= 8 ? 5 : 3) void k_back_window(
           }
         }
       }
+    };
+    auto one_view = [&](int k, int u) {
+      const int fl = lane_of(r_view, k);
+      const float fzb = lane_of(r_fzb, k);
+      const unsigned row = WIN ? 0 : lane_of(r_base, k), clamp = WIN ? 0 : lane_of(r_clamp, k);
+      float yr, au, col, A[ZB];
+      sample(k, u, fl, fzb, row, clamp, yr, au, col, A);
       // a touched sample is below -2^70, the others' sum within 16 * 2^61
       float sum = A[0];
 #pragma unroll
@@ -407,7 +433,7 @@ __global__ __launch_bounds__(256, ZB * NV <= 8 ? 5 : 3) void k_back_window(
         one_view(kc, 0);
         wave_sync();  // the window may be overwritten
       }
-    } else {
+    } else if constexpr (!SPLIT) {
       int kk[NV];
       float4 w[NV];
       int left = __popcll(m);
@@ -465,7 +491,124 @@ __global__ __launch_bounds__(256, ZB * NV <= 8 ? 5 : 3) void k_back_window(
         wave_sync();
         left -= NV;
       }
+    } else {
+      // lane k: the chunk's k-th view that meets the slice
+      const int cnt = __popcll(m);
+      const int below = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
+                                                  __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
+      const int order = __builtin_amdgcn_ds_permute((used ? below : cnt + lane - below) * 4, lane);
+      int kk[NV];
+      float4 w[NV];
+      auto take = [&](int p0) {  // this wave's views of the turn at p0 (the last one past the end)
+#pragma unroll
+        for (int u = 0; u < NV; u++) {
+          kk[u] = lane_of(order, min(p0 + wv * NV + u, cnt - 1));
+          w[u] = fetch(lane_of(r_base, kk[u]), lane_of(r_clamp, kk[u]), 0);
+        }
+      };
+      take(0);
+      for (int p0 = 0; p0 < cnt; p0 += kTurn, turn++) {
+        int kc[NV];
+        bool all = true;
+#pragma unroll
+        for (int u = 0; u < NV; u++) {
+          kc[u] = kk[u];
+          all = all && ((m_shared >> kk[u]) & 1) != 0;
+          *(float4*)(wst + u * wrows * kRowB) = w[u];
+        }
+        if (p0 + kTurn < cnt) take(p0 + kTurn);
+        wave_sync();
+        float A[NV][ZB], sum = 0.f;
+        float yr[NV], au[NV], col[NV];
+        if (all) {
+#pragma unroll
+          for (int u = 0; u < NV; u++) {
+            float c[ZB + 1];
+            column(kc[u], u, lane_of(r_view, kc[u]), yr[u], au[u], col[u]);
+            const float s0 = fmaf(yr[u], lane_of(r_fzb, kc[u]), fz0);
+            const float f0 = floorf(s0);
+            planes(f0, col[u], au[u], 0, 0, c);
+            A[u][0] = lerp1(c[0], c[1], s0 - f0);
+          }
+        } else {
+#pragma unroll
+          for (int u = 0; u < NV; u++)
+            sample(kc[u], u, lane_of(r_view, kc[u]), lane_of(r_fzb, kc[u]), 0, 0, yr[u], au[u],
+                   col[u], A[u]);
+        }
+        const int at = ((turn & 1) * kTurn + wv * NV) * 64 + lane;
+#pragma unroll
+        for (int u = 0; u < NV; u++) {
+          smp[at + u * 64] = A[u][0];
+          sum += A[u][0];
+        }
+        int exact = bad ? (1 << NV) - 1 : 0;
+        if (__builtin_amdgcn_ballot_w64(sum < -0.5f * kTouch) != 0 || bad) {
+#pragma unroll
+          for (int u = 0; u < NV; u++) {
+            const bool few = A[u][0] < -kTouch && A[u][0] > -kDrop;
+            if (__builtin_amdgcn_ballot_w64(few) == 0 && !bad) continue;
+            exact |= 1 << u;
+            const int a = lane_of(r_view, kc[u]) >> 2, si = (c0 + kc[u]) / nav;
+            const SegEntry se = G.seg[si];
+            const unsigned vrow = (unsigned)a * nr + (unsigned)(se.nza + 2 * si + 1 - se.zmin);
+            const int it = subset + a * nsub;
+            const Radial r = radial(G, xv, yv, G.sin_t[it], G.cos_t[it]);
+            float x[ZB] = {0.f}, ct[ZB] = {0.f};
+            if (bad) {
+              exact_view<ZB>(G, rv, rs, se, vrow, r, zb, act, x, ct);
+            } else {
+              const float t = (fmaf(yr[u], se.fzb, fz0) + 0.5f) - 0.5f;
+              const float f = floorf(t);
+              const unsigned o = (vrow + (unsigned)(int)f) * rowb + (unsigned)(r.iq + 1) * 4u;
+              float2 q[2];
+              pairs(f, col[u], 0, 0, q);
+              const float2 e = exact_sample(q[0].x, q[0].y, q[1].x, q[1].y, rs, o, rowb, au[u],
+                                            t - f, few);
+              x[0] = few ? e.x : A[u][0] < 0.f ? 0.f : A[u][0];
+              ct[0] = few ? e.y : A[u][0] < 0.f ? 0.f : 1.f;
+            }
+            smp[at + u * 64] = x[0];
+            cts[at + u * 64] = ct[0];
+          }
+        }
+        rare[(turn & 1) * 4 + wv] = exact << (wv * NV);
+        __syncthreads();
+        if ((turn & 3) == wv) {  // the others take the next turn meanwhile
+          const int nt = min(kTurn, cnt - p0);
+          const float* from = smp + (turn & 1) * kTurn * 64 + lane;
+          n[0] = sums[lane];
+          d[0] = sums[64 + lane];
+          const int4 rw = *(const int4*)(rare + (turn & 1) * 4);
+          const int rm = __builtin_amdgcn_readfirstlane(rw.x | rw.y | rw.z | rw.w);
+          if (rm) {
+            for (int v = 0; v < nt; v++) {
+              if ((rm >> v) & 1) {
+                n[0] += from[v * 64];
+                d[0] += from[(2 * kTurn + v) * 64];
+              } else {
+                const float x[ZB] = {from[v * 64]};
+                add_view(x);
+              }
+            }
+          } else {
+#pragma unroll 4
+            for (int v = 0; v < nt; v++) {
+              const float x[ZB] = {from[v * 64]};
+              add_view(x);
+            }
+          }
+          sums[lane] = n[0];
+          sums[64 + lane] = d[0];
+        }
+      }
     }
+  }
+  if constexpr (SPLIT) {
+    __syncthreads();
+    if (wv != 0) return;
+    n[0] = sums[lane];
+    d[0] = sums[64 + lane];
   }
   if (!act) return;
 #pragma unroll
@@ -492,19 +635,20 @@ int window_rows(const DevGeom& G, int zb) {
   return (int)ceilf(9.9f * G.fzb_absmax + (float)(zb - 1) + 0.01f) + 2;
 }
 
-template <int ZB, int NV, bool WIN>
+template <int ZB, int NV, bool WIN, bool SPLIT>
 hipError_t launch_zb(const DevGeom& G, const BackFrames& F, int nf, int subset, int nsub,
                      const int* dsub, int nav, hipStream_t st) {
   const unsigned nt = (G.res + 7) / 8, ns = (G.nzs + ZB - 1) / ZB;
-  const dim3 grid(nt, nt, (ns + 3) / 4 * nf);
+  const dim3 grid(nt, nt, (SPLIT ? ns : (ns + 3) / 4) * nf);
   const int rows = WIN ? max(16, window_rows(G, ZB)) : 0;
   const int tabf = nav <= kTabAngles ? nav * 192 : 0;
-  const unsigned lds = (unsigned)(tabf + 4 * NV * rows * kWinStride) * 4u;
+  const unsigned split = SPLIT ? 2 * 2 * 4 * NV * 64 + 128 + 8 : 0;
+  const unsigned lds = (unsigned)(tabf + 4 * NV * rows * kWinStride + split) * 4u;
   if (tabf)
-    hipLaunchKernelGGL((k_back_window<ZB, NV, true, WIN>), grid, dim3(256), lds, st, G, F, nf,
+    hipLaunchKernelGGL((k_back_window<ZB, NV, true, WIN, SPLIT>), grid, dim3(256), lds, st, G, F, nf,
                        subset, nsub, dsub, tabf, rows);
   else
-    hipLaunchKernelGGL((k_back_window<ZB, NV, false, WIN>), grid, dim3(256), lds, st, G, F, nf,
+    hipLaunchKernelGGL((k_back_window<ZB, NV, false, WIN, SPLIT>), grid, dim3(256), lds, st, G, F, nf,
                        subset, nsub, dsub, tabf, rows);
   return hipGetLastError();
 }
@@ -517,16 +661,17 @@ bool back_window_fits(const DevGeom& G, int zb) {
 }
 
 // Shape for a geometry that has not been measured. By the number of waves with
-// 8 slices each, against 1024 SIMDs that hold 5 of them (times of one subset,
-// 1-slice / 4 / 8 slices: 256 waves 63 / 88 / 117 us, 640 waves 124 / 145 /
-// 183, 1500 waves 235 / 177 / 257, 2160 waves 412 / 195 / 224, 2880 waves 290 /
-// 118 / 123, 3840 waves 678 / 249 / 310, 5120 waves 1170 / 378 / 299).
+// 8 slices each, against 1024 SIMDs that hold 5 of them (us of one subset with
+// 1 slice split / 1 / 4 / 8 slices: 108 waves 24 / 39 / 56 / 77, 256 waves 44 /
+// 59 / 84 / 121, 576 waves 64 / 52 / 66 / 90, 864 waves 108 / 92 / 76 / 98, 1536
+// waves 117 / 94 / 59 / 77, 3072 waves 442 / 388 / 139 / 150; 4 / 8 slices: 3840
+// waves 249 / 310, 5120 waves 378 / 299).
 static Tune untuned_shape(const DevGeom& G) {
   const int nt = (G.res + 7) / 8, w8 = nt * nt * ((G.nzs + 7) / 8);
   Tune t;
   t.back_lds = 1;
-  t.back_zb = w8 < 1000 ? 1 : w8 < 4500 ? 4 : 8;
-  t.back_ahead = t.back_zb == 1 ? 4 : 1;
+  t.back_zb = w8 < 700 ? 1 : w8 < 4500 ? 4 : 8;
+  t.back_ahead = w8 < 400 ? 2 : w8 < 700 ? 4 : 1;
   if (!back_window_fits(G, t.back_zb)) {  // as many slices as gathers from L1 favour
     t.back_lds = 0;
     t.back_zb = w8 < 4500 ? 2 : 6;
@@ -541,11 +686,12 @@ hipError_t launch_back_packed(const DevGeom& G, const BackFrames& F, int nf, int
   const Tune tune = asked.tuned ? asked : untuned_shape(G);
   if (packed_bytes(G, dsub ? 0 : subset, nsub) >= 0xFFFFFFF0u) return hipErrorInvalidValue;
   const int nav = (G.nang - (dsub ? 0 : subset) + nsub - 1) / nsub;
-#define GFR_BW(ZB, NV, WIN) \
-  return launch_zb<ZB, NV, WIN>(G, F, nf, subset, nsub, dsub, nav, st)
+#define GFR_BS(ZB, NV, WIN, SPLIT) \
+  return launch_zb<ZB, NV, WIN, SPLIT>(G, F, nf, subset, nsub, dsub, nav, st)
+#define GFR_BW(ZB, NV, WIN) GFR_BS(ZB, NV, WIN, false)
   const int zb = tune.back_zb;
   if (zb == 1 && tune.back_ahead > 1 && back_window_fits(G, 1) && window_rows(G, 1) <= 16) {  // NV > 1
-    if (tune.back_ahead == 2) GFR_BW(1, 2, true);
+    if (tune.back_ahead == 2) GFR_BS(1, 2, true, true);
     GFR_BW(1, 4, true);
   }
   if (tune.back_lds && back_window_fits(G, zb)) {
@@ -567,6 +713,7 @@ hipError_t launch_back_packed(const DevGeom& G, const BackFrames& F, int nf, int
     default: GFR_BW(8, 1, false);
   }
 #undef GFR_BW
+#undef GFR_BS
 }
 
 }  // namespace gfr

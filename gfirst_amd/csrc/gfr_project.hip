@@ -915,8 +915,8 @@ hipError_t tune_shapes(const DevGeom& G, int nsub, const FwdOut& fo, const float
   // backprojector: (LDS window, slices, views loaded ahead). One slice and
   // several views ahead: small images, where each wave's walk over the views,
   // not the device's throughput, sets the time.
-  const int bcand[9][3] = {{1, 8, 1}, {1, 4, 1}, {1, 5, 1}, {1, 6, 1}, {1, 16, 1},
-                           {0, 1, 4}, {0, 2, 1}, {0, 4, 1}, {0, 6, 1}};
+  const int bcand[10][3] = {{1, 8, 1}, {1, 4, 1}, {1, 5, 1}, {1, 6, 1}, {1, 16, 1},
+                            {0, 1, 4}, {0, 1, 2}, {0, 2, 1}, {0, 4, 1}, {0, 6, 1}};
   for (const auto& c : bcand) {
     Tune tt = t;
     // the gathering shapes serve what the windows cannot hold
