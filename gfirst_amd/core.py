@@ -125,12 +125,13 @@ class Context:
                    back_bw=4, back_ahead=1):
         """Fix the launch shapes for (geometry, nsub) instead of autotuning them:
         back_zb slices per backprojector thread (1 or 2 with cached reads; 4, 5,
-        6, 8, 16), back_lds the
-        per-block LDS row window, back_waves 6 (8 slices, cached reads) or 0,
-        zsum_sg sinograms per z-sum wave (4, 6, 8), rot_z planes per rotation
-        block (4, 16, 32), back_bw waves per backprojector block (4, or 1 with
-        cached reads and back_waves 0), back_ahead views whose rows are loaded
-        before the first is summed (2 or 4 with one slice and cached reads).
+        6, 8, 16), back_lds the LDS row window of each wave, zsum_sg sinograms per
+        z-sum wave (4, 6, 8; passes small enough take narrow waves instead), rot_z
+        planes per rotation block (4, 16, 32), back_ahead with one slice and
+        cached reads: 4 views at a time per wave, or 2 for each of the four waves
+        that then share the views. back_waves (0, or 6 with 8 slices and cached
+        reads) and back_bw (4, or 1 with cached reads) are accepted and select
+        nothing.
         Applies to sessions created afterwards; no shape changes any result."""
         t = _lib.GfrTuning(back_zb, int(back_lds), back_waves, zsum_sg, rot_z, back_bw, 0.0, 0.0,
                            back_ahead)

@@ -75,11 +75,11 @@ struct Tune {
   int back_zb = 8;   // slices per backprojector thread: 4, 5, 6, 8 or 16
   int zsum_sg = 8;   // consecutive sinograms per z-sum wave: 4, 6 or 8
   int zsum_narrow = -1;  // narrow z-sum waves: 1, 0, or by size (-1)
-  int back_lds = 0;  // 1: backprojector reads its rows through an LDS window
-  int back_waves = 0;     // register budget for this many waves per SIMD (0: compiler's)
+  int back_lds = 0;  // 1: backprojector reads its rows through an LDS window per wave
+  int back_waves = 0;     // kept for the caller, selects nothing
   int rot_z = 16;         // planes per rotation block: 4, 16 or 32
-  int back_bw = 4;        // waves per direct backprojector block: 4 (16x16) or 1 (8x8)
-  int back_ahead = 1;     // 1-slice shapes: views whose rows are loaded ahead (1, 2, 4)
+  int back_bw = 4;        // kept for the caller, selects nothing
+  int back_ahead = 1;     // 1-slice shapes: 4 views at a time per wave, 2: split block
   bool tuned = false;
   float ms_back = 0.f, ms_zsum = 0.f;
 };

@@ -132,17 +132,18 @@ int gfr_zero(gfr_ctx* ctx, void* dptr, size_t bytes, void* stream);
 typedef struct gfr_tuning {
   int back_zb;    /* slices per backprojector thread: 1, 2 (back_lds 0), 4, 5, 6,
                      8 or 16                                                    */
-  int back_lds;   /* 1: per-block LDS window of each view's rows; 0: cached reads */
-  int back_waves; /* 6: 8-slice direct kernel built for 6 waves/SIMD; else 0     */
+  int back_lds;   /* 1: LDS window of each view's rows per wave; 0: cached reads */
+  int back_waves; /* 0, or 6 with 8 slices and back_lds 0: accepted, selects
+                     nothing                                                    */
   int zsum_sg;    /* sinograms per forward z-sum wave: 4, 6 or 8                 */
   int rot_z;      /* planes per forward rotation block: 4, 16 or 32             */
-  int back_bw;    /* waves per backprojector block: 4 (16x16 columns) or 1 (8x8);
-                     1 only with back_lds 0 and back_waves 0                    */
+  int back_bw;    /* 4, or 1 with back_lds 0 and back_waves 0: accepted, selects
+                     nothing (every wave takes 8x8 columns)                     */
   float ms_back;  /* measured time of the chosen backprojector (0 if not measured) */
   float ms_zsum;  /* measured time of the chosen forward projector              */
-  int back_ahead; /* views whose rows are loaded before the first is summed: 1 (or
-                     0), 2 or 4; above 1 only with back_zb 1, back_lds 0 and
-                     back_waves 0                                               */
+  int back_ahead; /* with back_zb 1, back_lds 0 and back_waves 0, through LDS windows:
+                     4: a wave takes 4 views at a time; 2: the 4 waves of a block
+                     share the views, 2 each at a time; else 1 (or 0)           */
 } gfr_tuning;
 /* Returns 1 if the shapes were measured, 0 if defaults. */
 int gfr_tuning_get(gfr_ctx* ctx, const gfr_geometry* g, int nsub, gfr_tuning* t);
