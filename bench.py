@@ -132,25 +132,25 @@ def measured_traffic(dom, back_zb, storage, back_lds, back_bw=4):
 
 
 def measured_pipes(dom, tune):
-    """Busy fractions of the CU's vector-memory units (texture addresser TA,
-    texture data TD) for the backprojector shape in use, from the committed
-    rocprofv3 counter runs; None when no measurement matches."""
+    """VALU issue rate and busy fractions of the CU's LDS and vector-memory units
+    (texture addresser TA, texture data TD) for the backprojector shape in use,
+    from the committed rocprofv3 counter runs; None when no measurement matches."""
     path = os.path.join(ROOT, "profiles", "k_back_c1_pipes.json")
-    if dom != "back" or tune.get("back_lds") or tune.get("back_bw", 4) != 4 or \
-            not os.path.exists(path):
+    if dom != "back" or not tune.get("back_lds") or not os.path.exists(path):
         return None
     with open(path) as f:
         m = json.load(f)
-    e = m.get("by_kernel", {}).get("k_back_direct<%d, %d, float>" % (tune["back_zb"],
-                                                                    tune["back_waves"]))
+    e = m.get("by_kernel", {}).get("k_back_window<%d>" % tune["back_zb"])
     if e is None:
         return None
-    # VALU issue: a CU's four 16-lane SIMDs issue about one wave64 VALU
-    # instruction per cycle between them (4 cycles each)
-    return {"unit": "VALU issue and the vector-memory path (TA address, TD data)",
+    # VALU issue: a CU issues about 1.55 wave64 fma, add or mul instructions a
+    # cycle, and about 0.85 compares, min/max, conversions or instructions with a
+    # scalar operand
+    return {"unit": "VALU issue (mixed full and half rate), beside the windows' loads and LDS",
             "valu_wave_instr_per_cu_cycle": e["valu_wave_instr_per_cu_cycle"],
-            "valu_issue_limit_per_cu_cycle": 1.0, "ta_busy": e["ta_busy"],
-            "td_busy": e["td_busy"], "source": "profiles/k_back_c1_pipes.json"}
+            "valu_issue_limit_per_cu_cycle": 1.55, "lds_busy": e["lds_busy"],
+            "ta_busy": e["ta_busy"], "td_busy": e["td_busy"],
+            "source": "profiles/k_back_c1_pipes.json"}
 
 
 def cpu_baseline(g, d2, norm, pb, nsub, nsteps):
@@ -355,7 +355,7 @@ def run_c1(args):
         # The projectors are interpolation gathers: the binding roofline is the
         # FP32 vector path fed by the CU's vector-memory units (F_alg/t against
         # 157.3 TFLOP/s); the HBM fraction of the same launch is reported beside.
-        "roofline": {"kernel": "k_zsum+k_rotate_tile" if dom == "forward" else "k_back_direct",
+        "roofline": {"kernel": "k_zsum_wide+k_rotate_tile" if dom == "forward" else "k_back_window",
                      "bound": "fp32-valu (vector-memory fed)",
                      "achieved": round(flops, 2), "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(flops / PEAK_FP32_TFLOPS, 4),
@@ -544,7 +544,7 @@ def run_c2(args):
                                    if v[1]},
         # phases of the two chains overlap on the device: a phase's event
         # time includes the other chain's kernels running beside it
-        "roofline": {"kernel": "k_zsum+k_rotate_tile" if dom == "forward" else "k_back_direct",
+        "roofline": {"kernel": "k_zsum_wide+k_rotate_tile" if dom == "forward" else "k_back_window",
                      "bound": "fp32-valu (vector-memory fed)",
                      "achieved": round(flops, 2), "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(flops / PEAK_FP32_TFLOPS, 4), "traffic": None,

@@ -917,8 +917,11 @@ hipError_t tune_shapes(const DevGeom& G, int nsub, const FwdOut& fo, const float
   // not the device's throughput, sets the time.
   const int bcand[10][3] = {{1, 8, 1}, {1, 4, 1}, {1, 5, 1}, {1, 6, 1}, {1, 16, 1},
                             {0, 1, 4}, {0, 1, 2}, {0, 2, 1}, {0, 4, 1}, {0, 6, 1}};
+  const int w8 = ((G.res + 7) / 8) * ((G.res + 7) / 8) * ((G.nzs + 7) / 8);
   for (const auto& c : bcand) {
     Tune tt = t;
+    // one slice only where it can win (3072 waves of 8 slices: 388 us against 139)
+    if (c[2] > 1 && w8 > 2000) continue;
     // the gathering shapes serve what the windows cannot hold
     if (c[2] == 1 && c[0] != (int)back_window_fits(G, c[1])) continue;
     tt.back_lds = c[0];
