@@ -78,8 +78,10 @@ Sizes sizes_of(const GeomHost& h, const gfr_batch_params* p) {
   const size_t sino = store_bytes(p->storage) * (size_t)h.info.ndata;
   z.frame_nobg = z.img + sino;
   z.frame_bg = z.img + 2 * sino;
+  // An upper bound that callers size budgets by: a lane holds 2 + grp images and
+  // grp sets of rows of it.
   const size_t per_lane =
-      (2 + (size_t)grp) * z.img + (size_t)grp * z.rows + z.rot + z.llh;
+      (4 + 2 * (size_t)(grp - 1)) * z.img + (grp > 1 ? 3 : 1) * z.rows + z.rot + z.llh;
   const size_t slots = (size_t)p->max_frames * (3 * sizeof(int) + sizeof(double)) + 256;
   z.shared = (size_t)p->lanes * per_lane + (size_t)h.info.ndata /* mask */ + slots;
   return z;

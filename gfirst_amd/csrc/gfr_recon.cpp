@@ -103,9 +103,9 @@ Plan plan_of(const GeomHost& h, const gfr_recon_params* p, bool bgD, bool bgT) {
            std::min(nav, (size_t)kRotChunk);
   const bool two = p->mode >= 2;
   pl.two = two;
-  // xD num work xb and one more (+ xT jo, and the triples chain's xb num work and
-  // the doubles snapshot)
-  pl.nimg = 5 + (two ? 6 : 0);
+  // xD num work xb (+ xT jo, and the triples chain's xb num work and the doubles
+  // snapshot), and two spare (+ one): an upper bound that callers size budgets by
+  pl.nimg = 6 + (two ? 7 : 0);
   pl.nsino_f32 = p->mode == 3 ? 2 : 0;              // ptc dv (PROJ_BLANK is per geometry)
   pl.nsino_store = 1 + (bgD ? 1 : 0) + (two ? 1 + (bgT ? 1 : 0) : 0);
   return pl;
