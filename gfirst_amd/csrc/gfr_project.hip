@@ -1,4 +1,6 @@
-// gfr_project.hip — the two projectors of the OSEM path on gfx950.
+// gfr_project.hip — the forward projector of the OSEM path on gfx950, the packed
+// rows that the backprojector (gfr_back_window.hip) reads, the FP64 sensitivity
+// and the autotuner of both projectors.
 //
 // Forward projection (FORWPROJ_K, GFIRST_GPU_Kernels.cu:40-102): a LOR of view
 // (segment, angle theta), plane p, radial bin r sums RES+1 trilinear samples of
@@ -7,20 +9,10 @@
 // plane. Trilinear = lerp_z(bilinear_xy(plane z0), bilinear_xy(plane z1)), so
 // the kernel pair below computes every bilinear value once per angle:
 //   k_rotate_tile: R[a][l][z][r] = bilinear_xy(image plane z, x(theta,r,l), y(theta,r,l))
-//   k_zsum       : P(s, r) = sum_l lerp(R[a][l][z0][r], R[a][l][z1][r], alpha_z)
+//   k_zsum_*     : P(s, r) = sum_l lerp(R[a][l][z0][r], R[a][l][z1][r], alpha_z)
 // which is the same arithmetic, operation for operation, as sampling the
 // volume directly (bit-identical results). The z interpolation of sinogram s
-// at sample l, (z0, z1, alpha_z), is a per-geometry table, so a sample costs
-// two coalesced buffer loads with scalar offsets and one lerp.
-//
-// Backprojection (BACKWPROJ_K, GFIRST_GPU_Kernels.cu:109-164): one thread
-// per voxel column and ZB consecutive slices, views in the reference's order
-// (segment-major, angle-minor, GFIRST.cu:439-465). Per view the radial
-// interpolation (r0, r1, alpha_u) is shared by the thread's slices; the
-// ZB+1 planes its slices need are fetched together (one memory round trip
-// per view, row addresses without tests thanks to the padded packed rows)
-// and radially interpolated once each. Each slice keeps its own exactly
-// computed plane index and weight, as the reference's per-voxel sampling.
+// at sample l, (z0, z1, alpha_z), is a per-geometry table.
 #include "gfr_device.h"
 
 namespace gfr {
@@ -256,12 +248,15 @@ __device__ __forceinline__ void block_llh(double ll, double* part) {
 // Wide waves: one wave per (64 quads of bins, group of SG planes of a segment).
 // Its lanes are consecutive (angle, 4 bins) items, so a row load is one 16-byte
 // access per lane and a wave is full whatever the bin count; the SG LORs of a
-// lane share SG + 1 rows. The waves of an angle walk the samples together and
-// are the first to touch a sample's rows, so a load waits for memory and not
-// for L2: the rows of the next sample are requested before the current one is
-// summed. Row and weights of a sample are wave-uniform (scalar loads, further
-// ahead). Samples whose LORs do not blend consecutive rows (at the volume's
-// ends) load each LOR's two rows.
+// lane share SG + 1 rows. Row and weights of a sample are wave-uniform (scalar
+// loads, one sample ahead). The four waves of a block take the same planes of
+// four neighbouring segments, which blend nearly the same rows, so L1 serves
+// three of them. Groups whose LORs do not blend consecutive rows in every
+// sample (at the volume's ends) load each LOR's two rows.
+// What bounds it: the vector-memory path (16 cycles a row load) and the L2
+// misses of the rotation. 10 angles of 4319 x 128 LORs with ratio: 190 -> 145 us,
+// 16 angles of 1293 x 147: 150 -> 130 us (waves of two angles, half empty at 147
+// bins, with scalar table reads per LOR before).
 template <int S, bool RATIO, bool LLH, int SG>
 __global__ __launch_bounds__(256) void k_zsum_wide(DevGeom G, const float* __restrict__ R,
                                                    unsigned r_bytes, FwdArgs o, int subset,
