@@ -41,6 +41,7 @@ struct Lane {
   float* rows[kMaxGroup] = {};           // per frame of a group: packed rows,
   float* num[kMaxGroup] = {};            // update ratio
   double* llh_part = nullptr;
+  int llh_cap = 0;
   size_t r_floats = 0;
 };
 
@@ -63,6 +64,7 @@ int group_of(const gfr_batch_params* p) { return p->group == 0 ? kMaxGroup : p->
 
 struct Sizes {
   size_t img, rows, rot, llh, frame_nobg, frame_bg, shared;
+  int llh_cap;  // doubles
 };
 
 Sizes sizes_of(const GeomHost& h, const gfr_batch_params* p) {
@@ -74,14 +76,17 @@ Sizes sizes_of(const GeomHost& h, const gfr_batch_params* p) {
   const int grp = group_of(p);
   z.rot = sizeof(float) * (size_t)(h.info.lambda1 - h.info.lambda0 + 1) * h.g.nzs * h.g.nrad *
           std::min(nav, (size_t)kRotChunk);
-  z.llh = sizeof(double) * (size_t)llh_capacity(h, p->min_nsub) + 64;
+  z.llh_cap = llh_capacity(h, p->min_nsub);
+  z.llh = sizeof(double) * (size_t)z.llh_cap + 64;
   const size_t sino = store_bytes(p->storage) * (size_t)h.info.ndata;
   z.frame_nobg = z.img + sino;
   z.frame_bg = z.img + 2 * sino;
-  // An upper bound that callers size budgets by: a lane holds 2 + grp images and
-  // grp sets of rows of it.
+  // Callers size budgets by the first figure: it stays where it was while what a
+  // lane holds (the second) is no more.
   const size_t per_lane =
-      (4 + 2 * (size_t)(grp - 1)) * z.img + (grp > 1 ? 3 : 1) * z.rows + z.rot + z.llh;
+      z.rot + std::max((4 + 2 * (size_t)(grp - 1)) * z.img + (grp > 1 ? 3 : 1) * z.rows +
+                           llh_bound_bytes(h, p->min_nsub),
+                       (2 + (size_t)grp) * z.img + (size_t)grp * z.rows + z.llh);
   const size_t slots = (size_t)p->max_frames * (3 * sizeof(int) + sizeof(double)) + 256;
   z.shared = (size_t)p->lanes * per_lane + (size_t)h.info.ndata /* mask */ + slots;
   return z;
@@ -145,6 +150,7 @@ hipError_t enqueue_forward(gfr_batch* b, int f, const Lane& L, const PackedRows&
   fo.storage = b->p.storage;
   fo.yscale = (float)b->g.res;
   fo.llh_part = L.llh_part;
+  fo.llh_cap = L.llh_cap;
   if (e == hipSuccess)
     e = launch_forward(G, L.xb, L.R, L.r_floats, fo, 0, fr.nsub, dsub, fr.tune, L.st);
   if (e == hipSuccess)
@@ -352,6 +358,7 @@ int gfr_batch_create(gfr_ctx* ctx, const gfr_geometry* g, const gfr_batch_params
     for (int i = 0; i < group_of(p) && ok; i++)
       ok = A((void**)&L.rows[i], z.rows) && A((void**)&L.num[i], z.img);
     L.r_floats = z.rot / sizeof(float);
+    L.llh_cap = z.llh_cap;
   }
   if (!ok) return bfail(b, set_err(ctx, GFR_ENOMEM, "batch allocation failed"));
   // Shared calibration mask from the projection of the unblurred uniform
@@ -476,6 +483,7 @@ int gfr_batch_add(gfr_batch* b, int niter, int nsub, const float* prompts, const
     fo.storage = b->p.storage;
     fo.yscale = (float)b->g.res;
     fo.llh_part = L.llh_part;
+    fo.llh_cap = L.llh_cap;
     e = tune_shapes(G, nsub, fo, fr.x, L.R, L.r_floats, L.num[0], st, &t);
     if (e != hipSuccess) return undo(hip_err(ctx, e, "gfr_batch_add tuning"));
     std::lock_guard<std::mutex> lk(ctx->mu);

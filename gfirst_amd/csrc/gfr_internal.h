@@ -224,7 +224,8 @@ struct FwdOut {
   const void* bg = nullptr;       // background or NULL
   int storage = GFR_STORE_F32;
   float yscale = 1.f;             // RES
-  double* llh_part = nullptr;     // llh_capacity() doubles, or NULL
+  double* llh_part = nullptr;     // llh_cap doubles (llh_capacity()), or NULL
+  int llh_cap = 0;
 };
 // Scratch of the rotation stage: floats per angle; the launcher processes the
 // subset's angles in chunks of r_cap_floats / rotate_floats_per_angle().
@@ -291,9 +292,33 @@ hipError_t launch_advance(int* sub, const int* nsub, const int* slots, int n, hi
 hipError_t launch_poisson(const float* mean, double scale, const float* mean2, double scale2,
                           uint64_t seed, float* out, long long n, hipStream_t st);
 
-// Largest number of FP64 partials a forward pass with `nsub` subsets writes
-// (any tile shape).
+// What a forward pass launches, from the geometry's counts alone. The launcher,
+// the sum of the log-likelihood partials and the size of their buffer all take
+// it from zsum_plan.
+struct ZsumDims {
+  int nsinogs, nrad, nang;
+  int ngroups[3];  // z-sum groups of 4, 6 and 8 planes
+  size_t per;      // rotate_floats_per_angle()
+};
+struct ZsumPlan {
+  int kind;    // sinograms per z-sum wave, 0: narrow waves; one for all subsets
+  int chunk;   // angles per rotation chunk (0: not even one fits)
+  int ngb;     // blocks along the sinograms
+  int blocks;  // blocks (= log-likelihood partials) of the pass
+};
+ZsumDims zsum_dims(const GeomHost& h);
+ZsumPlan zsum_plan(const ZsumDims& d, const Tune& tune, int subset, int nsub, size_t r_cap_floats);
+// Largest number of FP64 partials that a forward pass of `nsub` or more subsets
+// writes (any tile shape) with rotation scratch for min(angles, kRotChunk)
+// angles of the longest subset.
 int llh_capacity(const GeomHost& h, int nsub);
+// What footprints count for the partials where the rest of their bound covers
+// the difference: a fixed figure per geometry and subset count.
+inline size_t llh_bound_bytes(const GeomHost& h, int nsub) {
+  const size_t nav = (size_t)(h.g.nang + nsub - 1) / nsub;
+  return sizeof(double) * (((size_t)h.g.nrad + 127) / 128) *
+             (((size_t)h.info.nsinogs + 15) / 16) * ((nav + 1) / 2) + 64;
+}
 // Times each tile shape of the two projectors on the given buffers (subset 0)
 // and returns the fastest; any shape gives identical results.
 hipError_t tune_shapes(const DevGeom& G, int nsub, const FwdOut& fo, const float* img, float* R,

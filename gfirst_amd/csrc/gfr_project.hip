@@ -13,6 +13,8 @@
 // which is the same arithmetic, operation for operation, as sampling the
 // volume directly (bit-identical results). The z interpolation of sinogram s
 // at sample l, (z0, z1, alpha_z), is a per-geometry table.
+#include <algorithm>
+
 #include "gfr_device.h"
 
 namespace gfr {
@@ -659,50 +661,64 @@ __host__ __device__ inline int zsum_nib(bool wide, int nrad, int na) {
   return (na * (wide ? (nrad + 3) / 4 : nrad) + 63) / 64;
 }
 
-// Blocks (partials) of a pass over nav angles in chunks of kRotChunk.
-inline int zsum_blocks(bool wide, int ngroups, int nsinogs, int nrad, int nav) {
-  return zsum_ngb(wide, ngroups, nsinogs) *
-         (nav / kRotChunk * zsum_nib(wide, nrad, kRotChunk) + zsum_nib(wide, nrad, nav % kRotChunk));
+// Blocks of a pass over nav angles in chunks.
+inline int zsum_blocks(bool wide, int ngb, int nrad, int nav, int chunk) {
+  return ngb * (nav / chunk * zsum_nib(wide, nrad, chunk) + zsum_nib(wide, nrad, nav % chunk));
 }
 // The narrow kernel serves passes up to this many of its blocks (measured,
 // narrow / best wide, us of a whole projection: 368 blocks 26 / 60, 750 40 / 79,
 // 1472 53 / 66, 2016 89 / 98, 2466 104 / 107, 2745 94 / 85, 4575 141 / 98).
 constexpr int kNarrowBlocks = 2400;
 
-// Which kernel a pass over nav angles takes: sinograms per wave, or 0 for the
-// narrow one. Where no measurement says: the narrow one where it serves, 4
-// sinograms where 6 leave too few waves (3.3M LORs a pass 150 us with 4, 163
-// with 6; 4.8M 202 and 170).
-int zsum_kind(const DevGeom& G, const Tune& tune, int nav) {
-  const bool fits = zsum_blocks(false, 0, G.nsinogs, G.nrad, nav) <= kNarrowBlocks;
+// Which kernel the passes of a subset count take: sinograms per wave, or 0 for
+// the narrow one. The longest subset (nav angles) decides for all of them.
+// Where no measurement says: the narrow one where it serves, 4 sinograms where 6
+// leave too few waves (3.3M LORs a pass 150 us with 4, 163 with 6; 4.8M 202 and
+// 170).
+int zsum_kind(const ZsumDims& d, const Tune& tune, int nav) {
+  const bool fits =
+      zsum_blocks(false, zsum_ngb(false, 0, d.nsinogs), d.nrad, nav, kRotChunk) <= kNarrowBlocks;
   if (fits && tune.zsum_narrow != 0) return 0;
   if (tune.tuned) return tune.zsum_sg;
-  return (long long)G.nsinogs * nav * G.nrad < 3800000 ? 4 : 6;
+  return (long long)d.nsinogs * nav * d.nrad < 3800000 ? 4 : 6;
 }
 
-// Angles per rotation chunk for nav angles.
-int forward_chunk(const DevGeom& G, int nav, size_t r_cap_floats) {
-  const size_t per = rotate_floats_per_angle(G);
-  size_t chunk = r_cap_floats / per;
-  if (chunk > (size_t)nav) chunk = nav;
-  if (chunk * per * sizeof(float) >= 0xFFFFFFF0u) chunk = 0xFFFFFFF0u / (per * 4);
-  return (int)chunk;
+}  // namespace
+
+ZsumDims zsum_dims(const GeomHost& h) {
+  return {h.info.nsinogs, h.g.nrad, h.g.nang,
+          {(int)h.zgrp[0].size(), (int)h.zgrp[1].size(), (int)h.zgrp[2].size()},
+          (size_t)(h.info.lambda1 - h.info.lambda0 + 1) * h.g.nzs * h.g.nrad};
 }
 
-int zsum_ngb_of(const DevGeom& G, int kind) {
-  return zsum_ngb(kind != 0, kind ? G.zg[zg_index(kind)].n : 0, G.nsinogs);
+ZsumPlan zsum_plan(const ZsumDims& d, const Tune& tune, int subset, int nsub,
+                   size_t r_cap_floats) {
+  const int nav = (d.nang - subset + nsub - 1) / nsub;
+  ZsumPlan p{};
+  p.kind = zsum_kind(d, tune, (d.nang + nsub - 1) / nsub);
+  size_t chunk = std::min(r_cap_floats / d.per, (size_t)nav);
+  if (chunk * d.per * sizeof(float) >= 0xFFFFFFF0u) chunk = 0xFFFFFFF0u / (d.per * sizeof(float));
+  p.chunk = (int)chunk;
+  p.ngb = zsum_ngb(p.kind != 0, p.kind ? d.ngroups[zg_index(p.kind)] : 0, d.nsinogs);
+  if (p.chunk > 0) p.blocks = zsum_blocks(p.kind != 0, p.ngb, d.nrad, nav, p.chunk);
+  return p;
 }
 
-hipError_t zsum_launch(const DevGeom& G, int kind, const float* R, unsigned rbytes,
+namespace {
+
+ZsumDims zsum_dims(const DevGeom& G) {
+  return {G.nsinogs, G.nrad, G.nang, {G.zg[0].n, G.zg[1].n, G.zg[2].n}, rotate_floats_per_angle(G)};
+}
+
+hipError_t zsum_launch(const DevGeom& G, const ZsumPlan& zp, const float* R, unsigned rbytes,
                        const FwdArgs& o, bool ratio, int storage, int subset, int nsub,
                        const int* dsub, int a0, int na, int nl, unsigned llh_off, hipStream_t st) {
-  const unsigned blocks =
-      (unsigned)zsum_ngb_of(G, kind) * (unsigned)zsum_nib(kind != 0, G.nrad, na);
+  const unsigned blocks = (unsigned)zp.ngb * (unsigned)zsum_nib(zp.kind != 0, G.nrad, na);
 #define GFR_ZK(K)                                                                             \
   hipLaunchKernelGGL(K, dim3(blocks), dim3(256), 0, st, G, R, rbytes, o, subset, nsub, dsub, \
                      a0, na, nl, llh_off)
 #define GFR_ZL(S, RT, LL)                                      \
-  switch (kind) {                                              \
+  switch (zp.kind) {                                           \
     case 0: GFR_ZK((k_zsum_narrow<S, RT, LL>)); break;         \
     case 4: GFR_ZK((k_zsum_wide<S, RT, LL, 4>)); break;        \
     case 6: GFR_ZK((k_zsum_wide<S, RT, LL, 6>)); break;        \
@@ -759,11 +775,11 @@ hipError_t launch_forward(const DevGeom& G, const float* img, float* R, size_t r
   const int nav = dsub ? nav_of(G, 0, nsub) : nav_of(G, subset, nsub);
   const int nl = G.l1 - G.l0 + 1;
   const size_t per = rotate_floats_per_angle(G);
-  const int chunk = forward_chunk(G, nav, r_cap_floats);
-  if (chunk < 1) return hipErrorInvalidValue;
-  const int kind = zsum_kind(G, tune, nav);
+  const ZsumPlan zp = zsum_plan(zsum_dims(G), tune, dsub ? 0 : subset, nsub, r_cap_floats);
+  const int chunk = zp.chunk;
+  if (chunk < 1 || (out.llh_part && zp.blocks > out.llh_cap)) return hipErrorInvalidValue;
   const unsigned llh_per_chunk =
-      (unsigned)zsum_ngb_of(G, kind) * (unsigned)zsum_nib(kind != 0, G.nrad, chunk);
+      (unsigned)zp.ngb * (unsigned)zsum_nib(zp.kind != 0, G.nrad, chunk);
   FwdArgs o{out.proj, out.corr,  out.rows,   out.mask,
             out.y,    out.bg,    out.yscale, out.llh_part};
   const bool ratio = out.corr || out.rows.v;
@@ -781,7 +797,7 @@ hipError_t launch_forward(const DevGeom& G, const float* img, float* R, size_t r
     const unsigned lds = (unsigned)(side * (side | 1) * sizeof(float2));
     // planes per block: 16, or 4 where that alone makes enough blocks (16 angles
     // at 64x64x32: the rotation 14 us with 16, 8 with 4; 64 angles: no difference)
-    const int rz = tune.tuned ? tune.rot_z : kind == 0 ? 4 : 16;
+    const int rz = tune.tuned ? tune.rot_z : zp.kind == 0 ? 4 : 16;
 #define GFR_RT(ZC)                                                                                \
   hipLaunchKernelGGL(k_rotate_tile<ZC>, dim3(gxy * ((G.nzs + ZC - 1) / ZC)), dim3(256), lds, st, G, \
                      img, R, subset, nsub, dsub, a0, nl, zouter, side)
@@ -791,7 +807,7 @@ hipError_t launch_forward(const DevGeom& G, const float* img, float* R, size_t r
 #undef GFR_RT
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    e = zsum_launch(G, kind, R, rbytes, o, ratio, out.storage, subset, nsub, dsub, a0, na, nl,
+    e = zsum_launch(G, zp, R, rbytes, o, ratio, out.storage, subset, nsub, dsub, a0, na, nl,
                     llh_per_chunk * (unsigned)(a0 / chunk), st);
     if (e != hipSuccess) return e;
   }
@@ -801,12 +817,10 @@ hipError_t launch_forward(const DevGeom& G, const float* img, float* R, size_t r
 hipError_t launch_llh_sum(const DevGeom& G, const double* part, int subset, int nsub,
                           const int* dsub, size_t r_cap_floats, const Tune& tune, double* out,
                           hipStream_t st) {
-  const int nav = nav_of(G, dsub ? 0 : subset, nsub);
-  const int chunk = forward_chunk(G, nav, r_cap_floats);
-  if (chunk < 1) return hipErrorInvalidValue;
-  const int kind = zsum_kind(G, tune, nav);
-  hipLaunchKernelGGL(k_llh_sum, dim3(1), dim3(256), 0, st, part, kind != 0, zsum_ngb_of(G, kind),
-                     G.nrad, chunk, G.nang, subset, nsub, dsub, out);
+  const ZsumPlan zp = zsum_plan(zsum_dims(G), tune, dsub ? 0 : subset, nsub, r_cap_floats);
+  if (zp.chunk < 1) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_llh_sum, dim3(1), dim3(256), 0, st, part, zp.kind != 0, zp.ngb, G.nrad,
+                     zp.chunk, G.nang, subset, nsub, dsub, out);
   return hipGetLastError();
 }
 
@@ -843,12 +857,21 @@ hipError_t launch_sensitivity(const DevGeom& G, const uint8_t* mask, float2* c2,
 }
 
 int llh_capacity(const GeomHost& h, int nsub) {
-  const int nav = (h.g.nang + nsub - 1) / nsub;
-  const int wide = zsum_blocks(true, (int)h.zgrp[0].size(), h.info.nsinogs, h.g.nrad, nav);
-  const int narrow = zsum_blocks(false, 0, h.info.nsinogs, h.g.nrad, nav);
-  int most = ((h.g.nrad + 127) / 128) * ((h.info.nsinogs + 15) / 16) * ((nav + 1) / 2);
-  if (wide > most) most = wide;
-  if (narrow <= kNarrowBlocks && narrow > most) most = narrow;
+  const ZsumDims d = zsum_dims(h);
+  const size_t r_cap = d.per * std::min((d.nang + nsub - 1) / nsub, kRotChunk);
+  int most = 0, last = 0;
+  for (int n = nsub; n <= d.nang; n++) {
+    const int nav = (d.nang + n - 1) / n;
+    if (nav == last) continue;  // the same passes
+    last = nav;
+    for (int sg : {4, 6, 8, 0}) {  // 0: narrow waves, where they serve
+      Tune t;
+      t.tuned = true;
+      t.zsum_narrow = sg == 0;
+      if (sg) t.zsum_sg = sg;
+      most = std::max(most, zsum_plan(d, t, 0, n, r_cap).blocks);
+    }
+  }
   return most;
 }
 

@@ -45,6 +45,7 @@ struct gfr_recon {
   uint8_t* mask = nullptr;
   gfr_vlor* vl = nullptr;
   double* llh_part = nullptr;
+  int llh_cap = 0;
   double* d_llh = nullptr;
   unsigned int* d_maxbits = nullptr;  // 16 words: [0] image maximum, [8 + chain] PackedRows::bad
   int llh_valid = 0;
@@ -78,8 +79,9 @@ namespace {
 size_t store_bytes(int storage) { return storage == GFR_STORE_F32 ? 4 : 2; }
 
 struct Plan {
-  size_t img, sino_f32, sino_store, mask, llh, rows, rot;
-  int nimg, nsino_f32, nsino_store;
+  size_t img, sino_f32, sino_store, mask, llh, llh_bound, rows, rot;
+  int llh_cap;  // doubles
+  int nimg, nimg_bound, nsino_f32, nsino_store;
   bool two;  // second (triples) chain
 };
 
@@ -95,7 +97,9 @@ Plan plan_of(const GeomHost& h, const gfr_recon_params* p, bool bgD, bool bgT) {
   pl.sino_f32 = sizeof(float) * (size_t)h.info.ndata;
   pl.sino_store = store_bytes(p->storage) * (size_t)h.info.ndata;
   pl.mask = (size_t)h.info.ndata;
-  pl.llh = sizeof(double) * (size_t)llh_capacity(h, p->nsub) + 64;
+  pl.llh_cap = llh_capacity(h, p->nsub);
+  pl.llh = sizeof(double) * (size_t)pl.llh_cap + 64;
+  pl.llh_bound = llh_bound_bytes(h, p->nsub);
   const size_t nav = (size_t)(h.g.nang + p->nsub - 1) / p->nsub;
   pl.rows = 2 * sizeof(float) * nav * ((size_t)h.info.nsinogs + 2 * (size_t)h.g.nseg) *
              ((size_t)h.g.nrad + 2);  // packed rows: NRAD + 2 entries
@@ -104,16 +108,22 @@ Plan plan_of(const GeomHost& h, const gfr_recon_params* p, bool bgD, bool bgT) {
   const bool two = p->mode >= 2;
   pl.two = two;
   // xD num work xb (+ xT jo, and the triples chain's xb num work and the doubles
-  // snapshot), and two spare (+ one): an upper bound that callers size budgets by
-  pl.nimg = 6 + (two ? 7 : 0);
+  // snapshot)
+  pl.nimg = 4 + (two ? 6 : 0);
+  pl.nimg_bound = 6 + (two ? 7 : 0);
   pl.nsino_f32 = p->mode == 3 ? 2 : 0;              // ptc dv (PROJ_BLANK is per geometry)
   pl.nsino_store = 1 + (bgD ? 1 : 0) + (two ? 1 + (bgT ? 1 : 0) : 0);
   return pl;
 }
 
+// Callers size budgets by the bound: it stays where it was while what a session
+// holds is no more.
 size_t plan_bytes(const Plan& pl) {
-  return pl.nimg * pl.img + pl.nsino_f32 * pl.sino_f32 + pl.nsino_store * pl.sino_store +
-         pl.mask + (pl.two ? 2 : 1) * (pl.llh + pl.rows + pl.rot);
+  const size_t sino =
+      pl.nsino_f32 * pl.sino_f32 + pl.nsino_store * pl.sino_store + pl.mask;
+  const size_t chains = pl.two ? 2 : 1;
+  return sino + std::max(pl.nimg_bound * pl.img + chains * (pl.llh_bound + pl.rows + pl.rot),
+                         pl.nimg * pl.img + chains * (pl.llh + pl.rows + pl.rot));
 }
 
 hipEvent_t take_event(gfr_recon* r) {
@@ -181,6 +191,7 @@ hipError_t autotune(gfr_recon* r) {
   fo.storage = r->p.storage;
   fo.yscale = (float)r->g.res;
   fo.llh_part = r->llh_part;
+  fo.llh_cap = r->llh_cap;
   Tune t;
   hipError_t e = tune_shapes(gd->dev, S, fo, r->xb, r->R, r->r_floats, r->num, r->st, &t);
   if (e != hipSuccess) return e;
@@ -345,6 +356,7 @@ int gfr_recon_create(gfr_ctx* ctx, const gfr_geometry* g, const gfr_recon_params
   hipStream_t st = r->st;
   const DevGeom& G = gd->dev;
   r->r_floats = pl.rot / sizeof(float);
+  r->llh_cap = pl.llh_cap;
   hipError_t e = hipSuccess;
   // Host arrays reach the device through a transient staging buffer; arrays in
   // this device's memory are read where they are.
@@ -493,6 +505,7 @@ int gfr_recon_step(gfr_recon* r) {
       fo.storage = p.storage;
       fo.yscale = (float)r->g.res;
       fo.llh_part = llh_part;
+      fo.llh_cap = r->llh_cap;
       GFR_HIP(ctx, launch_forward(G, xb, R, r->r_floats, fo, s, S, nullptr, r->tune, st));
     }
     GFR_HIP(ctx, launch_llh_sum(G, llh_part, s, S, nullptr, r->r_floats, r->tune, d_llh, st));
