@@ -637,10 +637,9 @@ int window_rows(const DevGeom& G, int zb) {
 
 template <int ZB, int NV, bool WIN, bool SPLIT>
 hipError_t launch_zb(const DevGeom& G, const BackFrames& F, int nf, int subset, int nsub,
-                     const int* dsub, int nav, hipStream_t st) {
+                     const int* dsub, int nav, int rows, hipStream_t st) {
   const unsigned nt = (G.res + 7) / 8, ns = (G.nzs + ZB - 1) / ZB;
   const dim3 grid(nt, nt, (SPLIT ? ns : (ns + 3) / 4) * nf);
-  const int rows = WIN ? max(16, window_rows(G, ZB)) : 0;
   const int tabf = nav <= kTabAngles ? nav * 192 : 0;
   const unsigned split = SPLIT ? 2 * 2 * 4 * NV * 64 + 128 + 8 : 0;
   const unsigned lds = (unsigned)(tabf + 4 * NV * rows * kWinStride + split) * 4u;
@@ -660,58 +659,78 @@ bool back_window_fits(const DevGeom& G, int zb) {
   return 9.9f * G.fxb + 2.01f <= 15.f && window_rows(G, zb) <= kWinRows;
 }
 
+// Several views at a time: their windows take one load of 16 rows each.
+static bool one_slice_fits(const DevGeom& G) {
+  return back_window_fits(G, 1) && window_rows(G, 1) <= 16;
+}
+
 // Shape for a geometry that has not been measured. By the number of waves with
 // 8 slices each, against 1024 SIMDs that hold 5 of them (us of one subset with
 // 1 slice split / 1 / 4 / 8 slices: 108 waves 24 / 39 / 56 / 77, 256 waves 44 /
 // 59 / 84 / 121, 576 waves 64 / 52 / 66 / 90, 864 waves 108 / 92 / 76 / 98, 1536
 // waves 117 / 94 / 59 / 77, 3072 waves 442 / 388 / 139 / 150; 4 / 8 slices: 3840
 // waves 249 / 310, 5120 waves 378 / 299).
+// Where windows do not fit, as many slices as gathers from L1 favour; where one
+// slice's window takes more than 16 rows, one slice gathers too (1 slice / 4 of
+// the window kernel: 192 waves 92 / 104, 576 waves 97 / 108; 2 slices gathering
+// 107 in both).
 static Tune untuned_shape(const DevGeom& G) {
   const int nt = (G.res + 7) / 8, w8 = nt * nt * ((G.nzs + 7) / 8);
   Tune t;
   t.back_lds = 1;
   t.back_zb = w8 < 700 ? 1 : w8 < 4500 ? 4 : 8;
   t.back_ahead = w8 < 400 ? 2 : w8 < 700 ? 4 : 1;
-  if (!back_window_fits(G, t.back_zb)) {  // as many slices as gathers from L1 favour
+  if (t.back_zb == 1 ? !one_slice_fits(G) : !back_window_fits(G, t.back_zb)) {
     t.back_lds = 0;
-    t.back_zb = w8 < 4500 ? 2 : 6;
+    t.back_zb = w8 < 700 ? 1 : w8 < 4500 ? 2 : 6;
     t.back_ahead = 1;
   }
   return t;
 }
 
+BackShape back_shape(const DevGeom& G, const Tune& asked) {
+  const Tune t = asked.tuned ? asked : untuned_shape(G);
+  const bool one = t.back_zb == 1 && t.back_ahead > 1 && one_slice_fits(G);
+  BackShape b{};
+  b.zb = t.back_zb;
+  b.win = one || (t.back_zb >= 4 && t.back_lds && back_window_fits(G, t.back_zb));
+  b.split = one && t.back_ahead == 2;
+  b.nv = b.split ? 2 : one ? 4 : 1;
+  b.rows = b.win ? max(16, window_rows(G, b.zb)) : 0;
+  return b;
+}
+
 hipError_t launch_back_packed(const DevGeom& G, const BackFrames& F, int nf, int subset, int nsub,
-                              const int* dsub, const Tune& asked, hipStream_t st) {
+                              const int* dsub, const Tune& tune, hipStream_t st) {
   if (nf < 1 || nf > kMaxGroup) return hipErrorInvalidValue;
-  const Tune tune = asked.tuned ? asked : untuned_shape(G);
   if (packed_bytes(G, dsub ? 0 : subset, nsub) >= 0xFFFFFFF0u) return hipErrorInvalidValue;
   const int nav = (G.nang - (dsub ? 0 : subset) + nsub - 1) / nsub;
+  const BackShape b = back_shape(G, tune);
 #define GFR_BS(ZB, NV, WIN, SPLIT) \
-  return launch_zb<ZB, NV, WIN, SPLIT>(G, F, nf, subset, nsub, dsub, nav, st)
+  return launch_zb<ZB, NV, WIN, SPLIT>(G, F, nf, subset, nsub, dsub, nav, b.rows, st)
 #define GFR_BW(ZB, NV, WIN) GFR_BS(ZB, NV, WIN, false)
-  const int zb = tune.back_zb;
-  if (zb == 1 && tune.back_ahead > 1 && back_window_fits(G, 1) && window_rows(G, 1) <= 16) {  // NV > 1
-    if (tune.back_ahead == 2) GFR_BS(1, 2, true, true);
-    GFR_BW(1, 4, true);
-  }
-  if (tune.back_lds && back_window_fits(G, zb)) {
-    switch (zb) {
+  if (b.split) GFR_BS(1, 2, true, true);
+  if (b.nv == 4) GFR_BW(1, 4, true);
+  if (b.win) {
+    switch (b.zb) {
       case 4: GFR_BW(4, 1, true);
       case 5: GFR_BW(5, 1, true);
       case 6: GFR_BW(6, 1, true);
+      case 8: GFR_BW(8, 1, true);
       case 16: GFR_BW(16, 1, true);
-      default: GFR_BW(8, 1, true);
     }
+    return hipErrorInvalidValue;
   }
-  switch (zb) {
+  switch (b.zb) {
     case 1: GFR_BW(1, 1, false);
     case 2: GFR_BW(2, 1, false);
     case 4: GFR_BW(4, 1, false);
     case 5: GFR_BW(5, 1, false);
     case 6: GFR_BW(6, 1, false);
+    case 8: GFR_BW(8, 1, false);
     case 16: GFR_BW(16, 1, false);
-    default: GFR_BW(8, 1, false);
   }
+  return hipErrorInvalidValue;
 #undef GFR_BW
 #undef GFR_BS
 }

@@ -249,6 +249,14 @@ hipError_t launch_back_packed(const DevGeom& G, const BackFrames& F, int nf, int
                               const int* dsub, const Tune& tune, hipStream_t st);
 // Whether a wave's window of zb slices holds every read of a tile.
 bool back_window_fits(const DevGeom& G, int zb);
+// The backprojector that a geometry and a tuning lead to: slices per wave, views
+// at a time, through windows of `rows` rows or gathering, a block's waves sharing
+// the views or not.
+struct BackShape {
+  int zb, nv, rows;
+  bool win, split;
+};
+BackShape back_shape(const DevGeom& G, const Tune& tune);
 // Sensitivity of a subset: the backprojector's denominator half in FP64
 // ({1, calib} pairs, packed_bytes of scratch, so only calibration gaps apply).
 hipError_t launch_sensitivity(const DevGeom& G, const uint8_t* mask, float2* c2, double* sens,
