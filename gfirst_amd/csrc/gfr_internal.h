@@ -34,6 +34,10 @@ struct ZGroups {
 };
 constexpr uint32_t kZReg = 1u << 31;
 inline __host__ __device__ int zg_index(int sg) { return sg == 4 ? 0 : sg == 6 ? 1 : 2; }
+// Row k of a sample that the n LORs of a group blend, counted from the group's
+// first: they need 0 .. n, and a group of fewer than SG LORs takes the last one
+// again instead of rows past the volume's end.
+inline __host__ __device__ int zg_row(int k, int n) { return k < n ? k : n; }
 
 // Geometry as the kernels see it (by value). Pointers are device tables owned
 // by the context, built once per distinct geometry.

@@ -299,6 +299,9 @@ __global__ __launch_bounds__(256) void k_zsum_wide(DevGeom G, const float* __res
     unsigned soff = 0;
     if (grp.y > 0) {
       float e[SG];
+      unsigned roff[SG + 1];
+#pragma unroll
+      for (int k = 0; k <= SG; k++) roff[k] = (unsigned)zg_row(k, ng) * rowb;
       uint32_t z = rows[0];
 #pragma unroll
       for (int i = 0; i < SG; i++) e[i] = wts[i];
@@ -306,7 +309,7 @@ __global__ __launch_bounds__(256) void k_zsum_wide(DevGeom G, const float* __res
         const unsigned base = soff + (z & ~kZReg) * rowb;
         float4 row[SG + 1];
 #pragma unroll
-        for (int k = 0; k <= SG; k++) row[k] = ld_f4(rr, voff, base + (unsigned)k * rowb);
+        for (int k = 0; k <= SG; k++) row[k] = ld_f4(rr, voff, base + roff[k]);
         float en[SG];
         if (li + 1 < nl) {  // the next sample's, while the rows come
           rows += zg.n;
