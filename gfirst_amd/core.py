@@ -126,7 +126,7 @@ class Context:
         """Fix the launch shapes for (geometry, nsub) instead of autotuning them:
         back_zb slices per backprojector thread (1 or 2 with cached reads; 4, 5,
         6, 8, 16), back_lds the LDS row window of each wave, zsum_sg sinograms per
-        z-sum wave (4, 6, 8; passes small enough take narrow waves instead), rot_z
+        z-sum wave (4, 6, 8, or 2: narrow waves, for passes small enough), rot_z
         planes per rotation block (4, 16, 32), back_ahead with one slice and
         cached reads: 4 views at a time per wave, or 2 for each of the four waves
         that then share the views. back_waves (0, or 6 with 8 slices and cached

@@ -673,9 +673,11 @@ int gfr_tuning_set(gfr_ctx* ctx, const gfr_geometry* g, int nsub, const gfr_tuni
   if (nsub < 1 || nsub > g->nang) return set_err(ctx, GFR_EINVAL, "nsub out of range");
   const int zb = in->back_zb, sg = in->zsum_sg;
   if (!(zb == 1 || zb == 2 || zb == 4 || zb == 5 || zb == 6 || zb == 8 || zb == 16) ||
-      !(sg == 4 || sg == 6 || sg == 8))
+      !(sg == kZsumNarrow || sg == 4 || sg == 6 || sg == 8))
     return set_err(ctx, GFR_EINVAL,
-                   "back_zb must be 1, 2, 4, 5, 6, 8 or 16 and zsum_sg 4, 6 or 8");
+                   "back_zb must be 1, 2, 4, 5, 6, 8 or 16 and zsum_sg 2, 4, 6 or 8");
+  if (sg == kZsumNarrow && !zsum_narrow_serves(zsum_dims(gd->host), nsub))
+    return set_err(ctx, GFR_EINVAL, "zsum_sg 2: the passes are too large for narrow waves");
   if (in->back_lds != 0 && in->back_lds != 1)
     return set_err(ctx, GFR_EINVAL, "back_lds must be 0 or 1");
   if (zb < 4 && in->back_lds)
@@ -697,7 +699,6 @@ int gfr_tuning_set(gfr_ctx* ctx, const gfr_geometry* g, int nsub, const gfr_tuni
   t.back_lds = in->back_lds;
   t.back_waves = in->back_waves;
   t.zsum_sg = in->zsum_sg;
-  t.zsum_narrow = -1;
   t.rot_z = in->rot_z;
   t.back_bw = in->back_bw;
   t.back_ahead = ahead;

@@ -73,12 +73,13 @@ struct PackedRows {
   unsigned* bad;
 };
 
+constexpr int kZsumNarrow = 2;  // two sinograms: the narrow z-sum waves
+
 // Tile shapes of the projectors (chosen per geometry and subset count by the
 // autotuner; none of them changes any summation order).
 struct Tune {
   int back_zb = 8;   // slices per backprojector thread: 4, 5, 6, 8 or 16
-  int zsum_sg = 8;   // consecutive sinograms per z-sum wave: 4, 6 or 8
-  int zsum_narrow = -1;  // narrow z-sum waves: 1, 0, or by size (-1)
+  int zsum_sg = 8;   // consecutive sinograms per z-sum wave: 4, 6 or 8, kZsumNarrow
   int back_lds = 0;  // 1: backprojector reads its rows through an LDS window per wave
   int back_waves = 0;     // kept for the caller, selects nothing
   int rot_z = 16;         // planes per rotation block: 4, 16 or 32
@@ -313,12 +314,14 @@ struct ZsumDims {
   size_t per;      // rotate_floats_per_angle()
 };
 struct ZsumPlan {
-  int kind;    // sinograms per z-sum wave, 0: narrow waves; one for all subsets
+  int kind;    // sinograms per z-sum wave, one for all subsets
   int chunk;   // angles per rotation chunk (0: not even one fits)
   int ngb;     // blocks along the sinograms
   int blocks;  // blocks (= log-likelihood partials) of the pass
 };
 ZsumDims zsum_dims(const GeomHost& h);
+// Whether passes of nsub subsets are small enough for the narrow waves.
+bool zsum_narrow_serves(const ZsumDims& d, int nsub);
 ZsumPlan zsum_plan(const ZsumDims& d, const Tune& tune, int subset, int nsub, size_t r_cap_floats);
 // Largest number of FP64 partials that a forward pass of `nsub` or more subsets
 // writes (any tile shape) with rotation scratch for min(angles, kRotChunk)

@@ -673,20 +673,23 @@ inline int zsum_blocks(bool wide, int ngb, int nrad, int nav, int chunk) {
 // 1472 53 / 66, 2016 89 / 98, 2466 104 / 107, 2745 94 / 85, 4575 141 / 98).
 constexpr int kNarrowBlocks = 2400;
 
-// Which kernel the passes of a subset count take: sinograms per wave, or 0 for
-// the narrow one. The longest subset (nav angles) decides for all of them.
-// Where no measurement says: the narrow one where it serves, 4 sinograms where 6
-// leave too few waves (3.3M LORs a pass 150 us with 4, 163 with 6; 4.8M 202 and
-// 170).
-int zsum_kind(const ZsumDims& d, const Tune& tune, int nav) {
-  const bool fits =
-      zsum_blocks(false, zsum_ngb(false, 0, d.nsinogs), d.nrad, nav, kRotChunk) <= kNarrowBlocks;
-  if (fits && tune.zsum_narrow != 0) return 0;
-  if (tune.tuned) return tune.zsum_sg;
-  return (long long)d.nsinogs * nav * d.nrad < 3800000 ? 4 : 6;
+}  // namespace
+
+bool zsum_narrow_serves(const ZsumDims& d, int nsub) {
+  const int nav = (d.nang + nsub - 1) / nsub;
+  return zsum_blocks(false, zsum_ngb(false, 0, d.nsinogs), d.nrad, nav, kRotChunk) <= kNarrowBlocks;
 }
 
-}  // namespace
+// Sinograms per wave for the passes of a subset count. The longest subset
+// decides for all of them. Where no measurement says: narrow waves where they
+// serve, 4 sinograms where 6 leave too few waves (3.3M LORs a pass 150 us with 4,
+// 163 with 6; 4.8M 202 and 170).
+static int zsum_kind(const ZsumDims& d, const Tune& tune, int nsub) {
+  if (tune.tuned) return tune.zsum_sg;
+  if (zsum_narrow_serves(d, nsub)) return kZsumNarrow;
+  const int nav = (d.nang + nsub - 1) / nsub;
+  return (long long)d.nsinogs * nav * d.nrad < 3800000 ? 4 : 6;
+}
 
 ZsumDims zsum_dims(const GeomHost& h) {
   return {h.info.nsinogs, h.g.nrad, h.g.nang,
@@ -698,12 +701,13 @@ ZsumPlan zsum_plan(const ZsumDims& d, const Tune& tune, int subset, int nsub,
                    size_t r_cap_floats) {
   const int nav = (d.nang - subset + nsub - 1) / nsub;
   ZsumPlan p{};
-  p.kind = zsum_kind(d, tune, (d.nang + nsub - 1) / nsub);
+  p.kind = zsum_kind(d, tune, nsub);
+  const bool wide = p.kind != kZsumNarrow;
   size_t chunk = std::min(r_cap_floats / d.per, (size_t)nav);
   if (chunk * d.per * sizeof(float) >= 0xFFFFFFF0u) chunk = 0xFFFFFFF0u / (d.per * sizeof(float));
   p.chunk = (int)chunk;
-  p.ngb = zsum_ngb(p.kind != 0, p.kind ? d.ngroups[zg_index(p.kind)] : 0, d.nsinogs);
-  if (p.chunk > 0) p.blocks = zsum_blocks(p.kind != 0, p.ngb, d.nrad, nav, p.chunk);
+  p.ngb = zsum_ngb(wide, d.ngroups[zg_index(p.kind)], d.nsinogs);
+  if (p.chunk > 0) p.blocks = zsum_blocks(wide, p.ngb, d.nrad, nav, p.chunk);
   return p;
 }
 
@@ -716,13 +720,13 @@ ZsumDims zsum_dims(const DevGeom& G) {
 hipError_t zsum_launch(const DevGeom& G, const ZsumPlan& zp, const float* R, unsigned rbytes,
                        const FwdArgs& o, bool ratio, int storage, int subset, int nsub,
                        const int* dsub, int a0, int na, int nl, unsigned llh_off, hipStream_t st) {
-  const unsigned blocks = (unsigned)zp.ngb * (unsigned)zsum_nib(zp.kind != 0, G.nrad, na);
+  const unsigned blocks = (unsigned)zp.ngb * (unsigned)zsum_nib(zp.kind != kZsumNarrow, G.nrad, na);
 #define GFR_ZK(K)                                                                             \
   hipLaunchKernelGGL(K, dim3(blocks), dim3(256), 0, st, G, R, rbytes, o, subset, nsub, dsub, \
                      a0, na, nl, llh_off)
 #define GFR_ZL(S, RT, LL)                                      \
   switch (zp.kind) {                                           \
-    case 0: GFR_ZK((k_zsum_narrow<S, RT, LL>)); break;         \
+    case kZsumNarrow: GFR_ZK((k_zsum_narrow<S, RT, LL>)); break; \
     case 4: GFR_ZK((k_zsum_wide<S, RT, LL, 4>)); break;        \
     case 6: GFR_ZK((k_zsum_wide<S, RT, LL, 6>)); break;        \
     default: GFR_ZK((k_zsum_wide<S, RT, LL, 8>)); break;       \
@@ -782,7 +786,7 @@ hipError_t launch_forward(const DevGeom& G, const float* img, float* R, size_t r
   const int chunk = zp.chunk;
   if (chunk < 1 || (out.llh_part && zp.blocks > out.llh_cap)) return hipErrorInvalidValue;
   const unsigned llh_per_chunk =
-      (unsigned)zp.ngb * (unsigned)zsum_nib(zp.kind != 0, G.nrad, chunk);
+      (unsigned)zp.ngb * (unsigned)zsum_nib(zp.kind != kZsumNarrow, G.nrad, chunk);
   FwdArgs o{out.proj, out.corr,  out.rows,   out.mask,
             out.y,    out.bg,    out.yscale, out.llh_part};
   const bool ratio = out.corr || out.rows.v;
@@ -800,7 +804,7 @@ hipError_t launch_forward(const DevGeom& G, const float* img, float* R, size_t r
     const unsigned lds = (unsigned)(side * (side | 1) * sizeof(float2));
     // planes per block: 16, or 4 where that alone makes enough blocks (16 angles
     // at 64x64x32: the rotation 14 us with 16, 8 with 4; 64 angles: no difference)
-    const int rz = tune.tuned ? tune.rot_z : zp.kind == 0 ? 4 : 16;
+    const int rz = tune.tuned ? tune.rot_z : zp.kind == kZsumNarrow ? 4 : 16;
 #define GFR_RT(ZC)                                                                                \
   hipLaunchKernelGGL(k_rotate_tile<ZC>, dim3(gxy * ((G.nzs + ZC - 1) / ZC)), dim3(256), lds, st, G, \
                      img, R, subset, nsub, dsub, a0, nl, zouter, side)
@@ -822,7 +826,7 @@ hipError_t launch_llh_sum(const DevGeom& G, const double* part, int subset, int 
                           hipStream_t st) {
   const ZsumPlan zp = zsum_plan(zsum_dims(G), tune, dsub ? 0 : subset, nsub, r_cap_floats);
   if (zp.chunk < 1) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_llh_sum, dim3(1), dim3(256), 0, st, part, zp.kind != 0, zp.ngb, G.nrad,
+  hipLaunchKernelGGL(k_llh_sum, dim3(1), dim3(256), 0, st, part, zp.kind != kZsumNarrow, zp.ngb, G.nrad,
                      zp.chunk, G.nang, subset, nsub, dsub, out);
   return hipGetLastError();
 }
@@ -867,11 +871,11 @@ int llh_capacity(const GeomHost& h, int nsub) {
     const int nav = (d.nang + n - 1) / n;
     if (nav == last) continue;  // the same passes
     last = nav;
-    for (int sg : {4, 6, 8, 0}) {  // 0: narrow waves, where they serve
+    for (int sg : {kZsumNarrow, 4, 6, 8}) {
+      if (sg == kZsumNarrow && !zsum_narrow_serves(d, n)) continue;
       Tune t;
       t.tuned = true;
-      t.zsum_narrow = sg == 0;
-      if (sg) t.zsum_sg = sg;
+      t.zsum_sg = sg;
       most = std::max(most, zsum_plan(d, t, 0, n, r_cap).blocks);
     }
   }
@@ -906,19 +910,18 @@ hipError_t tune_shapes(const DevGeom& G, int nsub, const FwdOut& fo, const float
   };
   Tune t;
   t.tuned = true;
-  const int cand[4] = {4, 6, 8, 0};  // 0: narrow waves
+  const int cand[4] = {4, 6, 8, kZsumNarrow};
   float bz = 1e30f, bb = 1e30f;
   for (int c : cand) {
+    if (c == kZsumNarrow && !zsum_narrow_serves(zsum_dims(G), nsub)) continue;
     Tune tt = t;
-    tt.zsum_narrow = c == 0;
-    if (c) tt.zsum_sg = c;
+    tt.zsum_sg = c;
     const float ms = time_it([&] {
       return launch_forward(G, img, R, r_floats, fo, 0, nsub, nullptr, tt, st);
     });
     if (ms < bz) {
       bz = ms;
       t.zsum_sg = tt.zsum_sg;
-      t.zsum_narrow = tt.zsum_narrow;
     }
   }
   const int rcand[3] = {4, 16, 32};  // planes per rotation block

@@ -135,7 +135,8 @@ typedef struct gfr_tuning {
   int back_lds;   /* 1: LDS window of each view's rows per wave; 0: cached reads */
   int back_waves; /* 0, or 6 with 8 slices and back_lds 0: accepted, selects
                      nothing                                                    */
-  int zsum_sg;    /* sinograms per forward z-sum wave: 4, 6 or 8                 */
+  int zsum_sg;    /* sinograms per forward z-sum wave: 4, 6 or 8, or 2: narrow
+                     waves, for passes small enough (others are refused)        */
   int rot_z;      /* planes per forward rotation block: 4, 16 or 32             */
   int back_bw;    /* 4, or 1 with back_lds 0 and back_waves 0: accepted, selects
                      nothing (every wave takes 8x8 columns)                     */

@@ -17,7 +17,7 @@ long long passes = 0, narrow_short = 0, cut = 0, bad = 0;
 // End of the partials that the launches of one pass write: chunks of plan.chunk
 // angles, each at a whole number of full chunks' blocks.
 long long written(const ZsumDims& d, const ZsumPlan& p, int nav) {
-  const bool wide = p.kind != 0;
+  const bool wide = p.kind != kZsumNarrow;
   const long long ngb = wide ? (d.ngroups[zg_index(p.kind)] + 3) / 4 : (d.nsinogs + 7) / 8;
   auto blocks = [&](int na) {
     const long long items = (long long)na * (wide ? (d.nrad + 3) / 4 : d.nrad);
@@ -36,21 +36,22 @@ void walk(const gfr_geometry& g, int made) {
   const ZsumDims d = zsum_dims(h);
   const int cap = llh_capacity(h, made);
   const size_t r_cap = d.per * std::min((g.nang + made - 1) / made, kRotChunk);
-  Tune shapes[6];
-  for (int k = 0; k < 5; k++) {
+  Tune shapes[5];
+  for (int k = 0; k < 4; k++) {
     shapes[k].tuned = true;
-    shapes[k].zsum_sg = k < 3 ? 4 + 2 * k : 8;
-    shapes[k].zsum_narrow = k < 3 ? 0 : k == 3 ? 1 : -1;
+    shapes[k].zsum_sg = k < 3 ? 4 + 2 * k : kZsumNarrow;
   }
   for (const Tune& t : shapes) {  // the last one: not measured
     for (int nsub : {made, made + 1, made + 3, 2 * made, 3 * made}) {
       if (nsub > g.nang) continue;
+      // refused by gfr_tuning_set, and not a candidate of the tuner
+      if (t.tuned && t.zsum_sg == kZsumNarrow && !zsum_narrow_serves(d, nsub)) continue;
       const int longest = zsum_plan(d, t, 0, nsub, r_cap).kind;
       for (int s : {0, nsub / 2, nsub - 1}) {
         const int nav = (g.nang - s + nsub - 1) / nsub;
         const ZsumPlan p = zsum_plan(d, t, s, nsub, r_cap);
         passes++;
-        narrow_short += p.kind == 0 && nav < (g.nang + nsub - 1) / nsub;
+        narrow_short += p.kind == kZsumNarrow && nav < (g.nang + nsub - 1) / nsub;
         cut += p.chunk < std::min(nav, kRotChunk);
         if (p.chunk < 1) continue;  // refused by the launcher
         const long long n = written(d, p, nav);
