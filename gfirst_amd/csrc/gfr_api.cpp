@@ -653,7 +653,8 @@ int gfr_tuning_get(gfr_ctx* ctx, const gfr_geometry* g, int nsub, gfr_tuning* ou
   GFR_GEOM(ctx, g, gd);
   GFR_NONNULL(ctx, out, "tuning");
   if (nsub < 1 || nsub > g->nang) return set_err(ctx, GFR_EINVAL, "nsub out of range");
-  const Tune t = tune_for(ctx, gd, nsub);
+  Tune t = tune_for(ctx, gd, nsub);
+  if (!t.tuned) t = untuned_tune(gd->dev, nsub);
   out->back_zb = t.back_zb;
   out->back_lds = t.back_lds;
   out->back_waves = t.back_waves;

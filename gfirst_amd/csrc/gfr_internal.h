@@ -334,6 +334,9 @@ inline size_t llh_bound_bytes(const GeomHost& h, int nsub) {
   return sizeof(double) * (((size_t)h.g.nrad + 127) / 128) *
              (((size_t)h.info.nsinogs + 15) / 16) * ((nav + 1) / 2) + 64;
 }
+// The shapes that launches take without a tuning, as gfr_tuning_set would name
+// them.
+Tune untuned_tune(const DevGeom& G, int nsub);
 // Times each tile shape of the two projectors on the given buffers (subset 0)
 // and returns the fastest; any shape gives identical results.
 hipError_t tune_shapes(const DevGeom& G, int nsub, const FwdOut& fo, const float* img, float* R,

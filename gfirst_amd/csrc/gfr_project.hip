@@ -775,6 +775,22 @@ __global__ void k_llh_sum(const double* __restrict__ part, int wide, int ngb, in
 
 }  // namespace
 
+// Planes per rotation block: 16, or 4 where that alone makes enough blocks (16
+// angles at 64x64x32: the rotation 14 us with 16, 8 with 4; 64 angles: no
+// difference)
+static int untuned_rot_z(int kind) { return kind == kZsumNarrow ? 4 : 16; }
+
+Tune untuned_tune(const DevGeom& G, int nsub) {
+  const BackShape b = back_shape(G, Tune());
+  Tune t;
+  t.zsum_sg = zsum_kind(zsum_dims(G), t, nsub);
+  t.rot_z = untuned_rot_z(t.zsum_sg);
+  t.back_zb = b.zb;
+  t.back_lds = b.win && b.zb > 1;  // one slice: back_ahead says how it reads
+  t.back_ahead = b.split ? 2 : b.nv;
+  return t;
+}
+
 hipError_t launch_forward(const DevGeom& G, const float* img, float* R, size_t r_cap_floats,
                           const FwdOut& out, int subset, int nsub, const int* dsub,
                           const Tune& tune, hipStream_t st) {
@@ -802,9 +818,7 @@ hipError_t launch_forward(const DevGeom& G, const float* img, float* R, size_t r
     const float diag = sqrtf(31.f * G.fxf * 31.f * G.fxf + (float)((tl - 1) * (tl - 1)));
     const int side = min(kRotTile, min((int)diag + 4, G.res));
     const unsigned lds = (unsigned)(side * (side | 1) * sizeof(float2));
-    // planes per block: 16, or 4 where that alone makes enough blocks (16 angles
-    // at 64x64x32: the rotation 14 us with 16, 8 with 4; 64 angles: no difference)
-    const int rz = tune.tuned ? tune.rot_z : zp.kind == kZsumNarrow ? 4 : 16;
+    const int rz = tune.tuned ? tune.rot_z : untuned_rot_z(zp.kind);
 #define GFR_RT(ZC)                                                                                \
   hipLaunchKernelGGL(k_rotate_tile<ZC>, dim3(gxy * ((G.nzs + ZC - 1) / ZC)), dim3(256), lds, st, G, \
                      img, R, subset, nsub, dsub, a0, nl, zouter, side)

@@ -146,7 +146,7 @@ typedef struct gfr_tuning {
                      4: a wave takes 4 views at a time; 2: the 4 waves of a block
                      share the views, 2 each at a time; else 1 (or 0)           */
 } gfr_tuning;
-/* Returns 1 if the shapes were measured, 0 if defaults. */
+/* The shapes in force. Returns 1 if they were measured or set, 0 if chosen by size. */
 int gfr_tuning_get(gfr_ctx* ctx, const gfr_geometry* g, int nsub, gfr_tuning* t);
 int gfr_tuning_set(gfr_ctx* ctx, const gfr_geometry* g, int nsub, const gfr_tuning* t);
 
