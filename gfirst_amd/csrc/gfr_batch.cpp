@@ -37,7 +37,6 @@ struct Lane {
   hipStream_t st = nullptr;
   hipEvent_t join = nullptr;
   float *xb = nullptr, *work = nullptr, *R = nullptr;
-  unsigned* bad = nullptr;               // PackedRows::bad
   float* rows[kMaxGroup] = {};           // per frame of a group: packed rows,
   float* num[kMaxGroup] = {};            // update ratio
   double* llh_part = nullptr;
@@ -81,14 +80,16 @@ Sizes sizes_of(const GeomHost& h, const gfr_batch_params* p) {
   const size_t sino = store_bytes(p->storage) * (size_t)h.info.ndata;
   z.frame_nobg = z.img + sino;
   z.frame_bg = z.img + 2 * sino;
-  // Callers size budgets by the first figure: it stays where it was while what a
-  // lane holds (the second) is no more.
-  const size_t per_lane =
-      z.rot + std::max((4 + 2 * (size_t)(grp - 1)) * z.img + (grp > 1 ? 3 : 1) * z.rows +
-                           llh_bound_bytes(h, p->min_nsub),
-                       (2 + (size_t)grp) * z.img + (size_t)grp * z.rows + z.llh);
-  const size_t slots = (size_t)p->max_frames * (3 * sizeof(int) + sizeof(double)) + 256;
-  z.shared = (size_t)p->lanes * per_lane + (size_t)h.info.ndata /* mask */ + slots;
+  // Callers size budgets by the bound: it stays where it was while what a batch
+  // holds is no more.
+  const size_t lanes = (size_t)p->lanes, slots = (size_t)p->max_frames;
+  const size_t per_slot = 3 * sizeof(int) + sizeof(double);
+  const size_t bound = lanes * ((4 + 2 * (size_t)(grp - 1)) * z.img + (grp > 1 ? 3 : 1) * z.rows +
+                                z.rot + llh_bound_bytes(h, p->min_nsub)) +
+                       slots * per_slot + 256;
+  const size_t held = lanes * ((2 + (size_t)grp) * z.img + (size_t)grp * z.rows + z.rot + z.llh) +
+                      slots * (per_slot + sizeof(unsigned));
+  z.shared = (size_t)h.info.ndata /* mask */ + std::max(bound, held);
   return z;
 }
 
@@ -107,7 +108,7 @@ struct gfr_batch {
   int* d_sub = nullptr;     // [max_frames] subset index per slot
   int* d_nsub = nullptr;    // [max_frames]
   int* d_slots = nullptr;   // [max_frames] active slots of the current graph
-  unsigned* d_bad = nullptr;  // [lanes] PackedRows::bad
+  unsigned* d_bad = nullptr;  // [max_frames] PackedRows::bad per slot, zero between steps
   double* d_llh = nullptr;  // [max_frames] FP64 log-likelihood of the last pass
   std::vector<void*> owned;
   size_t bytes = 0;
@@ -175,7 +176,7 @@ hipError_t enqueue_group(gfr_batch* b, const std::vector<int>& grp, const Lane& 
   BackFrames F{};
   hipError_t e = hipSuccess;
   for (size_t i = 0; i < grp.size() && e == hipSuccess; i++) {
-    F.rows[i] = packed_rows(G, L.rows[i], 0, f0.nsub, L.bad, 1);
+    F.rows[i] = packed_rows(G, L.rows[i], 0, f0.nsub, b->d_bad + grp[i], 1);
     F.numer[i] = L.num[i];
     e = enqueue_forward(b, grp[i], L, F.rows[i]);
   }
@@ -241,7 +242,7 @@ hipError_t enqueue_step(gfr_batch* b) {
     if (e == hipSuccess) e = hipStreamWaitEvent(b->st, L.join, 0);
   }
   if (e == hipSuccess)
-    e = launch_advance(b->d_sub, b->d_nsub, b->d_slots, (int)b->active.size(), b->st);
+    e = launch_advance(b->d_sub, b->d_nsub, b->d_slots, b->d_bad, (int)b->active.size(), b->st);
   return e;
 }
 
@@ -345,12 +346,12 @@ int gfr_batch_create(gfr_ctx* ctx, const gfr_geometry* g, const gfr_batch_params
             A((void**)&b->d_sub, sizeof(int) * p->max_frames) &&
             A((void**)&b->d_nsub, sizeof(int) * p->max_frames) &&
             A((void**)&b->d_slots, sizeof(int) * p->max_frames) &&
-            A((void**)&b->d_llh, sizeof(double) * p->max_frames) && A((void**)&b->d_bad, 64) &&
-            launch_zero(b->d_bad, 64, b->st) == hipSuccess;
+            A((void**)&b->d_llh, sizeof(double) * p->max_frames) &&
+            A((void**)&b->d_bad, sizeof(unsigned) * p->max_frames) &&
+            launch_zero(b->d_bad, sizeof(unsigned) * p->max_frames, b->st) == hipSuccess;
   b->lanes.resize(p->lanes);
   for (Lane& L : b->lanes) {
     if (!ok) break;
-    L.bad = b->d_bad + (&L - b->lanes.data());  // at most 16 lanes
     ok = hipStreamCreateWithFlags(&L.st, hipStreamNonBlocking) == hipSuccess &&
          hipEventCreateWithFlags(&L.join, hipEventDisableTiming) == hipSuccess &&
          A((void**)&L.xb, z.img) && A((void**)&L.work, z.img) && A((void**)&L.R, z.rot) &&
@@ -476,7 +477,7 @@ int gfr_batch_add(gfr_batch* b, int niter, int nsub, const float* prompts, const
   if (!t.tuned && !(env && env[0] == '0')) {
     Lane& L = b->lanes[0];
     FwdOut fo;
-    fo.rows = packed_rows(G, L.rows[0], 0, nsub, L.bad, 1);
+    fo.rows = packed_rows(G, L.rows[0], 0, nsub, b->d_bad + f, 1);
     fo.mask = b->mask;
     fo.y = fr.y;
     fo.bg = fr.bg;
@@ -485,6 +486,7 @@ int gfr_batch_add(gfr_batch* b, int niter, int nsub, const float* prompts, const
     fo.llh_part = L.llh_part;
     fo.llh_cap = L.llh_cap;
     e = tune_shapes(G, nsub, fo, fr.x, L.R, L.r_floats, L.num[0], st, &t);
+    if (e == hipSuccess) e = launch_zero(b->d_bad + f, sizeof(unsigned), st);
     if (e != hipSuccess) return undo(hip_err(ctx, e, "gfr_batch_add tuning"));
     std::lock_guard<std::mutex> lk(ctx->mu);
     b->gd->tune[nsub] = t;

@@ -299,8 +299,10 @@ hipError_t launch_any_positive(const float* v, long long n, unsigned int* flag, 
 // must start at 0).
 hipError_t launch_store_checked(const float* in, void* out, int storage, long long n,
                                 unsigned int* flag, hipStream_t st);
-// sub[slots[i]] = (sub[slots[i]] + 1) mod nsub[slots[i]] for i < n.
-hipError_t launch_advance(int* sub, const int* nsub, const int* slots, int n, hipStream_t st);
+// sub[slots[i]] = (sub[slots[i]] + 1) mod nsub[slots[i]] and bad[slots[i]] = 0
+// for i < n.
+hipError_t launch_advance(int* sub, const int* nsub, const int* slots, unsigned* bad, int n,
+                          hipStream_t st);
 // Synthetic measurements (gfr_synth.hip).
 hipError_t launch_poisson(const float* mean, double scale, const float* mean2, double scale2,
                           uint64_t seed, float* out, long long n, hipStream_t st);

@@ -678,14 +678,17 @@ hipError_t launch_fill_cylinder(const DevGeom& G, float val, float* img, hipStre
 }
 
 namespace {
-// Advances the subset index of each listed slot: sub = (sub + 1) mod nsub.
+// Advances the subset index of each listed slot: sub = (sub + 1) mod nsub, and
+// clears the flag of its packed rows (PackedRows::bad), so that ratios out of
+// range slow down the frame's one pass only.
 __global__ void k_advance(int* __restrict__ sub, const int* __restrict__ nsub,
-                          const int* __restrict__ slots, int n) {
+                          const int* __restrict__ slots, unsigned* __restrict__ bad, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const int s = slots[i];
   const int v = sub[s] + 1;
   sub[s] = v >= nsub[s] ? 0 : v;
+  bad[s] = 0u;
 }
 }  // namespace
 
@@ -711,9 +714,10 @@ hipError_t launch_any_positive(const float* v, long long n, unsigned int* flag, 
   return hipGetLastError();
 }
 
-hipError_t launch_advance(int* sub, const int* nsub, const int* slots, int n, hipStream_t st) {
+hipError_t launch_advance(int* sub, const int* nsub, const int* slots, unsigned* bad, int n,
+                          hipStream_t st) {
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_advance, dim3((n + 255) / 256), dim3(256), 0, st, sub, nsub, slots, n);
+  hipLaunchKernelGGL(k_advance, dim3((n + 255) / 256), dim3(256), 0, st, sub, nsub, slots, bad, n);
   return hipGetLastError();
 }
 

@@ -59,6 +59,7 @@ struct gfr_recon {
   hipEvent_t ev_tfree = nullptr;  // an iteration's triples passes are done with it
   hipEvent_t ev_join = nullptr;
   bool tfree_pending = false;
+  unsigned pack_epoch = 0;  // of the last pass's packed rows (the flag words start at 0)
   int llh_chain = 0;  // chain of the last pass's log-likelihood (0 doubles, 1 triples)
   std::vector<std::pair<void*, size_t>> owned;  // blocks from dev_alloc
   size_t bytes = 0;
@@ -184,7 +185,7 @@ hipError_t autotune(gfr_recon* r) {
     return hipSuccess;
   }
   FwdOut fo;
-  fo.rows = packed_rows(gd->dev, r->rows, 0, S, r->d_maxbits + 8, 1);
+  fo.rows = packed_rows(gd->dev, r->rows, 0, S, r->d_maxbits + 8, ++r->pack_epoch);
   fo.mask = r->mask;
   fo.y = r->yD;
   fo.bg = r->bD;
@@ -452,7 +453,9 @@ int gfr_recon_step(gfr_recon* r) {
   float* x = tc ? r->xT : r->xD;
   float* xb = tc ? r->xbT : r->xb;
   float* R = tc ? r->RT : r->R;
-  const PackedRows rows = packed_rows(G, tc ? r->rowsT : r->rows, s, S, r->d_maxbits + 8 + (tc ? 1 : 0), 1);
+  // an epoch of its own: ratios out of range slow down this pass only
+  const PackedRows rows = packed_rows(G, tc ? r->rowsT : r->rows, s, S,
+                                      r->d_maxbits + 8 + (tc ? 1 : 0), ++r->pack_epoch);
   float* num = tc ? r->numT : r->num;
   float* work = tc ? r->workT : r->work;
   double* llh_part = tc ? r->llh_partT : r->llh_part;
