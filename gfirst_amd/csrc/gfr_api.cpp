@@ -127,31 +127,22 @@ GeomDev* geom_for(gfr_ctx* ctx, const gfr_geometry* g) {
     total = (total + bytes + 15) & ~size_t(15);
     return at;
   };
-  const size_t off_za = place(h.za.size() * sizeof(float));
   size_t off_zg[3], off_zr[3];
-  for (int k = 0; k < 3; k++) {
-    off_zg[k] = place(h.zgrp[k].size() * sizeof(int2));
-    off_zr[k] = place(h.zrow[k].size() * sizeof(uint32_t));
-  }
-  std::vector<char> blob(total, 0);
+  for (int k = 0; k < 3; k++) off_zg[k] = place(h.zgrp[k].size() * sizeof(int2));
+  const size_t upload = total;  // the rest follows from these on the device
+  const size_t n_samp = (size_t)(h.info.lambda1 - h.info.lambda0 + 1);
+  const size_t off_za = place((n_samp * n_sino + kZPad) * sizeof(float));
+  for (int k = 0; k < 3; k++) off_zr[k] = place(n_samp * h.zgrp[k].size() * sizeof(uint32_t));
+  std::vector<char> blob(upload, 0);
   memcpy(blob.data(), h.sin_t.data(), n_ang * sizeof(float));
   memcpy(blob.data() + off_cos, h.cos_t.data(), n_ang * sizeof(float));
   memcpy(blob.data() + off_seg, h.seg.data(), n_seg * sizeof(SegEntry));
   memcpy(blob.data() + off_sino, h.sino.data(), n_sino * sizeof(int2));
   memcpy(blob.data() + off_zt, h.ztab.data(), h.ztab.size() * sizeof(uint2));
-  memcpy(blob.data() + off_za, h.za.data(), h.za.size() * sizeof(float));
-  for (int k = 0; k < 3; k++) {
+  for (int k = 0; k < 3; k++)
     memcpy(blob.data() + off_zg[k], h.zgrp[k].data(), h.zgrp[k].size() * sizeof(int2));
-    memcpy(blob.data() + off_zr[k], h.zrow[k].data(), h.zrow[k].size() * sizeof(uint32_t));
-  }
   hipError_t e = hipMalloc(&gd->block, total);
-  if (e == hipSuccess) e = hipMemcpy(gd->block, blob.data(), total, hipMemcpyHostToDevice);
-  if (e != hipSuccess) {
-    hip_err(ctx, e, "geometry tables");
-    if (gd->block) (void)hipFree(gd->block);
-    delete gd;
-    return nullptr;
-  }
+  if (e == hipSuccess) e = hipMemcpy(gd->block, blob.data(), upload, hipMemcpyHostToDevice);
   DevGeom& d = gd->dev;
   d.res = g->res;
   d.nzs = g->nzs;
@@ -176,10 +167,21 @@ GeomDev* geom_for(gfr_ctx* ctx, const gfr_geometry* g) {
   d.sino = (const int2*)(base + off_sino);
   d.ztab = (const uint2*)(base + off_zt);
   d.za = (const float*)(base + off_za);
+  int2* group[3];
+  uint32_t* row[3];
   for (int k = 0; k < 3; k++) {
-    d.zg[k].s = (const int2*)(base + off_zg[k]);
-    d.zg[k].row = (const uint32_t*)(base + off_zr[k]);
+    d.zg[k].s = group[k] = (int2*)(base + off_zg[k]);
+    d.zg[k].row = row[k] = (uint32_t*)(base + off_zr[k]);
     d.zg[k].n = (int)h.zgrp[k].size();
+  }
+  // on the stream of the copy, and waited for like it
+  if (e == hipSuccess) e = launch_zsum_tables(d, (float*)(base + off_za), group, row, nullptr);
+  if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+  if (e != hipSuccess) {
+    hip_err(ctx, e, "geometry tables");
+    if (gd->block) (void)hipFree(gd->block);
+    delete gd;
+    return nullptr;
   }
   ctx->geoms[key] = gd;
   return gd;

@@ -111,37 +111,20 @@ int derive_geometry(const gfr_geometry* g, GeomHost* out, std::string* err, bool
   if (!with_ztab) return GFR_OK;
   const int nl = h.info.lambda1 - h.info.lambda0 + 1;
   h.ztab.resize((size_t)acc * nl);
-  h.za.assign((size_t)acc * nl + kZPad, 0.f);
-  for (int j = 0; j < 3; j++) h.zrow[j].resize(h.zgrp[j].size() * nl);
-  // LORs from s on that blend consecutive rows, row of LOR s and row + 1 first
-  std::vector<int> run(acc + 1, 0);
-  for (int li = 0; li < nl; li++) {
-    uint2* t = &h.ztab[(size_t)li * acc];
-    for (int s = acc - 1; s >= 0; s--) {
-      const float dz = h.seg[h.sino[s].x].dzf;
-      const float zc = (float)h.sino[s].y + 0.5f;
+  for (int s = 0; s < acc; s++) {
+    const float dz = h.seg[h.sino[s].x].dzf;
+    const float zc = (float)h.sino[s].y + 0.5f;
+    for (int li = 0; li < nl; li++) {
       const float z = fmaf((float)(h.info.lambda0 + li), dz, zc);
-      const float tz = z - 0.5f;
-      const float f = floorf(tz);
-      const float a = tz - f;
+      const float t = z - 0.5f;
+      const float f = floorf(t);
+      const float a = t - f;
       const int i = (int)f;
       const int z0 = i < 0 ? 0 : (i > g->nzs - 1 ? g->nzs - 1 : i);
       const int z1 = i + 1 < 0 ? 0 : (i + 1 > g->nzs - 1 ? g->nzs - 1 : i + 1);
       uint32_t ab;
       memcpy(&ab, &a, 4);
-      t[s] = make_uint2((uint32_t)z0 | ((uint32_t)z1 << 16), ab);
-      h.za[(size_t)li * acc + s] = a;
-      const bool next = s + 1 < acc && (t[s + 1].x & 0xffffu) == (uint32_t)z0 + 1;
-      run[s] = z1 != z0 + 1 ? 0 : next ? 1 + run[s + 1] : 1;
-    }
-    for (int j = 0; j < 3; j++) {
-      const size_t n = h.zgrp[j].size();
-      for (size_t q = 0; q < n; q++) {
-        int2& e = h.zgrp[j][q];
-        const bool reg = run[e.x] >= abs(e.y);
-        h.zrow[j][(size_t)li * n + q] = (t[e.x].x & 0xffffu) | (reg ? kZReg : 0u);
-        if (!reg) e.y = -abs(e.y);
-      }
+      h.ztab[(size_t)li * acc + s] = make_uint2((uint32_t)z0 | ((uint32_t)z1 << 16), ab);
     }
   }
   return GFR_OK;

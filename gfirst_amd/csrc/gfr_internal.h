@@ -23,21 +23,27 @@ struct SegEntry {
 };
 
 // Groups of the wide z-sum: up to SG (4, 6 or 8) consecutive planes of one
-// segment. s: first sinogram and number of sinograms of a group, negative when
-// some sample of the group lacks kZReg; row: per
-// sample [l1-l0+1][n] the row (image plane) of the group's first LOR, with
-// kZReg set where LOR i blends rows row + i and row + i + 1.
+// segment. s: first sinogram and number of sinograms of a group, negative where
+// in some sample LOR i does not blend rows row + i and row + i + 1; row: per
+// sample [l1-l0+1][n] the row (image plane) of the group's first LOR.
 struct ZGroups {
   const int2* s;
   const uint32_t* row;
   int n;
 };
-constexpr uint32_t kZReg = 1u << 31;
 inline __host__ __device__ int zg_index(int sg) { return sg == 4 ? 0 : sg == 6 ? 1 : 2; }
 // Row k of a sample that the n LORs of a group blend, counted from the group's
 // first: they need 0 .. n, and a group of fewer than SG LORs takes the last one
 // again instead of rows past the volume's end.
 inline __host__ __device__ int zg_row(int k, int n) { return k < n ? k : n; }
+// Whether the n LORs of a group blend consecutive rows in a sample (ztab entries
+// of the group's LORs).
+inline __host__ __device__ bool zg_regular(const uint2* t, int n) {
+  const uint32_t row = t[0].x & 0xffffu;
+  bool reg = true;
+  for (int i = 0; i < n; i++) reg = reg && t[i].x == (row + i) + ((row + i + 1) << 16);
+  return reg;
+}
 
 // Geometry as the kernels see it (by value). Pointers are device tables owned
 // by the context, built once per distinct geometry.
@@ -56,7 +62,7 @@ struct DevGeom {
   // [l1-l0+1][nsinogs]: z interpolation of each LOR sample, x = z0 | z1 << 16,
   // y = bits of alpha_z (GFIRST_GPU_Kernels.cu:88, 96 through the clamp filter)
   const uint2* ztab;
-  const float* za;          // [l1-l0+1][nsinogs]: alpha_z alone
+  const float* za;          // [l1-l0+1][nsinogs]: alpha_z alone, kZPad zeros
   ZGroups zg[3];            // groups of 4, 6 and 8 planes
 };
 
@@ -99,15 +105,17 @@ struct GeomHost {
   std::vector<SegEntry> seg;
   std::vector<int2> sino;
   std::vector<uint2> ztab;
-  std::vector<float> za;  // kZPad zeros after (groups read whole)
-  std::vector<int2> zgrp[3];
-  std::vector<uint32_t> zrow[3];
+  std::vector<int2> zgrp[3];  // ZGroups::s, no group marked
   float RADM, RESM, fxf, fxb;
 };
 
-constexpr int kZPad = 16;
+constexpr int kZPad = 16;  // zeros after za: groups read it whole
 // with_ztab: also build the per-sample z table (device tables only need it).
 int derive_geometry(const gfr_geometry* g, GeomHost* out, std::string* err, bool with_ztab = false);
+// Fills za and zg[].row of a geometry on the device from its ztab and groups, and
+// marks the groups that are not regular in every sample (zg[].s = s).
+hipError_t launch_zsum_tables(const DevGeom& G, float* za, int2* const s[3],
+                              uint32_t* const row[3], hipStream_t st);
 void psf_taps(float psf, float* g9);
 void gz_taps(float* g5);
 

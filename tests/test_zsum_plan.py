@@ -22,5 +22,5 @@ def test_rows_lie_in_the_volume(tmp_path):
     (tests/zsum_rows_check.cpp)."""
     out = subprocess.run([build("zsum_rows_check.cpp", tmp_path)], capture_output=True, text=True)
     assert out.returncode == 0, out.stdout
-    samples, ends, bad = map(int, out.stdout.split())
-    assert samples > 100_000 and ends > 1000 and bad == 0
+    samples, ends, irregular, bad = map(int, out.stdout.split())
+    assert samples > 100_000 and ends > 1000 and irregular > 1000 and bad == 0
