@@ -301,7 +301,10 @@ __global__ __launch_bounds__(256) void k_zsum_wide(DevGeom G, const float* __res
       float e[SG];
       unsigned roff[SG + 1];
 #pragma unroll
-      for (int k = 0; k <= SG; k++) roff[k] = (unsigned)zg_row(k, ng) * rowb;
+      for (int k = 0; k <= SG; k++) {
+        roff[k] = (unsigned)zg_row(k, ng) * rowb;
+        asm("" : "+s"(roff[k]));  // one addition a row, not a product
+      }
       uint32_t z = rows[0];
 #pragma unroll
       for (int i = 0; i < SG; i++) e[i] = wts[i];
